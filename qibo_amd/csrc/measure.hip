@@ -209,25 +209,49 @@ __device__ R np_leaf_sum_psi(const cplx<R>* a, int n) {
 }
 
 // Pairwise sums of consecutive runs of lc probabilities (lc a power of two,
-// 128 <= lc <= 8192): one 64-thread block per run, 128-element leaves
-// combined as a balanced tree (the pairwise split of a power of two).
+// 128 <= lc <= 8192): 128-element leaves (np_leaf_sum_psi: eight chains of
+// sixteen additions each) combined as a balanced tree (the pairwise split of
+// a power of two). Eight lanes share a leaf, one chain each, so a wave reads
+// whole lines of eight leaves with its sixteen loads in flight, and the tree
+// is a butterfly over the lanes (a + b either way round), then over the
+// wave's steps of 1024 elements. HBM bound: 2^26 amplitudes (1 GiB) in
+// complex128 took 1.02 ms with one lane per leaf and one 64-lane workgroup per
+// run (a run of 256 kept two lanes busy).
 template <typename R>
-__global__ __launch_bounds__(64) void k_run_sums(const cplx<R>* __restrict__ psi, uint64_t lc,
+__global__ __launch_bounds__(kT) void k_run_sums(const cplx<R>* __restrict__ psi, uint64_t lc, uint64_t n,
                                                  R* __restrict__ runsum) {
-  __shared__ R leaf[kMargBuf / 128];
-  const uint64_t run = block_id();
-  const cplx<R>* a = psi + run * lc;
-  const int nleaf = int(lc / 128);
-  if (int(threadIdx.x) < nleaf) leaf[threadIdx.x] = np_leaf_sum_psi(a + uint64_t(threadIdx.x) * 128, 128);
-  __syncthreads();
-  for (int w = nleaf; w > 1; w >>= 1) {
-    R v = R(0);
-    if (int(threadIdx.x) < w / 2) v = leaf[2 * threadIdx.x] + leaf[2 * threadIdx.x + 1];
-    __syncthreads();
-    if (int(threadIdx.x) < w / 2) leaf[threadIdx.x] = v;
-    __syncthreads();
+  const uint64_t steps = lc > 1024 ? lc / 1024 : 1;  // per wave: one run, or 1024 elements of shorter runs
+  const uint64_t first = (block_id() * (kT / 64) + threadIdx.x / 64) * steps * 1024;
+  const int lane = threadIdx.x & 63;
+  if (first >= n) return;  // whole waves leave: no barrier follows
+  R part[8];
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    part[st] = R(0);
+    if (uint64_t(st) >= steps) continue;
+    // leaf lane / 8 of the step; leaves past the end (n < 1024) repeat leaf 0 and are not written
+    uint64_t at = first + uint64_t(st) * 1024 + uint64_t(lane >> 3) * 128;
+    if (at >= n) at = first;
+    const cplx<R>* a = psi + at + (lane & 7);
+    cplx<R> x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = ld(a, 8 * i);
+    R v = np_abs2(x[0]);
+#pragma unroll
+    for (int i = 1; i < 16; ++i) v = v + np_abs2(x[i]);
+    for (int w = 1; w < 8; w <<= 1) v = v + __shfl_xor(v, w, 64);
+    for (uint64_t w = 8; w < 64 && w * 16 < lc; w <<= 1) v = v + __shfl_xor(v, int(w), 64);
+    part[st] = v;
   }
-  if (threadIdx.x == 0) runsum[run] = leaf[0];
+#pragma unroll
+  for (int w = 1; w < 8; w <<= 1)
+    if (uint64_t(w) < steps)
+#pragma unroll
+      for (int st = 0; st < 8; st += 2 * w) part[st] = part[st] + part[st + w];
+  // lanes that hold a run's sum: every lc / 16-th, one of them for lc >= 1024
+  const uint64_t lanes = lc >= 1024 ? 64 : lc / 16;
+  const uint64_t e = first + uint64_t(lane / lanes) * (lanes * 16);
+  if (uint64_t(lane) % lanes == 0 && e < n) runsum[e / lc] = part[0];
 }
 
 struct NpMargArgs {
@@ -285,6 +309,162 @@ __global__ __launch_bounds__(kT) void k_marg_np_seq(const cplx<R>* __restrict__ 
   out[o] = acc;
 }
 
+// Long chains: the three sums above with the loads taken off the chain.
+//
+// One thread per outcome leaves a chain of dependent additions waiting for a
+// load each (0.74 us a step: 2^10 outcomes of 26 qubits took 48.3 ms, 16
+// wavefronts in all). Here a workgroup owns 2^g outcomes: fifteen waves form
+// the next 2^c values of every chain in LDS (all loads in flight at once,
+// addresses ascending), while the lanes of the first wave add the previous
+// 2^c values of their outcomes from LDS, in the same order -- the values and
+// the additions are those of the kernels above, bit for bit. What bounds it
+// is the dependent addition (2^16 steps: 0.43 ms for those 26 qubits), or HBM
+// where there are many outcomes.
+enum : int { kChainAbs2 = 0, kChainLeaf = 1, kChainRuns = 2 };
+constexpr int kChainT = 1024;       // threads: one wave adds, fifteen load
+constexpr int kChainTileBits = 12;  // values per chunk and workgroup
+constexpr int kChainMaxG = 6;       // outcomes per workgroup: lanes of the adding wave
+constexpr int kChainMinBits = 7;    // shorter chains stay with one thread per outcome
+
+struct ChainArgs {
+  uint64_t nchunk;   // 2^c-step chunks per chain
+  uint64_t leaf;     // kChainLeaf: elements per value
+  int c, g;
+  int m;
+  int nhc, nho;      // chain bits above c, outcome bits above g
+  uint8_t tpos[kChainTileBits];   // index bit of tile bit j, ascending
+  uint32_t tslot[kChainTileBits]; // its weight in the LDS slot
+  uint8_t cpos[kMaxFixed];  // index bits of the chain bits above c
+  uint8_t opos[kMaxFixed];  // index bits of the outcome bits above g
+  uint8_t gpos[kChainMaxG]; // index bits of the lowest g measured bits
+  uint8_t obit[kMaxFixed];  // index bit of requested output bit k (k = 0 most significant)
+};
+
+template <typename R>
+constexpr int chain_stride(int steps) { return steps + int(16 / sizeof(R)); }  // 16-byte rows, spread over the banks
+
+template <typename R, int MODE>
+__device__ __forceinline__ R chain_value(const void* src, uint64_t i, uint64_t leaf) {
+  if constexpr (MODE == kChainAbs2) return np_abs2(ld(reinterpret_cast<const cplx<R>*>(src), i));
+  if constexpr (MODE == kChainLeaf) return np_leaf_sum_psi(reinterpret_cast<const cplx<R>*>(src) + i * leaf, int(leaf));
+  return reinterpret_cast<const R*>(src)[i];
+}
+
+template <typename R, int MODE>
+__global__ __launch_bounds__(kChainT) void k_marg_chain(const void* __restrict__ src, R* __restrict__ out,
+                                                        const ChainArgs a) {
+  constexpr int kBuf = (1 << kChainTileBits) + (1 << kChainMaxG) * int(16 / sizeof(R));
+  __shared__ __align__(16) R buf[2][kBuf];
+  constexpr int kLoaders = kChainT - 64;
+  constexpr int kPer = ((1 << kChainTileBits) + kLoaders - 1) / kLoaders;
+  const int tile = 1 << (a.c + a.g);
+  uint64_t base = 0;  // the workgroup's outcomes
+  for (int k = 0; k < a.nho; ++k) base |= ((block_id() >> k) & 1) << a.opos[k];
+  const bool adder = threadIdx.x < 64;
+  uint64_t off[kPer];
+  uint32_t slot[kPer];
+  if (!adder) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const uint32_t e = threadIdx.x - 64 + i * kLoaders;
+      off[i] = 0;
+      slot[i] = 0;
+      for (int j = 0; j < a.c + a.g; ++j)
+        if ((e >> j) & 1) {
+          off[i] |= uint64_t(1) << a.tpos[j];
+          slot[i] += a.tslot[j];
+        }
+    }
+  }
+  const int steps = 1 << a.c;
+  R acc = R(0);
+  for (uint64_t ch = 0; ch <= a.nchunk; ++ch) {  // load chunk ch, add chunk ch - 1
+    if (!adder) {
+      if (ch < a.nchunk) {
+        uint64_t cb = base;
+        for (int k = 0; k < a.nhc; ++k) cb |= ((ch >> k) & 1) << a.cpos[k];
+        R v[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+          v[i] = int(threadIdx.x) - 64 + i * kLoaders < tile ? chain_value<R, MODE>(src, cb | off[i], a.leaf) : R(0);
+#pragma unroll
+        for (int i = 0; i < kPer; ++i)
+          if (int(threadIdx.x) - 64 + i * kLoaders < tile) buf[ch & 1][slot[i]] = v[i];
+      }
+    } else if (ch > 0 && int(threadIdx.x) < (1 << a.g)) {
+      const R* q = &buf[(ch - 1) & 1][int(threadIdx.x) * chain_stride<R>(steps)];
+      constexpr int U = 16;
+      R x[U], y[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) x[i] = q[i];
+      for (int s = U; s <= steps; s += U) {  // the next U values are read while these are added
+        const int nx = s < steps ? s : 0;
+#pragma unroll
+        for (int i = 0; i < U; ++i) y[i] = q[nx + i];
+#pragma unroll
+        for (int i = 0; i < U; ++i) acc = acc + x[i];
+#pragma unroll
+        for (int i = 0; i < U; ++i) x[i] = y[i];
+      }
+    }
+    __syncthreads();
+  }
+  if (int(threadIdx.x) < (1 << a.g)) {
+    for (int k = 0; k < a.g; ++k) base |= uint64_t((threadIdx.x >> k) & 1) << a.gpos[k];
+    uint64_t o = 0;
+    for (int k = 0; k < a.m; ++k) o |= ((base >> a.obit[k]) & 1) << (a.m - 1 - k);
+    out[o] = acc;
+  }
+}
+
+// The chain kernel over an index of `nbits` bits of which `mpos` (ascending)
+// are measured; false if the chains are too short for it. Outcomes per
+// workgroup: as many as leave 256 workgroups (one per CU), but at least those
+// that share a 128-byte line (the measured ones among the lowest 3 bits).
+// Chains below 2^7 steps stay with one thread per outcome, which has 2^(n-6)
+// threads there (24 qubits, chains of 2^6: 178 us against 231 us here; of
+// 2^8: 372 us against 104 us).
+template <typename R, int MODE>
+static bool launch_chain(const void* src, R* out, int nbits, const NpMargArgs& p, uint64_t leaf, hipStream_t s) {
+  ChainArgs a;
+  std::memset(&a, 0, sizeof(a));
+  const int m = p.m, cl = nbits - m;
+  if (cl < kChainMinBits) return false;
+  int low = 0;
+  for (int k = 0; k < m; ++k) low += p.mpos[k] < 3;
+  a.g = std::min(m, std::min(kChainMaxG, std::max(low, m - 8)));
+  a.c = std::min(cl, kChainTileBits - a.g);
+  a.m = m;
+  a.leaf = leaf;
+  a.nchunk = uint64_t(1) << (cl - a.c);
+  bool measured[64] = {false};
+  for (int k = 0; k < m; ++k) measured[p.mpos[k]] = true;
+  int nt = 0, nm = 0, nu = 0;
+  for (int b = 0; b < nbits; ++b) {
+    if (measured[b]) {
+      if (nm < a.g) {
+        a.tslot[nt] = uint32_t(chain_stride<R>(1 << a.c)) << nm;
+        a.tpos[nt++] = uint8_t(b);
+        a.gpos[nm] = uint8_t(b);
+      } else {
+        a.opos[a.nho++] = uint8_t(b);
+      }
+      ++nm;
+    } else {
+      if (nu < a.c) {
+        a.tslot[nt] = uint32_t(1) << nu;
+        a.tpos[nt++] = uint8_t(b);
+      } else {
+        a.cpos[a.nhc++] = uint8_t(b);
+      }
+      ++nu;
+    }
+  }
+  std::memcpy(a.obit, p.obit, sizeof(a.obit));
+  hipLaunchKernelGGL((k_marg_chain<R, MODE>), launch_grid(uint64_t(1) << a.nho), dim3(kChainT), 0, s, src, out, a);
+  return true;
+}
+
 // Launches numpy's order for a marginal; returns 1 if the serial chain is too
 // long (the caller then sums in parallel), 0 on launch, <0 on error.
 template <typename R>
@@ -301,7 +481,8 @@ static int marg_numpy_order(const cplx<R>* psi, int n, const int* qubits, int m,
     if (a.nred > kMaxSerial) return 1;
     for (int k = 0; k < m; ++k) a.obit[k] = uint8_t(n - 1 - qubits[k]);
     sorted_positions(n, qubits, m, nullptr, 0, a.mpos);
-    hipLaunchKernelGGL(k_marg_np_seq<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, psi, out, a);
+    if (!launch_chain<R, kChainAbs2>(psi, out, n, a, 1, s))
+      hipLaunchKernelGGL(k_marg_np_seq<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, psi, out, a);
     QSIM_CHECK_LAUNCH();
     return 0;
   }
@@ -317,7 +498,8 @@ static int marg_numpy_order(const cplx<R>* psi, int n, const int* qubits, int m,
   if (L < 128) {
     if (a.nred * L > kMaxSerial) return 1;
     a.nsub = L;
-    hipLaunchKernelGGL(k_marg_np_short<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, psi, out, a);
+    if (!launch_chain<R, kChainLeaf>(psi, out, outer_bits, a, L, s))
+      hipLaunchKernelGGL(k_marg_np_short<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, psi, out, a);
     QSIM_CHECK_LAUNCH();
     return 0;
   }
@@ -327,9 +509,17 @@ static int marg_numpy_order(const cplx<R>* psi, int n, const int* qubits, int m,
   const uint64_t nruns = (uint64_t(1) << n) / lc;
   QSIM_CHECK_ARG(ws != nullptr && ws_bytes >= nruns * sizeof(R), "qsim_probabilities: workspace too small");
   R* runsum = reinterpret_cast<R*>(ws);
-  hipLaunchKernelGGL(k_run_sums<R>, launch_grid(nruns), dim3(64), 0, s, psi, lc, runsum);
+  const uint64_t waves = ceil_div_u(uint64_t(1) << n, std::max<uint64_t>(lc, 1024));
+  hipLaunchKernelGGL(k_run_sums<R>, launch_grid(ceil_div_u(waves, kT / 64)), dim3(kT), 0, s, psi, lc,
+                     uint64_t(1) << n, runsum);
   QSIM_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_marg_np_runs<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, runsum, out, a);
+  // the run sums of one outer index are the lowest chain bits
+  int sub = 0;
+  while ((uint64_t(1) << sub) < a.nsub) ++sub;
+  NpMargArgs r = a;
+  for (int k = 0; k < m; ++k) r.obit[k] = uint8_t(a.obit[k] + sub), r.mpos[k] = uint8_t(a.mpos[k] + sub);
+  if (!launch_chain<R, kChainRuns>(runsum, out, outer_bits + sub, r, 1, s))
+    hipLaunchKernelGGL(k_marg_np_runs<R>, launch_grid(ceil_div_u(a.nout, kT)), dim3(kT), 0, s, runsum, out, a);
   QSIM_CHECK_LAUNCH();
   return 0;
 }
