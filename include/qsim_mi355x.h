@@ -368,7 +368,8 @@ int qsim_histogram(const int64_t* samples, int64_t nshots, int64_t* counts, int6
  * where masks are over amplitude-index bits (bit n-1-q for qubit q) and ny_t is
  * the number of Y factors of term t (Y = i X Z). Replaces the per-term einsum
  * loop of Backend.exp_value_observable_symbolic (abstract.py:2946-3054).
- * `out` is one device double. Terms sharing an X mask share one state pass.
+ * `out` is one device double. Terms whose X masks fit one tile of 12 index bits
+ * share one state pass.
  * `workspace` must hold qsim_expval_workspace(nqubits, nterms) bytes. */
 size_t qsim_expval_workspace(int nqubits, int nterms);
 int qsim_expval_pauli(const void* state, int nqubits, int dtype, int nterms, const uint64_t* xmasks,
@@ -399,6 +400,18 @@ int qsim_expval_noalloc_max_groups(void);
 int qsim_apply_pauli_sum(const void* state, int nqubits, int dtype, int nterms,
                          const uint64_t* xmasks, const uint64_t* zmasks, const int* ny,
                          const double* coeffs, void* out, void* stream);
+
+/* qsim_apply_pauli_sum for nbatch states of 2^nqubits amplitudes each, one
+ * after the other in `states` and in `out`, and energies[b] = Re <psi_b|out_b>
+ * (device doubles, from the products before they are rounded to the state's
+ * type): the seed of the adjoint sweep over a batch of parameter sets, in one
+ * launch for Hamiltonians of at most 40 X masks and 96 terms. `workspace` must
+ * hold qsim_apply_pauli_sum_batched_workspace(nbatch, nterms) bytes. */
+size_t qsim_apply_pauli_sum_batched_workspace(int nbatch, int nterms);
+int qsim_apply_pauli_sum_batched(const void* states, int nbatch, int nqubits, int dtype, int nterms,
+                                 const uint64_t* xmasks, const uint64_t* zmasks, const int* ny,
+                                 const double* coeffs, void* out, double* energies, void* workspace,
+                                 size_t workspace_bytes, void* stream);
 
 /* out = Re <bra| M_targets |ket> for a dense 2^k x 2^k host matrix (k = 1..3)
  * under `controls`, accumulated in FP64 into one device double. The

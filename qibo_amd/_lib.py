@@ -60,6 +60,8 @@ SIGNATURES = {
     "qsim_expval_pauli_noalloc": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     "qsim_expval_noalloc_max_groups": (_i, []),
     "qsim_apply_pauli_sum": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "qsim_apply_pauli_sum_batched_workspace": (_sz, [_i, _i]),
+    "qsim_apply_pauli_sum_batched": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "qsim_inner_matrix": (_i, [_vp, _vp, _i, _i, _c_int_p, _i, _c_int_p, _i, _vp, _vp, _vp, _sz, _vp]),
     "qsim_blocked_header_bytes": (_sz, []),
     "qsim_apply_blocked": (_i, [_vp, _i, _i, _c_int_p, _vp, _sz, _i, _vp]),

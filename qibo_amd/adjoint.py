@@ -542,10 +542,14 @@ def blocked_expectation_and_gradient(backend, circuit, hamiltonian, params: np.n
                                                     pdev.data_ptr() + off, stride, nbytes, p.count, stream)
             _lib.check(rc, lib)
         lam = torch.empty_like(psi)
-        for b in range(nb):
-            _lib.check(lib.qsim_apply_pauli_sum(psi[b].data_ptr(), n, code, len(c), xm.ctypes.data, zm.ctypes.data,
-                                                ny.ctypes.data, c.ctypes.data, lam[b].data_ptr(), stream), lib)
-            energies[b0 + b] = backend.expectation_pauli(psi[b], n, xm, zm, ny, c) + hamiltonian.constant
+        wsb = lib.qsim_apply_pauli_sum_batched_workspace(nb, len(c))
+        ws = backend._workspace(wsb, "pauli_batch", dev)
+        esub = energies[b0:b1]
+        _lib.check(lib.qsim_apply_pauli_sum_batched(psi.data_ptr(), nb, n, code, len(c), xm.ctypes.data,
+                                                    zm.ctypes.data, ny.ctypes.data, c.ctypes.data, lam.data_ptr(),
+                                                    esub.data_ptr(), ws.data_ptr(), wsb, stream), lib)
+        if hamiltonian.constant:
+            esub += hamiltonian.constant
         gsub = grads[b0:b1]
         pdev, layout = _upload_programs(tmpl.rev, tmpl, table, dev)
         keep.append(pdev)

@@ -28,22 +28,18 @@ namespace qsim {
 constexpr int kET = 256;
 constexpr int kEBlocks = 1024;  // fixed grid of every reduction pass
 constexpr int kMaxGroupTerms = 32;
+constexpr int kESpread = 256;   // workgroups the items of a few tiles are spread over (one per CU)
 
 struct PauliGroupArgs {
   uint64_t nwork;
-  uint64_t x;      // flip mask of the group (0 = diagonal)
-  uint64_t hbit;   // top bit of x (unused when x = 0)
+  uint64_t x;      // flip mask of the group
+  uint64_t hbit;   // top bit of x
   int hpos;
   int nterms;
   uint64_t z[kMaxGroupTerms];
   double c[kMaxGroupTerms];
   int ny[kMaxGroupTerms];
 };
-
-template <typename R>
-__device__ __forceinline__ double sq(cplx<R> v) {
-  return double(v.re) * double(v.re) + double(v.im) * double(v.im);
-}
 
 __device__ double block_sum(double v, double* lds) {
   lds[threadIdx.x] = v;
@@ -61,51 +57,466 @@ __global__ __launch_bounds__(kET) void k_pauli_group(const cplx<R>* __restrict__
   __shared__ double lds[kET];
   double acc = 0.0;
   const uint64_t stride = uint64_t(gridDim.x) * kET;
-  if (a.x == 0) {
-    for (uint64_t i = uint64_t(blockIdx.x) * kET + threadIdx.x; i < a.nwork; i += stride) {
-      const double p = sq(psi[i]);
-      double w = 0.0;
-      for (int t = 0; t < a.nterms; ++t) w += (__popcll(i & a.z[t]) & 1) ? -a.c[t] : a.c[t];
-      acc += w * p;
-    }
-  } else {
-    for (uint64_t j = uint64_t(blockIdx.x) * kET + threadIdx.x; j < a.nwork; j += stride) {
-      const uint64_t low = j & (a.hbit - 1);
-      const uint64_t i0 = low | ((j ^ low) << 1);
-      const uint64_t i1 = i0 ^ a.x;
-      const cplx<R> u = psi[i0], v = psi[i1];
-      // A = conj(u) * v
-      const double are = double(u.re) * double(v.re) + double(u.im) * double(v.im);
-      const double aim = double(u.re) * double(v.im) - double(u.im) * double(v.re);
-      for (int t = 0; t < a.nterms; ++t) {
-        const double s1 = (__popcll(i1 & a.z[t]) & 1) ? -1.0 : 1.0;
-        const double s0 = (__popcll(i0 & a.z[t]) & 1) ? -1.0 : 1.0;
-        // w = s1 A + s0 conj(A)
-        const double wre = (s1 + s0) * are;
-        const double wim = (s1 - s0) * aim;
-        // Re(i^ny w)
-        double re;
-        switch (a.ny[t] & 3) {
-          case 0: re = wre; break;
-          case 1: re = -wim; break;
-          case 2: re = -wre; break;
-          default: re = wim; break;
-        }
-        acc += a.c[t] * re;
+  for (uint64_t j = uint64_t(blockIdx.x) * kET + threadIdx.x; j < a.nwork; j += stride) {
+    const uint64_t low = j & (a.hbit - 1);
+    const uint64_t i0 = low | ((j ^ low) << 1);
+    const uint64_t i1 = i0 ^ a.x;
+    const cplx<R> u = psi[i0], v = psi[i1];
+    // A = conj(u) * v
+    const double are = double(u.re) * double(v.re) + double(u.im) * double(v.im);
+    const double aim = double(u.re) * double(v.im) - double(u.im) * double(v.re);
+    for (int t = 0; t < a.nterms; ++t) {
+      const double s1 = (__popcll(i1 & a.z[t]) & 1) ? -1.0 : 1.0;
+      const double s0 = (__popcll(i0 & a.z[t]) & 1) ? -1.0 : 1.0;
+      // w = s1 A + s0 conj(A)
+      const double wre = (s1 + s0) * are;
+      const double wim = (s1 - s0) * aim;
+      // Re(i^ny w)
+      double re;
+      switch (a.ny[t] & 3) {
+        case 0: re = wre; break;
+        case 1: re = -wim; break;
+        case 2: re = -wre; break;
+        default: re = wim; break;
       }
+      acc += a.c[t] * re;
     }
   }
   const double tot = block_sum(acc, lds);
   if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(kET) void k_sum_partials(const double* __restrict__ partial, int64_t count,
+// ---------------------------------------------------------------------------
+// Many X masks per read of the state.
+//
+// One pass per X mask reads the whole state each time (the transverse-field
+// Ising chain on 27 qubits: 28 passes of 0.39 ms). Here a workgroup holds a
+// tile of 4096 amplitudes -- 16 per lane in registers, all of them in LDS --
+// and forms every group whose mask flips tile bits only: the partner of
+// amplitude i is i ^ x of the same tile, from the lane's own registers or
+// from LDS. With the lowest 3 index bits in every tile (whole 128-byte lines)
+// a pass covers 9 more flip bits, so that chain takes 3 passes: 10.9 -> 1.6 ms,
+// 0.53 ms per 2 GiB read. A pass reads 16 bytes of LDS per amplitude and mask
+// that is not one register bit, and two workgroups (64 KB of LDS each) share
+// a CU, so loads and sums overlap only in part (complex64 takes the same time).
+//
+//   (P psi)_i = w(i) psi_{i ^ x},  w(i) = c i^ny (-1)^{|(i ^ x) & z|}
+//
+// The sign of a term factors into a tile part, a lane part and one of 16
+// patterns over the registers: one bit per term and lane (the tile's bits come
+// from one ballot), so no term's masks are read inside the loop over tiles.
+// ---------------------------------------------------------------------------
+constexpr int kPTileBits = 12;
+constexpr int kPReg = 16;
+constexpr int kPLaneBits = 8;     // local bits 0-7: the lane; 8-11: the register
+constexpr int kPLowBits = 3;      // index bits in every tile
+constexpr int kPMaxItems = 48;
+constexpr int kPMaxDiag = 64;
+
+enum : uint32_t { kPImag = 1u << 16, kPFar = 1u << 17, kPTwo = 1u << 18 };
+
+// One or two terms of one X mask, their coefficients both real or both
+// imaginary. A term's sign at amplitude i is a tile part times a lane part
+// (one bit per term, see SignBits) times `pat`: bit r set where it is negative
+// on register r.
+struct PauliItem {
+  uint32_t xl;      // flip mask on the local bits | flags
+  uint16_t pat[2];
+  double k[2];      // c (-1)^{|x & z|}, negated for ny = 2, 3
+  uint64_t x;       // the whole mask, read where it leaves the tile
+};
+
+struct PauliTileArgs {
+  uint64_t ntiles;
+  uint64_t stride;  // amplitudes between the states of a batch (grid y)
+  uint32_t valid;   // amplitudes of a tile that exist (registers below 12 qubits)
+  int nitems, ndiag;
+  int per;          // items per grid z (the terms of x = 0 belong to z = 0)
+  int accumulate;   // APPLY: out += instead of out =
+  uint8_t tbits[kPTileBits];  // index bit of local bit i, ascending
+  uint8_t dcount[kPReg];      // x = 0 terms per register pattern, dk sorted by it
+  PauliItem item[kPMaxItems];
+  double dk[kPMaxDiag];
+};
+static_assert(sizeof(PauliTileArgs) <= 2304, "kernel arguments");
+
+// z masks of the terms in bit order of the sign words: words 0 and 1 the
+// x = 0 terms, 2-4 the items' terms (two bits per item).
+constexpr int kPWords = 5;
+struct PauliZ {
+  uint64_t zout[32 * kPWords];  // outside the tile
+  uint16_t zl[32 * kPWords];    // local lane bits
+};
+static_assert(kPMaxDiag <= 64 && 2 * kPMaxItems <= 96, "sign words");
+
+template <typename R>
+__device__ __forceinline__ cplx<double> widen(cplx<R> v) {
+  cplx<double> d;
+  d.re = double(v.re);
+  d.im = double(v.im);
+  return d;
+}
+
+__device__ __forceinline__ double xor_sign(double k, uint32_t sign) {
+  return __hiloint2double(int(uint32_t(__double2hiint(k)) ^ sign), __double2loint(k));
+}
+
+// Visits the lane's 16 (register, partner) pairs of one item.
+template <bool FAR, typename R, typename F>
+__device__ __forceinline__ void pauli_pairs(const cplx<R>* v, const cplx<R>* lds, const cplx<R>* psi, uint64_t first,
+                                            const uint64_t* goff, const PauliItem& g, uint32_t lane, F&& f) {
+  if constexpr (FAR) {
+    if (g.xl & kPFar) {  // first: the index of the lane's register 0
+      const uint64_t at = first ^ g.x;
+#pragma unroll
+      for (int r0 = 0; r0 < kPReg; r0 += 8) {
+        cplx<R> u[8];  // eight loads in flight
+#pragma unroll
+        for (int r = 0; r < 8; ++r) u[r] = ld(psi, at ^ goff[r0 + r]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) f(r0 + r, widen(u[r]));
+      }
+      return;
+    }
+  }
+  const uint32_t xl = g.xl & ((1u << kPTileBits) - 1);
+  if (xl == (1u << kPLaneBits)) {
+#pragma unroll
+    for (int r = 0; r < kPReg; ++r) f(r, widen(v[r ^ 1]));
+  } else if (xl == (2u << kPLaneBits)) {
+#pragma unroll
+    for (int r = 0; r < kPReg; ++r) f(r, widen(v[r ^ 2]));
+  } else if (xl == (4u << kPLaneBits)) {
+#pragma unroll
+    for (int r = 0; r < kPReg; ++r) f(r, widen(v[r ^ 4]));
+  } else if (xl == (8u << kPLaneBits)) {
+#pragma unroll
+    for (int r = 0; r < kPReg; ++r) f(r, widen(v[r ^ 8]));
+  } else {
+    const uint32_t at = lane ^ xl;  // (lane bits and register bits are disjoint)
+#pragma unroll
+    for (int r0 = 0; r0 < kPReg; r0 += 8) {
+      cplx<R> u[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) u[r] = lds[at ^ (uint32_t(r0 + r) << kPLaneBits)];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f(r0 + r, widen(u[r]));
+    }
+  }
+}
+
+// Index bits contributed by local index u.
+__device__ __forceinline__ uint64_t pauli_deposit(const PauliTileArgs& a, uint32_t u) {
+  uint64_t i = 0;
+#pragma unroll
+  for (int b = 0; b < kPTileBits; ++b)
+    if ((u >> b) & 1) i |= uint64_t(1) << a.tbits[b];
+  return i;
+}
+
+// Energy (APPLY = false): partial[block] = sum over the block's tiles of
+// Re conj(psi_i) w(i) psi_{i ^ x}. APPLY: out_i (+)= sum of w(i) psi_{i ^ x}
+// and that sum beside it (masks that leave the tile read their partners from
+// memory), one state of a batch per grid y; partial may be null.
+template <typename R, bool APPLY>
+__global__ __launch_bounds__(kET, 2) void k_pauli_tile(const cplx<R>* __restrict__ psi, cplx<R>* __restrict__ out,
+                                                       const PauliTileArgs a, const PauliZ zz,
+                                                       double* __restrict__ partial) {
+  __shared__ cplx<R> lds[1 << kPTileBits];
+  __shared__ double red[kET];
+  const uint32_t lane = threadIdx.x;
+  psi += uint64_t(blockIdx.y) * a.stride;
+  const uint64_t lane_off = pauli_deposit(a, lane);
+  uint64_t goff[kPReg];
+#pragma unroll
+  for (int r = 0; r < kPReg; ++r) goff[r] = pauli_deposit(a, uint32_t(r) << kPLaneBits);
+  auto load = [&](uint64_t tile, cplx<R>* v) {
+    const uint64_t at = insert_zeros(tile, a.tbits, kPTileBits) | lane_off;
+    if (a.valid == (1u << kPTileBits)) {
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) v[r] = ld(psi, at | goff[r]);
+    } else {  // a register below 12 qubits: the amplitudes past it are zero (amplitude 0 is read in their place)
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) {
+        const bool there = (lane | (uint32_t(r) << kPLaneBits)) < a.valid;
+        v[r] = ld(psi, there ? at | goff[r] : 0);
+        v[r].re = there ? v[r].re : R(0);
+        v[r].im = there ? v[r].im : R(0);
+      }
+    }
+  };
+  const int i0 = int(blockIdx.z) * a.per;
+  const int i1 = i0 + a.per < a.nitems ? i0 + a.per : a.nitems;
+  const bool diag = a.ndiag > 0 && blockIdx.z == 0;
+  // one sign bit per term: the lane's part once, the tile's part per tile (a
+  // wave's lane t forms term t's)
+  uint32_t lane_sign[kPWords];
+  uint64_t zo[(kPWords + 1) / 2];
+#pragma unroll
+  for (int w = 0; w < kPWords; ++w) {
+    lane_sign[w] = 0;
+    const int cnt = w < 2 ? (a.ndiag - 32 * w) : (2 * a.nitems - 32 * (w - 2));
+    for (int t = 0; t < 32 && t < cnt; ++t)
+      lane_sign[w] |= uint32_t(__popc(lane & zz.zl[32 * w + t]) & 1) << t;
+  }
+#pragma unroll
+  for (int h = 0; h < (kPWords + 1) / 2; ++h) {
+    const int t = 64 * h + int(lane & 63);
+    zo[h] = t < 32 * kPWords ? zz.zout[t] : 0;
+  }
+  double acc = 0.0;
+  cplx<R> v[kPReg];
+  for (uint64_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
+    load(tile, v);
+    const uint64_t origin = insert_zeros(tile, a.tbits, kPTileBits);
+    uint32_t sign[kPWords];
+#pragma unroll
+    for (int h = 0; h < (kPWords + 1) / 2; ++h) {
+      const uint64_t odd = __ballot(__popcll(origin & zo[h]) & 1);
+      sign[2 * h] = lane_sign[2 * h] ^ uint32_t(odd);
+      if (2 * h + 1 < kPWords) sign[2 * h + 1] = lane_sign[2 * h + 1] ^ uint32_t(odd >> 32);
+    }
+#pragma unroll
+    for (int r = 0; r < kPReg; ++r) lds[lane | (uint32_t(r) << kPLaneBits)] = v[r];
+    __syncthreads();
+    cplx<double> o[APPLY ? kPReg : 1];
+    if constexpr (APPLY) {
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) o[r] = cplx<double>{0.0, 0.0};
+    }
+    if (diag) {
+      // coefficients per register pattern, then one 16-point Walsh-Hadamard
+      // transform: w on the lane's 16 amplitudes
+      double w[kPReg];
+      int t = 0;
+      uint32_t word = sign[0];
+#pragma unroll
+      for (int k = 0; k < kPReg; ++k) {
+        w[k] = 0.0;
+        for (int left = a.dcount[k]; left > 0; --left) {
+          w[k] += xor_sign(a.dk[t], word << 31);
+          word = ++t == 32 ? sign[1] : word >> 1;
+        }
+      }
+#pragma unroll
+      for (int h = 1; h < kPReg; h <<= 1)
+#pragma unroll
+        for (int r = 0; r < kPReg; ++r)
+          if (!(r & h)) {
+            const double x = w[r], y = w[r | h];
+            w[r] = x + y;
+            w[r | h] = x - y;
+          }
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) {
+        const cplx<double> u = widen(v[r]);
+        if constexpr (APPLY) {
+          o[r].re = w[r] * u.re;
+          o[r].im = w[r] * u.im;
+        } else {
+          acc = __builtin_fma(w[r], __builtin_fma(u.re, u.re, u.im * u.im), acc);
+        }
+      }
+    }
+    PauliItem next = a.item[i0 < i1 ? i0 : 0];
+    uint32_t word = sign[2];
+    if (i0 >= 32)
+      word = sign[4];
+    else if (i0 >= 16)
+      word = sign[3];
+    word >>= 2 * (i0 & 15);
+    for (int i = i0; i < i1; ++i) {
+      const PauliItem g = next;  // read one item ahead
+      next = a.item[i + 1 < i1 ? i + 1 : i];
+      const uint32_t s0 = word << 31, s1 = (word << 30) & 0x80000000u;
+      word = (i + 1) == 16 ? sign[3] : ((i + 1) == 32 ? sign[4] : word >> 2);
+      // (products of the lane's own amplitudes are formed where they are used,
+      // not kept in registers from one item to the next)
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) asm volatile("" : "+v"(v[r].re), "+v"(v[r].im));
+      double k0 = xor_sign(g.k[0], s0);
+      const double k1 = xor_sign(g.k[1], s1);
+      const bool same = (g.pat[0] | g.pat[1]) == 0;
+      if (same) k0 += k1;  // (k[1] = 0 of a single term)
+      const uint32_t p0 = g.pat[0], p1 = g.pat[1];
+      auto weight = [&](int r) {
+        return xor_sign(k0, p0 << (31 - r) & 0x80000000u) + xor_sign(k1, p1 << (31 - r) & 0x80000000u);
+      };
+      if constexpr (!APPLY) {
+        // Re(w B) with B = conj(psi_i) psi_{i ^ x}: w Re B, or -w Im B for imaginary w
+        double s[4] = {0.0, 0.0, 0.0, 0.0};  // four chains of additions
+        if (g.xl & kPImag) {
+          pauli_pairs<false>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            const double b = __builtin_fma(double(v[r].im), u.re, -(double(v[r].re) * u.im));
+            s[r & 3] = __builtin_fma(same ? k0 : weight(r), b, s[r & 3]);
+          });
+          acc += (s[0] + s[1]) + (s[2] + s[3]);
+        } else if (same) {
+          pauli_pairs<false>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            s[r & 3] = __builtin_fma(double(v[r].re), u.re, __builtin_fma(double(v[r].im), u.im, s[r & 3]));
+          });
+          acc = __builtin_fma(k0, (s[0] + s[1]) + (s[2] + s[3]), acc);
+        } else {
+          pauli_pairs<false>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            const double b = __builtin_fma(double(v[r].re), u.re, double(v[r].im) * u.im);
+            s[r & 3] = __builtin_fma(weight(r), b, s[r & 3]);
+          });
+          acc += (s[0] + s[1]) + (s[2] + s[3]);
+        }
+      } else {
+        if (g.xl & kPImag) {
+          pauli_pairs<true>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            const double k = same ? k0 : weight(r);
+            o[r].re = __builtin_fma(-k, u.im, o[r].re);
+            o[r].im = __builtin_fma(k, u.re, o[r].im);
+          });
+        } else if (same) {
+          pauli_pairs<true>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            o[r].re = __builtin_fma(k0, u.re, o[r].re);
+            o[r].im = __builtin_fma(k0, u.im, o[r].im);
+          });
+        } else {
+          pauli_pairs<true>(v, lds, psi, origin | lane_off, goff, g, lane, [&](int r, cplx<double> u) {
+            const double k = weight(r);
+            o[r].re = __builtin_fma(k, u.re, o[r].re);
+            o[r].im = __builtin_fma(k, u.im, o[r].im);
+          });
+        }
+      }
+    }
+    if constexpr (APPLY) {
+      cplx<R>* dst = out + uint64_t(blockIdx.y) * a.stride + (origin | lane_off);
+#pragma unroll
+      for (int r = 0; r < kPReg; ++r) {
+        if ((lane | (uint32_t(r) << kPLaneBits)) >= a.valid) continue;
+        acc = __builtin_fma(double(v[r].re), o[r].re, __builtin_fma(double(v[r].im), o[r].im, acc));
+        if (a.accumulate) {
+          o[r].re += double(dst[goff[r]].re);
+          o[r].im += double(dst[goff[r]].im);
+        }
+        dst[goff[r]].re = R(o[r].re);
+        dst[goff[r]].im = R(o[r].im);
+      }
+    }
+    __syncthreads();
+  }
+  const double tot = block_sum(acc, red);
+  if (threadIdx.x == 0 && partial != nullptr)
+    partial[(uint64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = tot;
+}
+
+// A launch being filled: its arguments, and the z masks of its terms.
+struct PauliBatch {
+  PauliTileArgs a;
+  PauliZ zz;
+  uint64_t item_z[kPMaxItems][2];
+  uint64_t diag_z[kPMaxDiag];
+  double diag_k[kPMaxDiag];
+
+  void clear() { std::memset(this, 0, sizeof(*this)); }
+  bool empty() const { return a.nitems == 0 && a.ndiag == 0; }
+
+  // Whether a group (at most 32 terms of one X mask) still fits.
+  bool fits(const PauliGroupArgs& p) const {
+    int odd = 0;
+    for (int i = 0; i < p.nterms; ++i) odd += p.ny[i] & 1;
+    const int even = p.nterms - odd;
+    if (p.x == 0) return a.ndiag + even <= kPMaxDiag && a.nitems + (odd + 1) / 2 <= kPMaxItems;
+    return a.nitems + (odd + 1) / 2 + (even + 1) / 2 <= kPMaxItems;
+  }
+
+  void append(const PauliGroupArgs& p) {
+    for (int odd = 0; odd < 2; ++odd) {
+      int used = 2;  // terms in the current item
+      for (int i = 0; i < p.nterms; ++i) {
+        // (a diagonal product with odd ny is anti-Hermitian: its expectation's
+        // real part is zero, its product with the state an imaginary weight)
+        if ((p.ny[i] & 1) != odd) continue;
+        const bool neg = ((p.ny[i] & 2) != 0) != ((__builtin_popcountll(p.x & p.z[i]) & 1) != 0);
+        const double k = neg ? -p.c[i] : p.c[i];
+        if (p.x == 0 && !odd) {
+          diag_z[a.ndiag] = p.z[i];
+          diag_k[a.ndiag++] = k;
+          continue;
+        }
+        if (used == 2) {
+          PauliItem& g = a.item[a.nitems++];
+          g.x = p.x;
+          g.xl = odd ? kPImag : 0;
+          used = 0;
+        }
+        item_z[a.nitems - 1][used] = p.z[i];
+        a.item[a.nitems - 1].k[used++] = k;
+      }
+    }
+  }
+
+  // Fixes the tile bits (`tmask` and the lowest free index bits up to 12) and
+  // writes the local forms of the terms.
+  void finish(int n, uint64_t tmask) {
+    const int nb = n < kPTileBits ? n : kPTileBits;
+    int have = __builtin_popcountll(tmask);
+    for (int b = 0; b < n && have < nb; ++b)
+      if (!((tmask >> b) & 1)) tmask |= uint64_t(1) << b, ++have;
+    int k = 0;
+    for (int b = 0; b < 64; ++b)
+      if ((tmask >> b) & 1) a.tbits[k++] = uint8_t(b);
+    for (; k < kPTileBits; ++k) a.tbits[k] = uint8_t(k);  // below 12 qubits: bits past the register, never loaded
+    a.valid = uint32_t(1) << nb;
+    a.ntiles = uint64_t(1) << (n - nb);
+    auto localize = [&](uint64_t m) {
+      uint32_t l = 0;
+      for (int i = 0; i < nb; ++i)
+        if ((m >> a.tbits[i]) & 1) l |= uint32_t(1) << i;
+      return l;
+    };
+    auto pattern = [&](uint64_t z) {
+      uint32_t p = 0;
+      for (int r = 0; r < kPReg; ++r)
+        if (__builtin_popcount(uint32_t(r) & (localize(z) >> kPLaneBits)) & 1) p |= 1u << r;
+      return uint16_t(p);
+    };
+    auto put = [&](int bit, uint64_t z) {
+      zz.zout[bit] = z & ~tmask;
+      zz.zl[bit] = uint16_t(localize(z) & ((1u << kPLaneBits) - 1));
+    };
+    int d = 0;
+    for (int c = 0; c < kPReg; ++c) {
+      const int first = d;
+      for (int i = 0; i < a.ndiag; ++i)
+        if ((localize(diag_z[i]) >> kPLaneBits) == uint32_t(c)) {
+          a.dk[d] = diag_k[i];
+          put(d++, diag_z[i]);
+        }
+      a.dcount[c] = uint8_t(d - first);
+    }
+    for (int i = 0; i < a.nitems; ++i) {
+      PauliItem& g = a.item[i];
+      if (g.x & ~tmask)
+        g.xl |= kPFar;
+      else
+        g.xl |= localize(g.x);
+      for (int t = 0; t < 2; ++t) {
+        g.pat[t] = pattern(item_z[i][t]);
+        put(64 + 2 * i + t, item_z[i][t]);
+      }
+    }
+  }
+};
+
+// out[b] = the sum of state b's partials: `count` of each of `nrow` launches,
+// row r of state b at partial[(r * gridDim.x + b) * count].
+__global__ __launch_bounds__(kET) void k_sum_partials(const double* __restrict__ partial, int64_t count, int nrow,
                                                       double* __restrict__ out) {
   __shared__ double lds[kET];
   double acc = 0.0;
-  for (int64_t i = threadIdx.x; i < count; i += kET) acc += partial[i];
+  for (int r = 0; r < nrow; ++r)
+    for (int64_t i = threadIdx.x; i < count; i += kET)
+      acc += partial[(int64_t(r) * gridDim.x + blockIdx.x) * count + i];
   const double tot = block_sum(acc, lds);
-  if (threadIdx.x == 0) out[0] = tot;
+  if (threadIdx.x == 0) out[blockIdx.x] = tot;
 }
 
 static int grid_for(uint64_t nwork) {
@@ -164,19 +575,12 @@ static int expval_impl(const void* state, int n, int nterms, const uint64_t* xm,
   double* partial = reinterpret_cast<double*>(ws);
   int64_t used = 0;
   int rc = QSIM_OK;
-  for_each_group(nterms, xm, zm, ny, c, [&](const PauliGroupArgs& g) {
-    if (rc != QSIM_OK) return;
-    PauliGroupArgs a = g;
-    if (a.x == 0) {
-      a.nwork = uint64_t(1) << n;
-    } else {
-      a.hpos = 63 - __builtin_clzll(a.x);
-      a.hbit = uint64_t(1) << a.hpos;
-      a.nwork = uint64_t(1) << (n - 1);
-    }
-    const int blocks = grid_for(a.nwork);
-    hipLaunchKernelGGL(k_pauli_group<R>, dim3(blocks), dim3(kET), 0, s, reinterpret_cast<const cplx<R>*>(state), a,
-                       partial + used);
+  const uint64_t low = (uint64_t(1) << std::min(n, kPLowBits)) - 1;
+  const int nb = std::min(n, kPTileBits);
+  PauliBatch cur;
+  cur.clear();
+  uint64_t tmask = low;
+  auto launched = [&](int blocks) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
       set_error(std::string(who) + ": launch failed: " + hipGetErrorString(e));
@@ -184,15 +588,54 @@ static int expval_impl(const void* state, int n, int nterms, const uint64_t* xm,
       return;
     }
     used += blocks;
+  };
+  auto flush = [&]() {
+    if (cur.empty()) return;
+    cur.finish(n, tmask);
+    // few tiles: the items are spread over more workgroups
+    const int blocks = int(std::min<uint64_t>(cur.a.ntiles, kEBlocks));
+    int parts = std::max(1, std::min(cur.a.nitems, kESpread / blocks));
+    cur.a.per = std::max(1, (cur.a.nitems + parts - 1) / parts);
+    parts = std::max(1, (cur.a.nitems + cur.a.per - 1) / cur.a.per);
+    hipLaunchKernelGGL((k_pauli_tile<R, false>), dim3(unsigned(blocks), 1, unsigned(parts)), dim3(kET), 0, s,
+                       reinterpret_cast<const cplx<R>*>(state), static_cast<cplx<R>*>(nullptr), cur.a, cur.zz,
+                       partial + used);
+    launched(blocks * parts);
+    cur.clear();
+    tmask = low;
+  };
+  // groups in ascending mask order share a tile pass while their flip bits
+  // (and the lowest bits) fit in 12; a mask that flips too many bits for any
+  // tile takes a pass of its own
+  for_each_group(nterms, xm, zm, ny, c, [&](const PauliGroupArgs& g) {
+    if (rc != QSIM_OK) return;
+    if (__builtin_popcountll(g.x | low) > nb) {
+      PauliGroupArgs a = g;
+      a.hpos = 63 - __builtin_clzll(a.x);
+      a.hbit = uint64_t(1) << a.hpos;
+      a.nwork = uint64_t(1) << (n - 1);
+      const int blocks = grid_for(a.nwork);
+      hipLaunchKernelGGL(k_pauli_group<R>, dim3(blocks), dim3(kET), 0, s, reinterpret_cast<const cplx<R>*>(state), a,
+                         partial + used);
+      launched(blocks);
+      return;
+    }
+    if (__builtin_popcountll(tmask | g.x) > nb || !cur.fits(g)) flush();
+    if (rc != QSIM_OK) return;
+    tmask |= g.x;
+    cur.append(g);
   });
+  if (rc == QSIM_OK) flush();
   if (rc != QSIM_OK) return rc;
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kET), 0, s, partial, used, out);
+  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kET), 0, s, partial, used, 1, out);
   QSIM_CHECK_LAUNCH();
   return QSIM_OK;
 }
 
 // ---------------------------------------------------------------------------
-// out = sum_t c_t P_t psi (gather form, one output amplitude per thread)
+// out = sum_t c_t P_t psi of one state of few tiles (gather form, one output
+// amplitude per thread: more workgroups than tiles; 16 qubits: 15 us against
+// 24 us by tiles, equal at 20 qubits, 23 qubits: 294 us against 207 us)
 // ---------------------------------------------------------------------------
 struct PauliApplyArgs {
   uint64_t n;
@@ -229,6 +672,52 @@ __global__ __launch_bounds__(kET) void k_pauli_apply(const cplx<R>* __restrict__
   }
   out[i].re = R(re);
   out[i].im = R(im);
+}
+
+// ---------------------------------------------------------------------------
+// out = sum_t c_t P_t psi for a batch of states, and <psi|out> beside it
+// ---------------------------------------------------------------------------
+// Launches of a term table (the groups of for_each_group, as many as fit one
+// launch's arguments): at most this many.
+static int apply_launches(int nterms) { return 1 + nterms / 16; }
+
+template <typename R>
+static int apply_impl(const void* state, int nbatch, int n, int nterms, const uint64_t* xm, const uint64_t* zm,
+                      const int* ny, const double* c, void* out, double* energies, double* partial, hipStream_t s,
+                      const char* who) {
+  PauliBatch cur;
+  cur.clear();
+  int rc = QSIM_OK, launches = 0, blocks = 0;
+  auto flush = [&]() {
+    if (cur.empty()) return;
+    cur.finish(n, 0);
+    cur.a.stride = uint64_t(1) << n;
+    cur.a.accumulate = launches > 0;
+    cur.a.per = std::max(1, cur.a.nitems);
+    blocks = int(std::min<uint64_t>(cur.a.ntiles, kEBlocks));
+    double* to = energies ? partial + size_t(launches) * size_t(nbatch) * size_t(blocks) : nullptr;
+    hipLaunchKernelGGL((k_pauli_tile<R, true>), dim3(unsigned(blocks), unsigned(nbatch)), dim3(kET), 0, s,
+                       reinterpret_cast<const cplx<R>*>(state), reinterpret_cast<cplx<R>*>(out), cur.a, cur.zz, to);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      set_error(std::string(who) + ": launch failed: " + hipGetErrorString(e));
+      rc = QSIM_EHIP;
+    }
+    ++launches;
+    cur.clear();
+  };
+  for_each_group(nterms, xm, zm, ny, c, [&](const PauliGroupArgs& g) {
+    if (rc != QSIM_OK) return;
+    if (!cur.fits(g)) flush();
+    if (rc != QSIM_OK) return;
+    cur.append(g);
+  });
+  if (rc == QSIM_OK) flush();
+  if (rc != QSIM_OK || !energies) return rc;
+  hipLaunchKernelGGL(k_sum_partials, dim3(unsigned(nbatch)), dim3(kET), 0, s, partial, int64_t(blocks), launches,
+                     energies);
+  QSIM_CHECK_LAUNCH();
+  return QSIM_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -291,7 +780,7 @@ static int launch_inner(const void* bra, const void* ket, int n, const int* targ
   hipLaunchKernelGGL((k_inner<R, NT>), dim3(blocks), dim3(kET), 0, s, reinterpret_cast<const cplx<R>*>(bra),
                      reinterpret_cast<const cplx<R>*>(ket), a, partial);
   QSIM_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kET), 0, s, partial, int64_t(blocks), out);
+  hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(kET), 0, s, partial, int64_t(blocks), 1, out);
   QSIM_CHECK_LAUNCH();
   return QSIM_OK;
 }
@@ -423,28 +912,65 @@ int qsim_apply_pauli_sum(const void* state, int nqubits, int dtype, int nterms, 
   for (int t = 0; t < nterms; ++t)
     QSIM_CHECK_ARG((xmasks[t] & ~full) == 0 && (zmasks[t] & ~full) == 0, "qsim_apply_pauli_sum: mask out of range");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const uint64_t N = uint64_t(1) << nqubits;
-  for (int t0 = 0; t0 < nterms; t0 += 64) {
-    PauliApplyArgs a;
-    std::memset(&a, 0, sizeof(a));
-    a.n = N;
-    a.nterms = std::min(64, nterms - t0);
-    for (int t = 0; t < a.nterms; ++t) {
-      a.x[t] = xmasks[t0 + t];
-      a.z[t] = zmasks[t0 + t];
-      a.c[t] = coeffs[t0 + t];
-      a.ny[t] = ny[t0 + t];
+  if (nqubits < kPTileBits + 8) {  // fewer tiles than CUs
+    const uint64_t N = uint64_t(1) << nqubits;
+    for (int t0 = 0; t0 < nterms; t0 += 64) {
+      PauliApplyArgs a;
+      std::memset(&a, 0, sizeof(a));
+      a.n = N;
+      a.nterms = std::min(64, nterms - t0);
+      for (int t = 0; t < a.nterms; ++t) {
+        a.x[t] = xmasks[t0 + t];
+        a.z[t] = zmasks[t0 + t];
+        a.c[t] = coeffs[t0 + t];
+        a.ny[t] = ny[t0 + t];
+      }
+      const int acc = t0 > 0 ? 1 : 0;
+      if (dtype == QSIM_C128)
+        hipLaunchKernelGGL(k_pauli_apply<double>, launch_grid(ceil_div_u(N, kET)), dim3(kET), 0, s, (const c128*)state,
+                           (c128*)out, a, acc);
+      else
+        hipLaunchKernelGGL(k_pauli_apply<float>, launch_grid(ceil_div_u(N, kET)), dim3(kET), 0, s, (const c64*)state,
+                           (c64*)out, a, acc);
+      QSIM_CHECK_LAUNCH();
     }
-    const int acc = t0 > 0 ? 1 : 0;
-    if (dtype == QSIM_C128)
-      hipLaunchKernelGGL(k_pauli_apply<double>, launch_grid(ceil_div_u(N, kET)), dim3(kET), 0, s, (const c128*)state,
-                         (c128*)out, a, acc);
-    else
-      hipLaunchKernelGGL(k_pauli_apply<float>, launch_grid(ceil_div_u(N, kET)), dim3(kET), 0, s, (const c64*)state,
-                         (c64*)out, a, acc);
-    QSIM_CHECK_LAUNCH();
+    return QSIM_OK;
   }
-  return QSIM_OK;
+  if (dtype == QSIM_C128)
+    return apply_impl<double>(state, 1, nqubits, nterms, xmasks, zmasks, ny, coeffs, out, nullptr, nullptr, s,
+                              "qsim_apply_pauli_sum");
+  return apply_impl<float>(state, 1, nqubits, nterms, xmasks, zmasks, ny, coeffs, out, nullptr, nullptr, s,
+                           "qsim_apply_pauli_sum");
+}
+
+size_t qsim_apply_pauli_sum_batched_workspace(int nbatch, int nterms) {
+  if (nbatch < 1 || nterms < 1) return 0;
+  return size_t(apply_launches(nterms)) * size_t(nbatch) * kEBlocks * sizeof(double);
+}
+
+int qsim_apply_pauli_sum_batched(const void* states, int nbatch, int nqubits, int dtype, int nterms,
+                                 const uint64_t* xmasks, const uint64_t* zmasks, const int* ny, const double* coeffs,
+                                 void* out, double* energies, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  const char* who = "qsim_apply_pauli_sum_batched";
+  QSIM_CHECK_ARG(states != nullptr && out != nullptr && states != out && energies != nullptr && workspace != nullptr,
+                 "qsim_apply_pauli_sum_batched: bad pointers");
+  QSIM_CHECK_ARG(dtype == QSIM_C128 || dtype == QSIM_C64, "qsim_apply_pauli_sum_batched: bad dtype");
+  QSIM_CHECK_ARG(nqubits >= 1 && nqubits <= QSIM_MAX_QUBITS, "qsim_apply_pauli_sum_batched: nqubits out of range");
+  QSIM_CHECK_ARG(nbatch >= 1 && nbatch <= 65535, "qsim_apply_pauli_sum_batched: 1..65535 states");
+  QSIM_CHECK_ARG(nterms >= 1 && xmasks && zmasks && ny && coeffs, "qsim_apply_pauli_sum_batched: bad term table");
+  const uint64_t full = (uint64_t(1) << nqubits) - 1;
+  for (int t = 0; t < nterms; ++t)
+    QSIM_CHECK_ARG((xmasks[t] & ~full) == 0 && (zmasks[t] & ~full) == 0,
+                   "qsim_apply_pauli_sum_batched: mask out of range");
+  QSIM_CHECK_ARG(workspace_bytes >= qsim_apply_pauli_sum_batched_workspace(nbatch, nterms),
+                 "qsim_apply_pauli_sum_batched: workspace too small");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  double* partial = reinterpret_cast<double*>(workspace);
+  if (dtype == QSIM_C128)
+    return apply_impl<double>(states, nbatch, nqubits, nterms, xmasks, zmasks, ny, coeffs, out, energies, partial, s,
+                              who);
+  return apply_impl<float>(states, nbatch, nqubits, nterms, xmasks, zmasks, ny, coeffs, out, energies, partial, s, who);
 }
 
 int qsim_inner_matrix(const void* bra, const void* ket, int nqubits, int dtype, const int* targets, int ntargets,
