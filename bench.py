@@ -724,7 +724,7 @@ def main():
     from qibo_amd import blocking
 
     ops = [backend.plan_gate(g) for g in circuit.queue if g.__class__.__name__ != "M"]
-    plan, program = blocking.compile_circuit(ops, n, np.complex128, 3)
+    plan, program = blocking.compile_circuit(ops, n, np.complex128, 3, device=True)
     pass_flops = [blocking.program_flops(program[e[2]:], e[3], 16) for e in plan if e[0] == "block"]
     step_dense = [d for _, d in launch_bytes[: len(pass_flops)]]
     if len(step_dense) == len(pass_flops) and any(step_dense):  # the passes over every tile

@@ -495,6 +495,17 @@ int qsim_compile_pass(int nqubits, const int* tile_bits, int nops, const int* op
                       const int64_t* data_offsets, int dtype, int ordered, uint8_t* out, size_t capacity,
                       size_t* out_bytes, int* count, int* switches);
 
+/* The same gates compiled into the form the backend runs by default: register
+ * bits chosen freely among the tile bits (layouts), two-qubit gates in
+ * registers, SWAPs as renamed bits, rotations divided by their cosines. Equal
+ * to qsim_compile_pass up to rounding. `low_bits` = the lowest index bits the
+ * pass keeps in its tile (stored in whole lines). Capacity: at least
+ * qsim_compile_program_capacity(nops, dtype) bytes. No device work. */
+size_t qsim_compile_program_capacity(int nops, int dtype);
+int qsim_compile_program(int nqubits, const int* tile_bits, int nops, const int* op_desc, const double* op_data,
+                         const int64_t* data_offsets, int dtype, int low_bits, uint8_t* out, size_t capacity,
+                         size_t* out_bytes, int* count, int* switches);
+
 /* Neighbour-fusion planner of Circuit.fuse (circuit.py:954-1003, with
  * _Queue.to_fused / from_fused :55-95 and FusedGate.can_fuse / fuse
  * gates/special.py:81-153), host code. Gate i of the queue acts on the qubits

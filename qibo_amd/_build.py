@@ -31,6 +31,7 @@ SOURCES = {
     "density.hip": ["-ffp-contract=off"],
     "planner.hip": [],
     "compile.hip": ["-ffp-contract=off"],
+    "program.hip": ["-ffp-contract=off"],
     "fuse.hip": ["-ffp-contract=off"],
     "compare.hip": [],
     # run-time specialised blocked passes: the device headers' text is

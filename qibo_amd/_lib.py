@@ -87,6 +87,8 @@ SIGNATURES = {
     "qsim_dm_expval_workspace": (_sz, [_i]),
     "qsim_dm_expval_pauli": (_i, [_vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "qsim_plan_pass": (_i, [_i, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]),
+    "qsim_compile_program_capacity": (_sz, [_i, _i]),
+    "qsim_compile_program": (_i, [_i, _c_int_p, _i, _vp, _vp, _vp, _i, _i, _vp, _sz, _vp, _vp, _vp]),
     "qsim_compile_pass_capacity": (_sz, [_i, _i]),
     "qsim_fuse_plan": (_i, [_i, _i, _vp, _vp, _i, _vp, _vp, _vp]),
     "qsim_matrix_fused": (_i, [_i, _c_int_p, _i, _vp, _vp, _vp, _vp]),

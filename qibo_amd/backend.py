@@ -1300,7 +1300,7 @@ class MI355XBackend(GatePlanner):
                     record.append(("single", payload))
                 continue
             tile_bits, pops = payload
-            program, count, _ = blocking.compile_pass(tile_bits, pops, nqubits, cdtype, ordered)
+            program, count = blocking.compile_program(tile_bits, pops, nqubits, cdtype, low, ordered)
             # zero padding: the kernel may read QSIM_BLOCKED_PAD bytes past the stream
             host = torch.frombuffer(bytearray(program) + bytes(blocking.PAD_BYTES), dtype=torch.uint8).pin_memory()
             prog = host.to(state.device, non_blocking=True)

@@ -79,6 +79,8 @@ PAD_BYTES = 1056  # readable bytes required past a record stream (QSIM_BLOCKED_P
 OP_DIAG, OP_DENSE1, OP_MAP, OP_DENSE_LDS = 0, 1, 2, 3
 OP_DENSE1_REAL, OP_REG_PHASE, OP_LANE_PHASE, OP_NEG = 4, 5, 6, 7
 OP_ROT = 10
+OP_ROTS, OP_DENSE2, OP_FLIP = 13, 14, 15  # compile_program's further forms (csrc/program.hip)
+MAP_LAYOUT, MAP_START, MAP_RELABEL = 3, 4, 5  # MAP arguments that carry layouts
 ROT_RY, ROT_H, ROT_RX = 0, 1, 2  # ROT modes (arg = register bit | mode << 2)
 OP_LANE_REGPHASE, OP_QFLUSH = 11, 12
 OP_NOP = 0xFF  # header only, no effect: pads programs of a batched launch to one record count
@@ -504,7 +506,10 @@ def _desc(op):
     return cached
 
 
-def _compile_pass_native(tile_bits, ops, nqubits, cdtype, ordered):
+def _native_compile(capacity, entry, tile_bits, ops, nqubits, cdtype, option):
+    """Planned ops through one of the library's compilers (``capacity`` and
+    ``entry`` its C entry points, ``option`` the integer between the dtype and
+    the output buffer): (program bytes, record count, layout changes)."""
     from . import _lib
 
     lib = _lib.load()
@@ -523,14 +528,31 @@ def _compile_pass_native(tile_bits, ops, nqubits, cdtype, ordered):
     data = np.concatenate(datas) if datas else np.zeros(1, dtype=np.complex128)
     offs = np.asarray(offs if offs else [-1], dtype=np.int64)
     code = _lib.C64 if np.dtype(cdtype) == np.complex64 else _lib.C128
-    cap = lib.qsim_compile_pass_capacity(len(ops), code)
+    cap = getattr(lib, capacity)(len(ops), code)
     out = np.empty(cap, dtype=np.uint8)
     nbytes, count, switches = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
-    rc = lib.qsim_compile_pass(nqubits, _lib.int_array(tile_bits), len(ops), desc.ctypes.data, data.ctypes.data,
-                               offs.ctypes.data, code, 1 if ordered else 0, out.ctypes.data, cap,
-                               ctypes.byref(nbytes), ctypes.byref(count), ctypes.byref(switches))
+    rc = getattr(lib, entry)(nqubits, _lib.int_array(tile_bits), len(ops), desc.ctypes.data, data.ctypes.data,
+                             offs.ctypes.data, code, option, out.ctypes.data, cap, ctypes.byref(nbytes),
+                             ctypes.byref(count), ctypes.byref(switches))
     _lib.check(rc, lib)
     return out[: nbytes.value].tobytes(), count.value, switches.value
+
+
+def _compile_pass_native(tile_bits, ops, nqubits, cdtype, ordered):
+    return _native_compile("qsim_compile_pass_capacity", "qsim_compile_pass", tile_bits, ops, nqubits, cdtype,
+                           1 if ordered else 0)
+
+
+def compile_program(tile_bits: Sequence[int], ops: Sequence, nqubits: int, cdtype, low_bits: int,
+                    ordered: bool = False) -> Tuple[bytes, int]:
+    """(program, record count) of one blocked pass as the backend runs it:
+    qsim_compile_program's records (free layouts, two-qubit gates in
+    registers, scaled rotations), or with ``ordered`` compile_pass's exact
+    per-gate forms in circuit order."""
+    if ordered:
+        return compile_pass(tile_bits, ops, nqubits, cdtype, True)[:2]
+    return _native_compile("qsim_compile_program_capacity", "qsim_compile_program", tile_bits, ops, nqubits, cdtype,
+                           int(low_bits))[:2]
 
 
 def compile_pass(tile_bits: Sequence[int], ops: Sequence, nqubits: int, cdtype,
@@ -859,12 +881,14 @@ def compile_pass_batched(tile_bits: Sequence[int], ops: Sequence, nqubits: int, 
 # FP64/FP32 floating-point operations per amplitude of the tile that each
 # record form performs (multiply = 1, fused multiply-add = 2), as the kernel
 # executes them: real 2x2: 2 mul + 2 fma per component; rotation: 3 fma per
-# real pair; complex 2x2: a complex
+# real pair (scaled: 2 fma); complex 2x2: a complex
 # multiply (6) and a complex multiply-add (8); diagonal / table: a complex
 # multiply; a per-lane factor: one complex multiply per 16 amplitudes;
 # dense 2^k block: 6 + 8 (2^k - 1).
 _FLOPS = {OP_DENSE1_REAL: 6.0, OP_ROT: 6.0, OP_LANE_REGPHASE: 6.0 / 16, OP_QFLUSH: 3.0, OP_DENSE1: 14.0, OP_DIAG: 6.0, OP_REG_PHASE: 6.0, OP_LANE_PHASE: 6.0 / 16,
-          OP_NEG: 0.0, OP_MAP: 0.0}
+          OP_NEG: 0.0, OP_MAP: 0.0, OP_ROTS: 4.0, OP_FLIP: 0.0}
+# 4x4 in registers, by kind (arg >> 3): complex, real, complex and real on the pairs (00, 11), (01, 10)
+_DENSE2_FLOPS = (30.0, 14.0, 14.0, 6.0)
 
 
 def program_flops(program: bytes, count: int, itemsize: int) -> float:
@@ -875,6 +899,8 @@ def program_flops(program: bytes, count: int, itemsize: int) -> float:
         nent = int.from_bytes(program[off + 4: off + 8], "little")
         if op == OP_DENSE_LDS:
             total += 6.0 + 8.0 * (2**arg - 1)
+        elif op == OP_DENSE2:
+            total += _DENSE2_FLOPS[min(arg >> 3, 3)]
         elif op == OP_REG_PHASE and arg & 15:
             total += 6.0 * int(_REG_DEP[arg & 15].sum()) / 16
         else:
@@ -883,9 +909,10 @@ def program_flops(program: bytes, count: int, itemsize: int) -> float:
     return total
 
 
-def compile_circuit(ops: Sequence, nqubits: int, cdtype, low_bits: int, ordered: bool = False):
+def compile_circuit(ops: Sequence, nqubits: int, cdtype, low_bits: int, ordered: bool = False, device: bool = False):
     """Partition and compile: a list of ("single", op) / ("block", tile_bits, byte_offset,
-    count, ngates) plus the concatenated records of all blocked passes."""
+    count, ngates) plus the concatenated records of all blocked passes. With
+    ``device`` the passes are compile_program's, the ones the backend runs."""
     plan = []
     program = bytearray()
     for kind, payload in partition(ops, nqubits, low_bits, ordered):
@@ -893,7 +920,10 @@ def compile_circuit(ops: Sequence, nqubits: int, cdtype, low_bits: int, ordered:
             plan.append(("single", payload))
             continue
         tile_bits, pops = payload
-        code, count, _ = compile_pass(tile_bits, pops, nqubits, cdtype, ordered)
+        if device:
+            code, count = compile_program(tile_bits, pops, nqubits, cdtype, low_bits, ordered)
+        else:
+            code, count, _ = compile_pass(tile_bits, pops, nqubits, cdtype, ordered)
         plan.append(("block", tuple(tile_bits), len(program), count, len(pops)))
         program.extend(code)
     return plan, bytes(program)

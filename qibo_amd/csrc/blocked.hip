@@ -31,6 +31,10 @@
 //                   next MAP / DENSE_LDS / store (it commutes with everything
 //                   that stays inside the lane's registers)
 //   NEG (7)         v = -v (the -1 phase of CZ-like gates)
+//   ROT (10), ROTS (13)  rotations as three shears, or divided by their cosine
+//   LANE_REGPHASE (11), QFLUSH (12)  controlled phases of a register bit
+//   DENSE2 (14)     4x4 on two register bits; FLIP (15) X under conditions
+// MAP may also name any layout of the local bits (blocked_dev.h).
 // Conditions: `tmask` = condition bits outside the tile (the same for the
 // whole tile: a record whose tmask fails is skipped by the workgroup);
 // `cmask` = condition bits inside the tile that select lanes (DENSE_LDS: all
@@ -52,6 +56,17 @@
 
 namespace qsim {
 
+template <typename R, int PAIR>
+__device__ __forceinline__ void dense2_kind(cplx<R>* v, const cplx<R>* m, uint32_t kind) {
+  constexpr int HI = kPairHi[PAIR], LO = kPairLo[PAIR];
+  switch (kind) {
+    case 0: dense2_regs<R, HI, LO, 0>(v, m); break;
+    case 1: dense2_regs<R, HI, LO, 1>(v, m); break;
+    case 2: dense2_regs<R, HI, LO, 2>(v, m); break;
+    default: dense2_regs<R, HI, LO, 3>(v, m); break;
+  }
+}
+
 // FROM_ZERO: the input is |0...0>, generated in registers (the state is only written).
 template <typename R, bool FROM_ZERO>
 __global__ __launch_bounds__(kBT) __attribute__((amdgpu_waves_per_eu(QSIM_BLOCKED_WAVES)))
@@ -62,24 +77,29 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
   if (tile >= a.ntiles) return;
   psi += blockIdx.z * a.state_stride;  // state and program of this batch entry
   prog += blockIdx.z * a.prog_stride;
-  uint64_t gbit[kBTileBits];
-#pragma clang loop unroll(full)
-  for (int i = 0; i < kBTileBits; ++i) gbit[i] = uint64_t(1) << a.tbits[i];
   const uint64_t tile_base = tile_origin(a, tile);
 
-  int map = 0;
+  // the layout the tile is loaded in: a program's first record may name it
+  uint64_t layout = kLayout0;
+  Hdr h = {};
+  if (a.ninstr > 0) h = load_hdr(prog);
+  if (h.op == kOpMap && h.arg == kMapStart) layout = h.cmask;
   // global index of the lane's amplitudes with the register bits cleared
-  uint64_t lane_idx = tile_base | deposit(local_index(0, threadIdx.x, 0), gbit);
+  uint64_t lane_idx = tile_base | lay_lane_index(a, layout);
 
   cplx<R> v[kBReg];
-  if constexpr (FROM_ZERO) {
+  {
+    uint64_t rb[4];
+    lay_reg_bits(a, layout, rb);
+    if constexpr (FROM_ZERO) {
 #pragma clang loop unroll(full)
-    for (int r = 0; r < kBReg; ++r) {
-      v[r].re = (lane_idx | deposit(uint32_t(r) << 8, gbit)) == 0 ? R(1) : R(0);
-      v[r].im = R(0);
+      for (int r = 0; r < kBReg; ++r) {
+        v[r].re = (lane_idx | reg_index(rb, r)) == 0 ? R(1) : R(0);
+        v[r].im = R(0);
+      }
+    } else {
+      load_lane(a, psi, lane_idx, layout, rb, v);
     }
-  } else {
-    load_lane(a, psi, lane_idx, gbit, v);
   }
 
   cplx<R> P;  // pending per-lane factor of LANE_PHASE records
@@ -103,8 +123,6 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
   const uint64_t tb_hi = __builtin_amdgcn_readfirstlane(uint32_t(tile_base >> 32));
   const uint64_t tile_base_s = tb_lo | (tb_hi << 32);  // uniform copy (scalar registers)
   uint32_t off = 0;
-  Hdr h = {};
-  if (a.ninstr > 0) h = load_hdr(prog);
   for (int k = 0; k < a.ninstr && off + uint32_t(sizeof(BlkHdr)) <= nbytes; ++k) {
     const cplx<R>* m = reinterpret_cast<const cplx<R>*>(prog + off + sizeof(BlkHdr));
     const uint32_t nent = h.nent < kMaxEntries ? h.nent : kMaxEntries;  // no record is larger
@@ -173,6 +191,35 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
         }
         break;
       }
+      case kOpRotS: {
+        const R t = rots_t<R>(h);
+        const uint32_t mode = h.arg >> 2;
+        switch (h.arg & 3) {
+          case 0: rots_regs<R, 0>(v, mode, t); break;
+          case 1: rots_regs<R, 1>(v, mode, t); break;
+          case 2: rots_regs<R, 2>(v, mode, t); break;
+          default: rots_regs<R, 3>(v, mode, t); break;
+        }
+        break;
+      }
+      case kOpDense2:
+        switch (h.arg & 7) {
+          case 0: dense2_kind<R, 0>(v, m, h.arg >> 3); break;
+          case 1: dense2_kind<R, 1>(v, m, h.arg >> 3); break;
+          case 2: dense2_kind<R, 2>(v, m, h.arg >> 3); break;
+          case 3: dense2_kind<R, 3>(v, m, h.arg >> 3); break;
+          case 4: dense2_kind<R, 4>(v, m, h.arg >> 3); break;
+          default: dense2_kind<R, 5>(v, m, h.arg >> 3); break;
+        }
+        break;
+      case kOpFlip:
+        switch (h.arg & 3) {
+          case 0: flip_regs<R, 0>(v, h, lane_idx); break;
+          case 1: flip_regs<R, 1>(v, h, lane_idx); break;
+          case 2: flip_regs<R, 2>(v, h, lane_idx); break;
+          default: flip_regs<R, 3>(v, h, lane_idx); break;
+        }
+        break;
       case kOpRegPhase:
         switch (h.arg & 15) {
           case 0: reg_phase<R, 0>(v, m); break;
@@ -221,22 +268,30 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
         diag_regs(v, h, m, lane_idx, lane_ok());
         break;
       case kOpMap: {
-        flush_lane_phase(v, P, pdirty);
-        const int nmap = h.arg < 3 ? int(h.arg) : 0;
-        remap(lds, v, map, nmap);
-        map = nmap;
-        lane_idx = tile_base | deposit(local_index(map, threadIdx.x, 0), gbit);
+        if (h.arg == kMapStart) break;  // (applied before the load)
+        if (h.arg == kMapRelabel) {
+          relabel_fence(v);
+          layout = h.cmask;
+        } else {
+          flush_lane_phase(v, P, pdirty);
+          const bool given = h.arg == kMapLayout;
+          const uint64_t from = given ? (uint64_t(h.b0) | (uint64_t(h.b1) << 32)) : layout;
+          const uint64_t to = given ? h.cmask : map_layout(h.arg);
+          lay_remap(lds, v, from, to);
+          layout = to;
+        }
+        lane_idx = tile_base | lay_lane_index(a, layout);
         break;
       }
       case kOpDenseLds: {
         flush_lane_phase(v, P, pdirty);
         const uint32_t kk = h.arg;
         if (kk <= 1)
-          dense_lds<R, 1>(lds, v, map, h, m, tile_base, gbit);
+          dense_lds<R, 1>(lds, v, layout, h, m, tile_base, a);
         else if (kk == 2)
-          dense_lds<R, 2>(lds, v, map, h, m, tile_base, gbit);
+          dense_lds<R, 2>(lds, v, layout, h, m, tile_base, a);
         else
-          dense_lds<R, 3>(lds, v, map, h, m, tile_base, gbit);
+          dense_lds<R, 3>(lds, v, layout, h, m, tile_base, a);
         break;
       }
       default:
@@ -246,16 +301,18 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
   }
 
   flush_lane_phase(v, P, pdirty);
-  if (map != 0) {
-    remap(lds, v, map, 0);
-    map = 0;
-    lane_idx = tile_base | deposit(local_index(0, threadIdx.x, 0), gbit);
+  if (lay_low_in_regs(layout)) {  // lines are stored whole
+    lay_remap(lds, v, layout, kLayout0);
+    layout = kLayout0;
   }
-  // recompute the store addresses here instead of keeping the load addresses
+  // the store addresses are formed here instead of keeping the load addresses
   // live through the instruction loop (which spilled them to scratch)
+  lane_idx = tile_base | lay_lane_index(a, layout);
   asm volatile("" : "+v"(lane_idx));
+  uint64_t rb[4];
+  lay_reg_bits(a, layout, rb);
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) st_nt(psi, lane_idx | deposit(uint32_t(r) << 8, gbit), v[r]);
+  for (int r = 0; r < kBReg; ++r) st_nt(psi, lane_idx | reg_index(rb, r), v[r]);
 }
 
 // The tiles of a pass with tile bits `tbits` over n qubits whose input

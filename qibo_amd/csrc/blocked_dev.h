@@ -30,13 +30,17 @@ enum : uint32_t {
                      // no entries: t, s in the header (cmask, bits fields), float64 or float32
   kOpLaneRegPhase = 11,  // per-lane factor Q of the registers with one bit set (kept in LDS)
   kOpQFlush = 12,        // apply Q to the registers with bit arg set, reset it to 1
+  kOpRotS = 13,          // a rotation divided by its cosine (see rots_regs): tan in the header (cmask field)
+  kOpDense2 = 14,        // 4x4 on two register bits: arg = pair (kPairHi/Lo) | kind << 3, 16 entries
+  kOpFlip = 15,          // X on register bit arg under conditions
   kOpNop = 0xFF          // no effect (pads the programs of a batched launch to one record count)
 };
 
 // Record header (the host packs the same layout).
 struct BlkHdr {
   uint8_t op;
-  uint8_t arg;       // DENSE1*: register bit 0..3; ROT: bit | mode << 2; MAP: mapping 0..2; DENSE_LDS: number of targets 1..3
+  uint8_t arg;       // DENSE1*: register bit 0..3; ROT: bit | mode << 2; MAP: mapping 0..2 or kMapLayout.. (see
+                     // there); DENSE_LDS: number of targets 1..3
   uint8_t nt;        // DIAG / LANE_PHASE: number of target bits (0..5)
   uint8_t rreq;      // register-bit conditions (bit j: register bit j must be 1)
   uint32_t nent;     // complex entries following the header
@@ -171,6 +175,47 @@ __device__ __forceinline__ uint32_t local_index(int map, uint32_t lane, uint32_t
 // own part XOR a per-register constant.
 __device__ __forceinline__ uint32_t swz(uint32_t u) { return u ^ ((u >> 4) & 15u) ^ (((u >> 8) & 3u) << 4); }
 
+// ---------------------------------------------------------------------------
+// Layouts. A pass's 12 local bits sit at 12 positions: positions 0-7 are the
+// bits of the lane number, 8-11 the bits of the register number. A layout is
+// 12 nibbles, nibble p = the local bit at position p. Mappings 0-2 are three
+// of them; a compiled program may use any (MAP records with the arguments
+// below carry the layouts in their header):
+//   kMapLayout   from the layout in `bits` to the one in `cmask`, through LDS
+//   kMapStart    the layout the tile is loaded in (first record of a program)
+//   kMapRelabel  the local bits at the positions change names (a SWAP gate on
+//                them: no data moves), the layout from then on in `cmask`
+// Whatever the layout, the amplitude at local index u lives at LDS slot(u)
+// during an exchange.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kMapLayout = 3, kMapStart = 4, kMapRelabel = 5;
+constexpr uint64_t kLayout0 = 0xBA9876543210ull;  // registers: local bits 8-11
+constexpr uint64_t kLayout1 = 0x7654BA983210ull;  // local bits 4-7
+constexpr uint64_t kLayout2 = 0x3210BA987654ull;  // local bits 0-3
+
+__device__ __forceinline__ uint64_t map_layout(uint32_t map) {
+  return map == 1 ? kLayout1 : (map == 2 ? kLayout2 : kLayout0);
+}
+
+__device__ __forceinline__ uint32_t lay_bit(uint64_t L, int p) { return uint32_t(L >> (4 * p)) & 15u; }
+
+// Whether a register position holds one of the lowest 3 local bits: the
+// tile's lines are then split between registers, and it is not stored so.
+__device__ __forceinline__ bool lay_low_in_regs(uint64_t L) {
+  return lay_bit(L, 8) < 3 || lay_bit(L, 9) < 3 || lay_bit(L, 10) < 3 || lay_bit(L, 11) < 3;
+}
+
+// XOR swizzle of the layout exchanges: the low 5 slot bits of local bits 0-11
+// are 1, 2, 4, 8, 16, 1, 2, 4, 16, 8, 31, 30 (the residues of the additive
+// layout's weights below), so a half-wave hits 32 distinct pairs of banks in
+// every layout whose lane positions 0-4 hold bits of five different kinds
+// {0,5,10} {1,6,11} {2,7} {3,9} {4,8}; the compiler orders them so. Linear over
+// GF(2) and a bijection (bits 5-11 are kept).
+__device__ __forceinline__ uint32_t swl(uint32_t u) {
+  return u ^ ((u >> 5) & 7u) ^ (((u >> 8) & 1u) << 4) ^ (((u >> 9) & 1u) << 3) ^ (((u >> 10) & 1u) * 31u) ^
+         (((u >> 11) & 1u) * 30u);
+}
+
 // LDS slots of 8-byte components: an additive layout, slot(u) = the sum of
 // kSlotW[i] over the set bits i of u (u + 1, 2, 4 for bits 5-7 and + 16, 40,
 // 63, 126 for bits 8-11). The weights grow faster than the sum of the smaller
@@ -222,6 +267,79 @@ struct LdsSlots {
   __device__ static __forceinline__ uint32_t join(uint32_t sa, uint32_t sb) { return kAdd ? sa + sb : sa ^ sb; }
 };
 
+// Slots in the layout exchanges: the additive layout where LdsSlots has it,
+// the swizzle `swl` otherwise.
+template <typename R>
+__device__ __forceinline__ uint32_t lay_slot(uint32_t u) {
+  return LdsSlots<R>::kAdd ? slot_f64(u) : swl(u);
+}
+
+// All-ones where bit p of the lane number is set.
+__device__ __forceinline__ uint32_t lane_mask(int p) { return uint32_t(int32_t(threadIdx.x << (31 - p)) >> 31); }
+
+// Slot of the lane's part of a layout, and of a register's part.
+template <typename R>
+__device__ __forceinline__ uint32_t lay_lane_slot(uint64_t L) {
+  uint32_t s = 0;
+#pragma clang loop unroll(full)
+  for (int p = 0; p < 8; ++p) s = LdsSlots<R>::join(s, lane_mask(p) & lay_slot<R>(1u << lay_bit(L, p)));
+  return s;
+}
+
+template <typename R>
+__device__ __forceinline__ uint32_t lay_reg_slot(uint64_t L, uint32_t r) {
+  uint32_t s = 0;
+#pragma clang loop unroll(full)
+  for (int j = 0; j < 4; ++j)
+    if ((r >> j) & 1) s = LdsSlots<R>::join(s, lay_slot<R>(1u << lay_bit(L, 8 + j)));
+  return s;
+}
+
+// The local bits of the lane's amplitudes (registers zero).
+__device__ __forceinline__ uint32_t lay_lane_local(uint64_t L) {
+  uint32_t u = 0;
+#pragma clang loop unroll(full)
+  for (int p = 0; p < 8; ++p) u |= lane_mask(p) & (1u << lay_bit(L, p));
+  return u;
+}
+
+__device__ __forceinline__ uint32_t lay_reg_local(uint64_t L, uint32_t r) {
+  uint32_t u = 0;
+#pragma clang loop unroll(full)
+  for (int j = 0; j < 4; ++j)
+    if ((r >> j) & 1) u |= 1u << lay_bit(L, 8 + j);
+  return u;
+}
+
+// Global index bits: of a local bit, of the lane's part, of a register's part.
+__device__ __forceinline__ uint64_t lay_gbit(const BlkArgs& a, uint32_t b) {
+  // (dwords of the argument block: it has no scalar byte loads)
+  const uint32_t* w = reinterpret_cast<const uint32_t*>(a.tbits);
+  const uint32_t d = b < 4 ? w[0] : (b < 8 ? w[1] : w[2]);
+  return uint64_t(1) << ((d >> (8 * (b & 3))) & 63u);
+}
+
+__device__ __forceinline__ uint64_t lay_lane_index(const BlkArgs& a, uint64_t L) {
+  uint32_t lo = 0, hi = 0;
+#pragma clang loop unroll(full)
+  for (int p = 0; p < 8; ++p) {
+    const uint64_t g = lay_gbit(a, lay_bit(L, p));
+    const uint32_t m = lane_mask(p);
+    lo |= m & uint32_t(g);
+    hi |= m & uint32_t(g >> 32);
+  }
+  return uint64_t(lo) | (uint64_t(hi) << 32);
+}
+
+__device__ __forceinline__ void lay_reg_bits(const BlkArgs& a, uint64_t L, uint64_t* rb) {
+#pragma clang loop unroll(full)
+  for (int j = 0; j < 4; ++j) rb[j] = lay_gbit(a, lay_bit(L, 8 + j));
+}
+
+__device__ __forceinline__ uint64_t reg_index(const uint64_t* rb, int r) {
+  return ((r & 1) ? rb[0] : 0) | ((r & 2) ? rb[1] : 0) | ((r & 4) ? rb[2] : 0) | ((r & 8) ? rb[3] : 0);
+}
+
 // Local index of register 0 of `lane` under mapping `map` (register bits zero).
 __device__ __forceinline__ uint32_t lane_local(int map, uint32_t lane) { return local_index(map, lane, 0); }
 
@@ -234,20 +352,21 @@ __device__ __forceinline__ uint64_t deposit(uint32_t u, const uint64_t* gbit) {
   return g;
 }
 
-// The lane's amplitudes under mapping 0 (lane_idx: their global index with
-// the register bits cleared), reading only those inside the support.
+// The lane's amplitudes under layout L (lane_idx: their global index with
+// the register bits cleared, rb: the register bits), reading only those
+// inside the support.
 template <typename R>
-__device__ __forceinline__ void load_lane(const BlkArgs& a, const cplx<R>* psi, uint64_t lane_idx,
-                                          const uint64_t* gbit, cplx<R>* v) {
+__device__ __forceinline__ void load_lane(const BlkArgs& a, const cplx<R>* psi, uint64_t lane_idx, uint64_t L,
+                                          const uint64_t* rb, cplx<R>* v) {
   if (a.zload == 0) {
 #pragma clang loop unroll(full)
-    for (int r = 0; r < kBReg; ++r) v[r] = ld_nt(psi, lane_idx | deposit(uint32_t(r) << 8, gbit));
+    for (int r = 0; r < kBReg; ++r) v[r] = ld_nt(psi, lane_idx | reg_index(rb, r));
   } else {
-    const uint32_t lz = local_index(0, threadIdx.x, 0) & a.zload;
+    const uint32_t lz = lay_lane_local(L) & a.zload;
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r) {
-      if ((lz | ((uint32_t(r) << 8) & a.zload)) == 0)
-        v[r] = ld_nt(psi, lane_idx | deposit(uint32_t(r) << 8, gbit));
+      if ((lz | (lay_reg_local(L, uint32_t(r)) & a.zload)) == 0)
+        v[r] = ld_nt(psi, lane_idx | reg_index(rb, r));
       else
         v[r] = cplx<R>{R(0), R(0)};
     }
@@ -356,6 +475,79 @@ __device__ __forceinline__ void remap(R* lds, cplx<R>* v, int from, int to) {
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) v[r].im = x[r];
+}
+
+// Change of layout: the amplitude at local index u moves from its place in
+// `from` to its place in `to`. In the kernels specialised to one sequence the
+// layouts are constants and every access is the lane's base plus an immediate.
+template <typename R>
+__device__ __forceinline__ void lay_put(R* lds, const R* x, uint64_t L) {
+  if constexpr (LdsSlots<R>::kAdd) {
+    R* base = lds + lay_lane_slot<R>(L);
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r) base[lay_reg_slot<R>(L, uint32_t(r))] = x[r];
+  } else {
+    const uint32_t s = lay_lane_slot<R>(L) * uint32_t(sizeof(R));
+    char* base = reinterpret_cast<char*>(lds);
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r)
+      *reinterpret_cast<R*>(base + slot_bytes(s, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R)))) = x[r];
+  }
+}
+
+template <typename R>
+__device__ __forceinline__ void lay_get(const R* lds, R* x, uint64_t L) {
+  if constexpr (LdsSlots<R>::kAdd) {
+    const R* base = lds + lay_lane_slot<R>(L);
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r) x[r] = base[lay_reg_slot<R>(L, uint32_t(r))];
+  } else {
+    const uint32_t s = lay_lane_slot<R>(L) * uint32_t(sizeof(R));
+    const char* base = reinterpret_cast<const char*>(lds);
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r)
+      x[r] = *reinterpret_cast<const R*>(base + slot_bytes(s, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R))));
+  }
+}
+
+template <typename R>
+__device__ __forceinline__ void lay_remap(R* lds, cplx<R>* v, uint64_t from, uint64_t to) {
+  if constexpr (LdsSlots<R>::kPair) {
+    cplx<R>* l = reinterpret_cast<cplx<R>*>(lds);  // 8-byte aligned (the buffer is 16-byte aligned)
+    lay_put(l, v, from);
+    __syncthreads();
+    lay_get(l, v, to);
+    __syncthreads();
+    return;
+  }
+  R x[kBReg];
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) x[r] = v[r].re;
+  lay_put(lds, x, from);
+  __syncthreads();
+  lay_get(lds, x, to);
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    v[r].re = x[r];
+    x[r] = v[r].im;
+  }
+  lay_put(lds, x, from);
+  __syncthreads();
+  lay_get(lds, x, to);
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) v[r].im = x[r];
+}
+
+// Before a renamed layout is stored: amplitudes change places within the tile
+// without passing through LDS, so every lane must have loaded its own before
+// any lane stores (the empty asm waits for the loads).
+template <typename R>
+__device__ __forceinline__ void relabel_fence(cplx<R>* v) {
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) asm volatile("" : "+v"(v[r].re), "+v"(v[r].im));
+  __syncthreads();
 }
 
 // Register r satisfies the register-bit conditions `rreq` (r is a constant
@@ -471,6 +663,120 @@ __device__ __forceinline__ void rot_regs(cplx<R>* v, uint32_t mode, R t, R s) {
   }
 }
 
+// A rotation divided by its cosine: with t = tan of the angle,
+//   mode 0: x0 - t x1, x1 + t x0   (RY)     mode 1: x0 + t x1, t x0 - x1   (H)
+//   mode 2: x0 - i t x1, x1 - i t x0   (RX)
+// -- two multiply-adds per real pair instead of the three of the shears, and
+// no chain between them. The cosine is a factor of the whole state: the host
+// multiplies the cosines of a run of rotations into the entries of one table
+// or 2x2 of the pass. Each result is rounded once, relative to itself, so
+// steep angles lose nothing; the host keeps the shears where the product of
+// the cosines would leave the range.
+template <bool NEG, bool REFL, typename R>
+__device__ __forceinline__ void rots_pair(R& x0, R& x1, R t) {
+  // NEG: the opposite angle; REFL: x1' = t x0 - x1 (and x0 + t x1)
+#if QSIM_LDS_ADDITIVE
+  // straight-line kernels: the compiler renames the registers
+  const R n0 = fmaR((NEG != REFL) ? t : -t, x1, x0);
+  x1 = REFL ? fmaR(t, x0, -x1) : fmaR(NEG ? -t : t, x0, x1);
+  x0 = n0;
+#else
+  // the interpreter updates in place (see real2_inplace)
+  R n;
+  if constexpr (sizeof(R) == 8) {
+    if constexpr (REFL)
+      asm("v_mov_b64 %[n], %[x0]\n\tv_fma_f64 %[x0], %[t], %[x1], %[x0]\n\tv_fma_f64 %[x1], %[t], %[n], -%[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+    else if constexpr (NEG)
+      asm("v_mov_b64 %[n], %[x0]\n\tv_fma_f64 %[x0], %[t], %[x1], %[x0]\n\tv_fma_f64 %[x1], -%[t], %[n], %[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+    else
+      asm("v_mov_b64 %[n], %[x0]\n\tv_fma_f64 %[x0], -%[t], %[x1], %[x0]\n\tv_fma_f64 %[x1], %[t], %[n], %[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+  } else {
+    if constexpr (REFL)
+      asm("v_mov_b32 %[n], %[x0]\n\tv_fma_f32 %[x0], %[t], %[x1], %[x0]\n\tv_fma_f32 %[x1], %[t], %[n], -%[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+    else if constexpr (NEG)
+      asm("v_mov_b32 %[n], %[x0]\n\tv_fma_f32 %[x0], %[t], %[x1], %[x0]\n\tv_fma_f32 %[x1], -%[t], %[n], %[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+    else
+      asm("v_mov_b32 %[n], %[x0]\n\tv_fma_f32 %[x0], -%[t], %[x1], %[x0]\n\tv_fma_f32 %[x1], %[t], %[n], %[x1]"
+          : [x0] "+v"(x0), [x1] "+v"(x1), [n] "=&v"(n) : [t] "s"(t));
+  }
+#endif
+}
+
+template <typename R, int J>
+__device__ __forceinline__ void rots_regs(cplx<R>* v, uint32_t mode, R t) {
+  if (mode == 0) {
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r) {
+      if ((r >> J) & 1) continue;
+      rots_pair<false, false>(v[r].re, v[r | (1 << J)].re, t);
+      rots_pair<false, false>(v[r].im, v[r | (1 << J)].im, t);
+    }
+  } else if (mode == 1) {
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r) {
+      if ((r >> J) & 1) continue;
+      rots_pair<false, true>(v[r].re, v[r | (1 << J)].re, t);
+      rots_pair<false, true>(v[r].im, v[r | (1 << J)].im, t);
+    }
+  } else {
+#pragma clang loop unroll(full)
+    for (int r = 0; r < kBReg; ++r) {
+      if ((r >> J) & 1) continue;
+      rots_pair<false, false>(v[r].im, v[r | (1 << J)].re, t);
+      rots_pair<true, false>(v[r].re, v[r | (1 << J)].im, t);
+    }
+  }
+}
+
+// The t of a ROTS record.
+template <typename R>
+__device__ __forceinline__ R rots_t(const Hdr& h) {
+  if constexpr (sizeof(R) == 8)
+    return __longlong_as_double(static_cast<long long>(h.cmask));
+  else
+    return __uint_as_float(uint32_t(h.cmask));
+}
+
+// DENSE2: a 4x4 on the register bits HI (the more significant index bit) and
+// LO. Kinds by the entries that are not zero, so that each form performs only
+// the products of its own: 0 complex, 1 real, 2 complex on the pairs (00, 11)
+// and (01, 10) alone, 3 the same with real entries.
+constexpr int kPairHi[6] = {1, 2, 3, 2, 3, 3};
+constexpr int kPairLo[6] = {0, 0, 0, 1, 1, 2};
+
+template <typename R, int HI, int LO, int KIND>
+__device__ __forceinline__ void dense2_regs(cplx<R>* v, const cplx<R>* m) {
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    if (((r >> HI) & 1) || ((r >> LO) & 1)) continue;
+    const int at[4] = {r, r | (1 << LO), r | (1 << HI), r | (1 << HI) | (1 << LO)};
+    const cplx<R> x[4] = {v[at[0]], v[at[1]], v[at[2]], v[at[3]]};
+#pragma clang loop unroll(full)
+    for (int i = 0; i < 4; ++i) {
+      cplx<R> y;
+      if constexpr (KIND == 0) {
+        y = cfma(m[4 * i + 3], x[3], cfma(m[4 * i + 2], x[2], cfma(m[4 * i + 1], x[1], cmul(m[4 * i], x[0]))));
+      } else if constexpr (KIND == 1) {
+        y.re = fmaR(m[4 * i + 3].re, x[3].re,
+                    fmaR(m[4 * i + 2].re, x[2].re, fmaR(m[4 * i + 1].re, x[1].re, m[4 * i].re * x[0].re)));
+        y.im = fmaR(m[4 * i + 3].re, x[3].im,
+                    fmaR(m[4 * i + 2].re, x[2].im, fmaR(m[4 * i + 1].re, x[1].im, m[4 * i].re * x[0].im)));
+      } else if constexpr (KIND == 2) {
+        y = cfma(m[4 * i + 3 - i], x[3 - i], cmul(m[4 * i + i], x[i]));
+      } else {
+        y.re = fmaR(m[4 * i + 3 - i].re, x[3 - i].re, m[4 * i + i].re * x[i].re);
+        y.im = fmaR(m[4 * i + 3 - i].re, x[3 - i].im, m[4 * i + i].re * x[i].im);
+      }
+      v[at[i]] = y;
+    }
+  }
+}
+
 // x *= d with d uniform: exactly cmul(d, x) (re = fma(d.re, x.re, -(d.im x.im)),
 // im = fma(d.re, x.im, d.im x.re)).
 __device__ __forceinline__ void cmul_inplace(cplx<double>& x, cplx<double> d) {
@@ -522,6 +828,20 @@ __device__ __forceinline__ cplx<R> csel(bool c, cplx<R> a, cplx<R> b) {
   r.re = c ? a.re : b.re;
   r.im = c ? a.im : b.im;
   return r;
+}
+
+// FLIP: X on register bit J where the conditions hold.
+template <typename R, int J>
+__device__ __forceinline__ void flip_regs(cplx<R>* v, const Hdr& h, uint64_t lane_idx) {
+  const bool on = (lane_idx & h.cmask) == h.cmask;
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    if ((r >> J) & 1) continue;
+    if (!reg_ok(r, h.rreq)) continue;
+    const cplx<R> a = v[r], b = v[r | (1 << J)];
+    v[r] = csel(on, b, a);
+    v[r | (1 << J)] = csel(on, a, b);
+  }
 }
 
 // Lane conditions are applied with selects, not branches: a divergent branch
@@ -639,13 +959,22 @@ __device__ __forceinline__ void flush_q_bit(cplx<R>* v, cplx<R> q) {
     if ((r >> J) & 1) v[r] = cmul(q, v[r]);
 }
 
+// Global-index bits of local index u.
+__device__ __forceinline__ uint64_t insert_local(uint32_t u, const BlkArgs& a) {
+  uint64_t g = 0;
+#pragma clang loop unroll(full)
+  for (int i = 0; i < kBTileBits; ++i)
+    if ((u >> i) & 1) g |= uint64_t(1) << a.tbits[i];
+  return g;
+}
+
 // Dense 2^k block (k = 1..3) on local bits. Each lane owns 16 / 2^k groups of
 // 2^k amplitudes (group g = lane + 256 i); the groups are gathered from the
 // tile through LDS one component at a time, multiplied in registers, and
-// scattered back the same way.
+// scattered back the same way (L: the layout in force).
 template <typename R, int K>
-__device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr& in, const cplx<R>* m,
-                                          uint64_t tile_base, const uint64_t* gbit) {
+__device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, uint64_t L, const Hdr& in, const cplx<R>* m,
+                                          uint64_t tile_base, const BlkArgs& args) {
   constexpr int D = 1 << K;
   constexpr int NG = (kBTile >> K) / kBT;  // groups per lane
   uint32_t srt[K];
@@ -673,23 +1002,19 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr
       b = low | ((b ^ low) << 1);
     }
     base[i] = b;
-    act[i] = ((tile_base | deposit(b, gbit)) & in.cmask) == in.cmask;
+    act[i] = ((tile_base | insert_local(b, args)) & in.cmask) == in.cmask;
   }
-  using L = LdsSlots<R>;
-  uint32_t slot[kBReg];  // the lane's amplitudes in the current mapping
-  const uint32_t s0 = L::of(lane_local(map, threadIdx.x));
+  using S = LdsSlots<R>;
+  uint32_t slot[kBReg];  // the lane's amplitudes in the current layout
+  const uint32_t s0 = lay_lane_slot<R>(L);
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) {  // per-register constants, selected by the uniform mapping
-    const uint32_t rs =
-        map == 0 ? L::of(uint32_t(r) << 8) : (map == 1 ? L::of(uint32_t(r) << 4) : L::of(uint32_t(r)));
-    slot[r] = L::join(s0, rs);
-  }
+  for (int r = 0; r < kBReg; ++r) slot[r] = S::join(s0, lay_reg_slot<R>(L, uint32_t(r)));
   // group i's input c sits at base[i] | off[c] (disjoint bits)
   uint32_t bslot[NG], oslot[D];
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i) bslot[i] = L::of(base[i]);
+  for (int i = 0; i < NG; ++i) bslot[i] = lay_slot<R>(base[i]);
 #pragma clang loop unroll(full)
-  for (int c = 0; c < D; ++c) oslot[c] = L::of(off[c]);
+  for (int c = 0; c < D; ++c) oslot[c] = lay_slot<R>(off[c]);
   cplx<R> g[kBReg];  // g[i * D + c]: input c of group i
   // gather: real parts, then imaginary parts
 #pragma clang loop unroll(full)
@@ -698,7 +1023,7 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr
 #pragma clang loop unroll(full)
   for (int i = 0; i < NG; ++i)
 #pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) g[i * D + c].re = lds[L::join(bslot[i], oslot[c])];
+    for (int c = 0; c < D; ++c) g[i * D + c].re = lds[S::join(bslot[i], oslot[c])];
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) lds[slot[r]] = v[r].im;
@@ -706,7 +1031,7 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr
 #pragma clang loop unroll(full)
   for (int i = 0; i < NG; ++i)
 #pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) g[i * D + c].im = lds[L::join(bslot[i], oslot[c])];
+    for (int c = 0; c < D; ++c) g[i * D + c].im = lds[S::join(bslot[i], oslot[c])];
   __syncthreads();
   // multiply (the arithmetic of the one-gate kernels: cmul, then cfma in column order)
 #pragma clang loop unroll(full)
@@ -727,7 +1052,7 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr
 #pragma clang loop unroll(full)
   for (int i = 0; i < NG; ++i)
 #pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) lds[L::join(bslot[i], oslot[c])] = g[i * D + c].re;
+    for (int c = 0; c < D; ++c) lds[S::join(bslot[i], oslot[c])] = g[i * D + c].re;
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) v[r].re = lds[slot[r]];
@@ -735,7 +1060,7 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, int map, const Hdr
 #pragma clang loop unroll(full)
   for (int i = 0; i < NG; ++i)
 #pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) lds[L::join(bslot[i], oslot[c])] = g[i * D + c].im;
+    for (int c = 0; c < D; ++c) lds[S::join(bslot[i], oslot[c])] = g[i * D + c].im;
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) v[r].im = lds[slot[r]];

@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
 
+#include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -44,6 +45,7 @@ struct RecView {
   bool cond;      // nonzero tile condition: the record runs only where it holds
   uint32_t nent;  // entries (at most kMaxEntries): fixes the next record's offset
   uint32_t off;
+  uint64_t to, from;  // MAP with a layout: the header's layouts
 };
 
 // What a specialised kernel does: a pass (k_blocked), a pass whose input is
@@ -59,7 +61,12 @@ bool decode(const uint8_t* prog, size_t nbytes, int ninstr, int dtype, std::vect
     BlkHdr h;
     std::memcpy(&h, prog + off, sizeof(BlkHdr));
     const uint32_t nent = h.nent < kMaxEntries ? h.nent : kMaxEntries;
-    out.push_back({h.op, h.arg, h.tmask != 0, nent, off});
+    RecView r{h.op, h.arg, h.tmask != 0, nent, off, 0, 0};
+    if (h.op == kOpMap && h.arg >= kMapLayout && h.arg <= kMapRelabel) {
+      r.to = h.cmask;
+      if (h.arg == kMapLayout) std::memcpy(&r.from, h.bits, 8);
+    }
+    out.push_back(r);
     if (h.op == kOpMap && h.tmask != 0) {
       // the mapping after a conditional MAP depends on the tile: not static
       why = "conditional mapping change";
@@ -81,10 +88,10 @@ uint64_t spec_cost_ms(const std::vector<RecView>& recs) {
   uint64_t c = 0;
   for (const RecView& r : recs) {
     switch (r.op) {
-      case kOpRot: case kOpRegPhase: case kOpNeg: c += 15; break;
+      case kOpRot: case kOpRotS: case kOpRegPhase: case kOpNeg: case kOpFlip: c += 15; break;
       case kOpLanePhase: case kOpLaneRegPhase: case kOpQFlush: c += 30; break;
       case kOpMap: case kOpDense1: case kOpDense1Real: c += 100; break;
-      case kOpDiag: c += 120; break;
+      case kOpDiag: case kOpDense2: c += 120; break;
       case kOpDenseLds: c += 300; break;
       case kOpInner1: case kOpInnerDiag: c += 450; break;
       default: break;
@@ -103,13 +110,30 @@ std::string structure_key(const std::vector<RecView>& recs, int dtype, int varia
     key.push_back(char(r.arg));
     key.push_back(char(r.cond ? 1 : 0));
     key.push_back(char(r.nent));  // <= 64
+    if (r.op == kOpMap && r.arg >= kMapLayout && r.arg <= kMapRelabel)  // the layouts are constants of the kernel
+      for (int i = 0; i < 6; ++i) {
+        key.push_back(char((r.to >> (8 * i)) & 255));
+        key.push_back(char((r.from >> (8 * i)) & 255));
+      }
   }
   return key;
 }
 
+std::string hex(uint64_t v) {
+  char buf[32];
+  std::snprintf(buf, sizeof(buf), "0x%llxull", static_cast<unsigned long long>(v));
+  return buf;
+}
+
+bool low_in_regs(uint64_t layout) {  // lay_low_in_regs on the host
+  for (int p = 8; p < 12; ++p)
+    if (((layout >> (4 * p)) & 15u) < 3) return true;
+  return false;
+}
+
 // One record's code: the body of k_blocked's switch for this opcode with the
-// argument fixed; `map` is the mapping in force (every MAP is unconditional).
-void emit_record(std::string& s, const RecView& r, bool dbl, int& map) {
+// argument fixed; `layout` is the layout in force (every MAP is unconditional).
+void emit_record(std::string& s, const RecView& r, bool dbl, uint64_t& layout) {
   const std::string off = std::to_string(r.off);
   s += "  {\n    const Hdr h = load_hdr(prog + " + off + "u);\n";
   s += "    const cplx<R>* m = reinterpret_cast<const cplx<R>*>(prog + " + std::to_string(r.off + 32) + "u);\n";
@@ -119,13 +143,23 @@ void emit_record(std::string& s, const RecView& r, bool dbl, int& map) {
   const std::string J = std::to_string(r.arg & 3);
   switch (r.op) {
     case kOpLaneRegPhase:
-      s += "      const cplx<R> q = q_lds[threadIdx.x];\n"
-           "      q_lds[threadIdx.x] = csel(lane_ok(), cmul(me[0], q), q);\n";
+      s += "      Q = csel(lane_ok(), cmul(me[0], Q), Q);\n";
       break;
     case kOpQFlush:
-      s += "      const cplx<R> q = q_lds[threadIdx.x];\n"
-           "      q_lds[threadIdx.x] = cplx<R>{R(1), R(0)};\n"
-           "      flush_q_bit<R, " + J + ">(v, q);\n";
+      s += "      flush_q_bit<R, " + J + ">(v, Q);\n"
+           "      Q = cplx<R>{R(1), R(0)};\n";
+      break;
+    case kOpRotS:
+      s += "      rots_regs<R, " + J + ">(v, " + std::to_string(r.arg >> 2) + "u, rots_t<R>(h));\n";
+      break;
+    case kOpDense2: {
+      const int pair = int(r.arg & 7u) < 5 ? int(r.arg & 7u) : 5, kind = int(r.arg >> 3) < 3 ? int(r.arg >> 3) : 3;
+      s += "      dense2_regs<R, " + std::to_string(kPairHi[pair]) + ", " + std::to_string(kPairLo[pair]) + ", " +
+           std::to_string(kind) + ">(v, m);\n";
+      break;
+    }
+    case kOpFlip:
+      s += "      flip_regs<R, " + J + ">(v, h, lane_idx);\n";
       break;
     case kOpDense1Real:
       s += "      dense1_regs<R, " + J + ", true>(v, h, me, lane_idx);\n";
@@ -169,19 +203,24 @@ void emit_record(std::string& s, const RecView& r, bool dbl, int& map) {
     case kOpDiag:
       s += "      diag_regs(v, h, m, lane_idx, lane_ok());\n";
       break;
-    case kOpMap: {
-      const int nmap = r.arg < 3 ? int(r.arg) : 0;
-      s += "      flush_lane_phase(v, P, pdirty);\n";
-      s += "      remap(lds, v, " + std::to_string(map) + ", " + std::to_string(nmap) + ");\n";
-      s += "      lane_idx = tile_base | deposit(local_index(" + std::to_string(nmap) + ", threadIdx.x, 0), gbit);\n";
-      map = nmap;
+    case kOpMap:
+      if (r.arg == kMapStart) break;  // applied before the load
+      if (r.arg == kMapRelabel) {
+        s += "      relabel_fence(v);\n";
+        layout = r.to;
+      } else {
+        const bool given = r.arg == kMapLayout;
+        const uint64_t from = given ? r.from : layout;
+        layout = given ? r.to : (r.arg == 1 ? kLayout1 : (r.arg == 2 ? kLayout2 : kLayout0));
+        s += "      flush_lane_phase(v, P, pdirty);\n";
+        s += "      lay_remap(lds, v, " + hex(from) + ", " + hex(layout) + ");\n";
+      }
+      s += "      lane_idx = tile_base | lay_lane_index(a, " + hex(layout) + ");\n";
       break;
-    }
     case kOpDenseLds: {
       const int kk = r.arg <= 1 ? 1 : (r.arg == 2 ? 2 : 3);
       s += "      flush_lane_phase(v, P, pdirty);\n";
-      s += "      dense_lds<R, " + std::to_string(kk) + ">(lds, v, " + std::to_string(map) +
-           ", h, m, tile_base, gbit);\n";
+      s += "      dense_lds<R, " + std::to_string(kk) + ">(lds, v, " + hex(layout) + ", h, m, tile_base, a);\n";
       break;
     }
     default:  // NOP and the adjoint-only forms: no effect, as in k_blocked
@@ -336,51 +375,44 @@ std::string make_source(const std::vector<RecView>& recs, int dtype, int variant
   if (tile >= a.ntiles) return;
   psi += blockIdx.z * a.state_stride;
   prog += blockIdx.z * a.prog_stride;
-  uint64_t gbit[kBTileBits];
-#pragma clang loop unroll(full)
-  for (int i = 0; i < kBTileBits; ++i) gbit[i] = uint64_t(1) << a.tbits[i];
   const uint64_t tile_base = tile_origin(a, tile);
-  uint64_t lane_idx = tile_base | deposit(local_index(0, threadIdx.x, 0), gbit);
-  cplx<R> v[kBReg];
 )";
+  uint64_t layout = kLayout0;
+  if (!recs.empty() && recs[0].op == kOpMap && recs[0].arg == kMapStart) layout = recs[0].to;
+  s += "  uint64_t lane_idx = tile_base | lay_lane_index(a, " + hex(layout) + ");\n";
+  s += "  cplx<R> v[kBReg];\n  {\n    uint64_t rb[4];\n    lay_reg_bits(a, " + hex(layout) + ", rb);\n";
   if (from_zero)
     s += R"(#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) {
-    v[r].re = (lane_idx | deposit(uint32_t(r) << 8, gbit)) == 0 ? R(1) : R(0);
-    v[r].im = R(0);
-  }
+    for (int r = 0; r < kBReg; ++r) {
+      v[r].re = (lane_idx | reg_index(rb, r)) == 0 ? R(1) : R(0);
+      v[r].im = R(0);
+    }
 )";
   else
-    s += "  load_lane(a, psi, lane_idx, gbit, v);\n";
-  s += R"(  cplx<R> P;
+    s += "    load_lane(a, psi, lane_idx, " + hex(layout) + ", rb, v);\n";
+  s += R"(  }
+  cplx<R> P;
   P.re = R(1);
   P.im = R(0);
   bool pdirty = false;
-)";
-  // the per-lane factor of LANE_REGPHASE records lives in LDS; a sequence
-  // without them leaves it out, so the kernel needs only the transpose buffer
-  // (32 KiB in complex128: five workgroups per CU instead of four)
-  bool qfactor = false;
-  for (const RecView& r : recs) qfactor |= r.op == kOpLaneRegPhase || r.op == kOpQFlush;
-  if (qfactor)
-    s += R"(  __shared__ cplx<R> q_lds[kBT];
-  q_lds[threadIdx.x] = cplx<R>{R(1), R(0)};
-)";
-  s += R"(  const uint64_t tb_lo = __builtin_amdgcn_readfirstlane(uint32_t(tile_base));
+  cplx<R> Q = P;  // the per-lane factor of LANE_REGPHASE records
+  (void)Q;
+  const uint64_t tb_lo = __builtin_amdgcn_readfirstlane(uint32_t(tile_base));
   const uint64_t tb_hi = __builtin_amdgcn_readfirstlane(uint32_t(tile_base >> 32));
   const uint64_t tile_base_s = tb_lo | (tb_hi << 32);
   (void)tile_base_s;
 )";
-  int map = 0;
-  for (const RecView& r : recs) emit_record(s, r, dbl, map);
+  for (const RecView& r : recs) emit_record(s, r, dbl, layout);
   s += "  flush_lane_phase(v, P, pdirty);\n";
-  if (map != 0) {
-    s += "  remap(lds, v, " + std::to_string(map) + ", 0);\n";
-    s += "  lane_idx = tile_base | deposit(local_index(0, threadIdx.x, 0), gbit);\n";
+  if (low_in_regs(layout)) {
+    s += "  lay_remap(lds, v, " + hex(layout) + ", kLayout0);\n";
+    layout = kLayout0;
   }
+  s += "  lane_idx = tile_base | lay_lane_index(a, " + hex(layout) + ");\n";
+  s += "  uint64_t rb[4];\n  lay_reg_bits(a, " + hex(layout) + ", rb);\n";
   s += R"(  asm volatile("" : "+v"(lane_idx));
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) st_nt(psi, lane_idx | deposit(uint32_t(r) << 8, gbit), v[r]);
+  for (int r = 0; r < kBReg; ++r) st_nt(psi, lane_idx | reg_index(rb, r), v[r]);
 }
 }  // namespace qsim
 )";

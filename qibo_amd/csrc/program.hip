@@ -1,0 +1,829 @@
+// Host-side compiler of one blocked pass into the form the backend runs
+// (qsim_compile_program). qsim_compile_pass (compile.hip) keeps the local bits
+// in three fixed mappings and is restated record for record in Python; this
+// compiler starts from the same planned gates and dependency rules and goes
+// further where that is cheaper on the device:
+//
+//  * any four of the pass's local bits may be register bits (MAP records with
+//    layouts): a change of layout picks the bits that let the most waiting
+//    gates run, two-qubit gates included, which then run in registers
+//    (DENSE2: at most 0.25 CU-cycles per amplitude) instead of through an LDS
+//    gather (DENSE_LDS: 0.75);
+//  * a SWAP, and the SWAP part of a gate like iSWAP, only renames two local
+//    bits: no data moves until the next change of layout;
+//  * rotations are divided by their cosines (ROTS: two multiply-adds per real
+//    pair instead of three), the cosines multiplied into the entries of one
+//    unconditional record of the run;
+//  * a diagonal gate between one register bit and lane bits is split into a
+//    table, a per-lane phase and a controlled phase (0.30 CU-cycles as DIAG);
+//  * phases whose conditions lie outside the tile are skipped by whole
+//    workgroups;
+//  * conditional X gates exchange registers instead of multiplying.
+
+#include <algorithm>
+#include <array>
+#include <deque>
+
+#include "compile_ops.h"
+
+namespace {
+
+constexpr uint8_t kRRotS = 13, kRDense2 = 14, kRFlip = 15;
+constexpr int kMapLayout = 3, kMapStart = 4, kMapRelabel = 5;
+
+// Local bits of one kind share the low bits of their LDS slot (blocked_dev.h:
+// swl, kSlotW): the first five lane positions take bits of five kinds.
+constexpr int kBankKind[kTileBits] = {0, 1, 2, 3, 4, 0, 1, 2, 4, 3, 0, 1};
+
+struct Item {
+  Op op;
+  uint32_t need = 0;   // local bits that must be register bits
+  bool lds = false;    // runs through LDS in any layout (last choice)
+  bool relabel = false;
+  int weight = 0;      // gates it counts for when a layout is chosen
+};
+
+struct Layout {
+  uint8_t at[kTileBits];  // local bit at each position (0-7 lane, 8-11 register)
+
+  uint32_t regs() const {
+    uint32_t m = 0;
+    for (int p = 8; p < kTileBits; ++p) m |= 1u << at[p];
+    return m;
+  }
+  uint64_t word() const {
+    uint64_t w = 0;
+    for (int p = 0; p < kTileBits; ++p) w |= uint64_t(at[p]) << (4 * p);
+    return w;
+  }
+  int reg_of(int lb) const {
+    for (int p = 8; p < kTileBits; ++p)
+      if (at[p] == lb) return p - 8;
+    return -1;
+  }
+};
+
+// The layout with the register bits R: the pass's lowest bits at the lowest
+// lane positions (whole lines per access of a lane group), then bits of the
+// kinds the first five positions still lack, then the rest ascending.
+Layout make_layout(uint32_t R, int low) {
+  Layout l;
+  int p = 0;
+  uint32_t left = ((1u << kTileBits) - 1) & ~R, kinds = 0;
+  auto take = [&](int b) {
+    l.at[p++] = uint8_t(b);
+    left &= ~(1u << b);
+    kinds |= 1u << kBankKind[b];
+  };
+  for (int b = 0; b < low; ++b)
+    if ((left >> b) & 1) take(b);
+  while (p < 5) {
+    int pick = -1;
+    for (int b = 0; b < kTileBits && pick < 0; ++b)
+      if (((left >> b) & 1) && !((kinds >> kBankKind[b]) & 1)) pick = b;
+    if (pick < 0) pick = __builtin_ctz(left);  // a kind held by the registers alone: two lanes share a bank
+    take(pick);
+  }
+  while (left) take(__builtin_ctz(left));
+  for (int b = 0; b < kTileBits; ++b)
+    if ((R >> b) & 1) l.at[p++] = uint8_t(b);
+  return l;
+}
+
+class Compiler {
+ public:
+  Compiler(int n, const int* tile_bits, int low, Writer& w) : n_(n), tb_(tile_bits), low_(low), w_(w) {
+    for (int b = 0; b < 64; ++b) local_[b] = -1;
+    for (int i = 0; i < kTileBits; ++i) local_[tile_bits[i]] = i;
+    lowmask_ = (1u << low) - 1;
+  }
+
+  int run(std::vector<Op>& ops, int* switches);
+
+ private:
+  int n_;
+  const int* tb_;
+  int low_;
+  uint32_t lowmask_;
+  Writer& w_;
+  int local_[64];
+  std::vector<Item> items_;
+  std::deque<std::array<C, 16>> made_;  // entries of gates rewritten here
+  std::vector<std::vector<int>> succ_;
+  std::vector<int> npred_, ready_;
+
+  Layout lay_;
+  bool stale_ = false;  // lane positions were renamed since the kernel formed the lane's index
+  bool relabelled_unseen_ = false;  // any position was renamed since the kernel last saw a layout
+  bool have_pending_ = false;
+  C pending_[16];
+  long reg_first_off_ = -1;
+  size_t reg_first_ev_ = 0;
+  C gfac_ = {1.0, 0.0};
+  bool sign_ = false;
+  int qpend_ = -1;
+  int switches_ = 0;
+
+  // rotations and the records that can take their cosines, in order
+  struct Event {
+    int kind;  // 0 rotation, 1 takes factors, 2 a table of some registers
+    long off;  // rotation: header; others: first entry
+    double t = 0, s = 0, tan = 0, c = 0;
+    int dep = 0;
+    std::vector<C> entries;
+  };
+  std::vector<Event> events_;
+
+  void note(uint8_t op, int arg, uint64_t cmask, uint64_t tmask, int rreq, const C* data, int ndata);
+  void emit(uint8_t op, int arg, uint64_t cmask, int nt, const int* bits, int nbits, const C* data, int ndata,
+            int rreq = 0, uint64_t tmask = 0, bool lane_index = false);
+  void build_items(std::vector<Op>& ops);
+  void dependencies();
+  uint32_t choose_regs(bool first);
+  void change_layout(uint32_t R);
+  void flush_reg(int j);
+  void qflush(int j);
+  void emit_diag(const Op& o);
+  void emit_phase(const int* tbits, int nt, const int* cbits, int nc, const C* d);
+  void emit_dense1(const Op& o, int j);
+  void emit_dense2(const Op& o);
+  void emit_lds(const Op& o);
+  void fold_cosines();
+  int gbit(int lb) const { return tb_[lb]; }
+  uint64_t outside(uint64_t m) const {
+    uint64_t o = 0;
+    for (int b = 0; b < 64; ++b)
+      if (((m >> b) & 1) && local_[b] < 0) o |= uint64_t(1) << b;
+    return o;
+  }
+};
+
+// Remembers a record that multiplies the whole state, or a table of some
+// registers, as a place for the cosines.
+void Compiler::note(uint8_t op, int arg, uint64_t cmask, uint64_t tmask, int rreq, const C* data, int ndata) {
+  if (cmask || tmask || rreq || !data) return;
+  Event e;
+  e.off = long(w_.len) + kHeader;
+  e.entries.assign(data, data + ndata);
+  if (op == kRRegPhase && arg != 0) {
+    e.kind = 2;
+    e.dep = arg;
+  } else if (op == kRDense1 || op == kRDense1Real || op == kRRegPhase || op == kRLanePhase || op == kRDiag ||
+             op == kRDense2) {
+    e.kind = 1;
+  } else {
+    return;
+  }
+  events_.push_back(std::move(e));
+}
+
+void Compiler::emit(uint8_t op, int arg, uint64_t cmask, int nt, const int* bits, int nbits, const C* data, int ndata,
+                    int rreq, uint64_t tmask, bool lane_index) {
+  if (stale_ && (cmask != 0 || lane_index)) {
+    stale_ = relabelled_unseen_ = false;
+    w_.emit(kRMap, kMapRelabel, lay_.word(), 0, nullptr, 0, nullptr, 0);
+  }
+  note(op, arg, cmask, tmask, rreq, data, ndata);
+  const size_t at = w_.len;
+  w_.emit(op, arg, cmask, nt, bits, nbits, data, ndata, rreq);
+  if (!w_.overflow && tmask) std::memcpy(w_.out + at + 24, &tmask, 8);
+}
+
+void Compiler::build_items(std::vector<Op>& ops) {
+  for (Op& o : ops) {
+    Item it;
+    if (o.kind == kDense && o.nt == 2 && o.nc == 0) {
+      // one entry per row in the pattern of a SWAP: a SWAP, then a diagonal
+      const C* m = o.data;
+      auto zero = [&](int i) { return m[i].re == 0 && m[i].im == 0; };
+      bool swap = true;
+      for (int i = 0; i < 16; ++i) swap = swap && (zero(i) != (i == 0 || i == 6 || i == 9 || i == 15));
+      if (swap) {
+        Op d = o;
+        made_.emplace_back();
+        made_.back()[0] = m[0], made_.back()[1] = m[6], made_.back()[2] = m[9], made_.back()[3] = m[15];
+        d.kind = kDiag;
+        d.data = made_.back().data();
+        d.ndata = 4;
+        d.nd_mask = 0;
+        o.kind = kSwap;
+        o.data = nullptr;
+        o.ndata = 0;
+        it.op = o;
+        it.relabel = true;
+        items_.push_back(it);
+        bool one = true;
+        for (int i = 0; i < 4; ++i) one = one && d.data[i].re == 1 && d.data[i].im == 0;
+        if (!one) {
+          Item id;
+          id.op = d;
+          items_.push_back(id);
+        }
+        continue;
+      }
+    }
+    it.op = o;
+    if (o.kind == kSwap) {
+      it.relabel = o.nc == 0;
+      it.lds = o.nc != 0;
+    } else if (o.kind == kDense) {
+      if (o.nt == 1 || (o.nt == 2 && o.nc == 0)) {
+        for (int k = 0; k < o.nt; ++k) it.need |= 1u << local_[n_ - 1 - o.t[k]];
+        it.weight = o.nt == 1 ? 1 : 3;
+      } else {
+        it.lds = true;
+      }
+    }
+    items_.push_back(it);
+  }
+}
+
+// As qsim_compile_pass: per amplitude bit, a non-diagonal user follows the
+// last non-diagonal user and every diagonal user since, a diagonal user the
+// last non-diagonal one.
+void Compiler::dependencies() {
+  const int N = int(items_.size());
+  succ_.assign(size_t(N), {});
+  npred_.assign(size_t(N), 0);
+  int last_nd[64];
+  for (int b = 0; b < 64; ++b) last_nd[b] = -1;
+  std::vector<int> since[64];
+  std::vector<int> preds;
+  for (int j = 0; j < N; ++j) {
+    const Op& o = items_[size_t(j)].op;
+    preds.clear();
+    for (uint64_t m = o.all_mask; m; m &= m - 1) {
+      const int b = __builtin_ctzll(m);
+      const bool nd = (o.nd_mask >> b) & 1;
+      if (nd) preds.insert(preds.end(), since[b].begin(), since[b].end());
+      if (last_nd[b] >= 0) preds.push_back(last_nd[b]);
+      if (nd) {
+        last_nd[b] = j;
+        since[b].clear();
+      } else {
+        since[b].push_back(j);
+      }
+    }
+    std::sort(preds.begin(), preds.end());
+    preds.erase(std::unique(preds.begin(), preds.end()), preds.end());
+    for (int i : preds) succ_[size_t(i)].push_back(j);
+    npred_[size_t(j)] = int(preds.size());
+  }
+  for (int i = 0; i < N; ++i)
+    if (npred_[size_t(i)] == 0) ready_.push_back(i);
+}
+
+// The register bits of the next layout: grown greedily by the bits of a
+// waiting gate that let the most gates run per bit added (every gate that
+// then becomes ready and runs counts, renames included).
+uint32_t Compiler::choose_regs(bool first) {
+  struct Sim {
+    std::vector<int> left, blocked;
+    uint32_t R = 0;
+    int done = 0;
+  };
+  auto extend = [&](Sim& s, uint32_t add) {
+    s.R |= add;
+    std::vector<int> work;
+    bool again = true;
+    while (again) {
+      again = false;
+      size_t keep = 0;
+      for (size_t i = 0; i < s.blocked.size(); ++i) {
+        const int g = s.blocked[i];
+        const Item& it = items_[size_t(g)];
+        if (!it.lds && !(it.need & ~s.R))
+          work.push_back(g);
+        else
+          s.blocked[keep++] = g;
+      }
+      s.blocked.resize(keep);
+      while (!work.empty()) {
+        const int g = work.back();
+        work.pop_back();
+        const Item& it = items_[size_t(g)];
+        s.done += it.weight;
+        if (it.relabel) {
+          const uint32_t a = 1u << local_[n_ - 1 - it.op.t[0]], b = 1u << local_[n_ - 1 - it.op.t[1]];
+          const bool ra = s.R & a, rb = s.R & b;
+          if (ra != rb) {
+            s.R ^= a | b;
+            again = true;
+          }
+        }
+        for (int j : succ_[size_t(g)])
+          if (--s.left[size_t(j)] == 0) {
+            const Item& nx = items_[size_t(j)];
+            if (!nx.lds && !(nx.need & ~s.R))
+              work.push_back(j);
+            else
+              s.blocked.push_back(j);
+          }
+      }
+    }
+  };
+  Sim cur;
+  cur.left = npred_;
+  cur.blocked = ready_;
+  uint32_t chosen = 0;
+  extend(cur, 0);
+  const uint32_t banned = first ? lowmask_ : 0;
+  while (__builtin_popcount(chosen) < 4) {
+    uint32_t cands[96];
+    int nc = 0;
+    auto add_cand = [&](uint32_t m) {
+      m &= ~chosen;
+      if (!m || (m & banned) || __builtin_popcount(chosen | m) > 4 || nc == 96) return;
+      for (int i = 0; i < nc; ++i)
+        if (cands[i] == m) return;
+      cands[nc++] = m;
+    };
+    for (int g : cur.blocked)
+      if (!items_[size_t(g)].lds) add_cand(items_[size_t(g)].need & ~cur.R);
+    uint32_t best = 0;
+    double best_score = 0;
+    Sim best_sim;
+    for (int i = 0; i < nc; ++i) {
+      Sim s = cur;
+      extend(s, cands[i]);
+      const double score = double(s.done - cur.done) / __builtin_popcount(cands[i]);
+      if (score > best_score) {
+        best_score = score;
+        best = cands[i];
+        best_sim = std::move(s);
+      }
+    }
+    if (!best) break;
+    chosen |= best;
+    cur = std::move(best_sim);
+  }
+  // the rest: bits that leave every kind of bank to the lanes, highest first
+  for (int pass = 0; pass < 2; ++pass)
+    for (int b = kTileBits - 1; b >= 0 && __builtin_popcount(chosen) < 4; --b) {
+      if (((chosen >> b) & 1) || ((lowmask_ >> b) & 1)) continue;
+      if (pass == 0) {
+        uint32_t kinds = 0;
+        for (int c = 0; c < kTileBits; ++c)
+          if (!((chosen >> c) & 1) && c != b) kinds |= 1u << kBankKind[c];
+        if (kinds != 31u) continue;
+      }
+      chosen |= 1u << b;
+    }
+  return chosen;
+}
+
+void Compiler::change_layout(uint32_t R) {
+  flush_reg(-1);
+  qflush(-1);
+  const Layout to = make_layout(R, low_);
+  const uint64_t from = lay_.word();
+  int bytes[8];
+  for (int i = 0; i < 8; ++i) bytes[i] = int((from >> (8 * i)) & 255);
+  w_.emit(kRMap, kMapLayout, to.word(), 0, bytes, 8, nullptr, 0);
+  lay_ = to;
+  stale_ = relabelled_unseen_ = false;
+  ++switches_;
+}
+
+void Compiler::qflush(int j) {
+  if (qpend_ < 0 || (j >= 0 && j != qpend_)) return;
+  emit(kRQFlush, qpend_, 0, 0, nullptr, 0, nullptr, 0);
+  qpend_ = -1;
+}
+
+// The pending table, before a gate on register j that does not commute with
+// it (j = -1: whatever it holds). After the first table the value at
+// register 0 goes to the first one, and the record multiplies only the
+// registers whose bits it depends on.
+void Compiler::flush_reg(int j) {
+  if (!have_pending_) return;
+  auto depends_on = [&](int k) {
+    for (int r = 0; r < 16; ++r)
+      if (!ceq(pending_[r], pending_[r ^ (1 << k)])) return true;
+    return false;
+  };
+  if (j >= 0 && !depends_on(j)) return;
+  have_pending_ = false;
+  const C t0 = pending_[0];
+  const double mag = t0.re * t0.re + t0.im * t0.im;
+  if (reg_first_off_ < 0 || std::fabs(mag - 1.0) > 1e-12) {
+    if (reg_first_off_ < 0) {
+      reg_first_off_ = long(w_.len) + kHeader;
+      reg_first_ev_ = events_.size();
+    }
+    emit(kRRegPhase, 0, 0, 0, nullptr, 0, pending_, 16);
+    return;
+  }
+  int dep = 0;
+  for (int k = 0; k < 4; ++k)
+    if (depends_on(k)) dep |= 1 << k;
+  gfac_ = cmulf(gfac_, t0);
+  if (!dep) return;
+  const C inv = {t0.re / mag, -t0.im / mag};
+  C table[16];
+  for (int r = 0; r < 16; ++r) table[r] = (r & dep) ? cmulf(pending_[r], inv) : C{1.0, 0.0};
+  emit(kRRegPhase, dep, 0, 0, nullptr, 0, table, 16);
+}
+
+// A diagonal on the global bits tbits (first = most significant index bit)
+// under the bits cbits.
+void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, const C* d) {
+  auto reg = [&](int b) { return local_[b] >= 0 ? lay_.reg_of(local_[b]) : -1; };
+  int nreg_t = 0, nreg_c = 0, jt = -1;
+  for (int k = 0; k < nt; ++k)
+    if (reg(tbits[k]) >= 0) ++nreg_t, jt = k;
+  for (int k = 0; k < nc; ++k) nreg_c += reg(cbits[k]) >= 0;
+  uint64_t cm = 0;
+  int rreq = 0;
+  for (int k = 0; k < nc; ++k) {
+    if (reg(cbits[k]) >= 0)
+      rreq |= 1 << reg(cbits[k]);
+    else
+      cm |= uint64_t(1) << cbits[k];
+  }
+  if (nreg_t == 0 && nreg_c == 0) {
+    const uint64_t tm = outside(cm);
+    emit(kRLanePhase, 0, cm & ~tm, nt, tbits, nt, d, 1 << nt, 0, tm, true);
+    return;
+  }
+  if (nreg_t == nt && nreg_c == nc) {
+    if (!have_pending_) {
+      for (int r = 0; r < 16; ++r) pending_[r] = {1.0, 0.0};
+      have_pending_ = true;
+    }
+    for (int r = 0; r < 16; ++r) {
+      if ((r & rreq) != rreq) continue;
+      int di = 0;
+      for (int k = 0; k < nt; ++k) di = (di << 1) | ((r >> reg(tbits[k])) & 1);
+      pending_[r] = cmulf(pending_[r], d[di]);
+    }
+    return;
+  }
+  if (nt == 0) {
+    if (d[0].re == -1.0 && d[0].im == 0.0) {
+      emit(kRNeg, 0, cm, 0, nullptr, 0, nullptr, 0, rreq);
+      return;
+    }
+    if ((rreq & (rreq - 1)) == 0) {  // one register bit: the lane's factor of its upper half
+      const int j = __builtin_ctz(unsigned(rreq));
+      if (qpend_ != j) {
+        qflush(-1);
+        qpend_ = j;
+      }
+      const uint64_t tm = outside(cm);
+      emit(kRLaneRegPhase, j, cm & ~tm, 0, nullptr, 0, d, 1, 0, tm);
+      return;
+    }
+  }
+  // one register bit and lane bits: f(0, lanes) f(1, lanes) / f(0, lanes)
+  auto unit = [](C x) { return std::fabs(x.re * x.re + x.im * x.im - 1.0) <= 1e-6; };
+  auto over = [](C x, C y) {  // x / y
+    const double m = y.re * y.re + y.im * y.im;
+    return cmulf(x, C{y.re / m, -y.im / m});
+  };
+  bool units = true;
+  for (int i = 0; i < (1 << nt); ++i) units = units && unit(d[i]);
+  if (units && nreg_t + nreg_c == 1) {
+    auto phase = [&](std::vector<int> c, C x) {  // x where every bit of c is 1
+      if (!(x.re == 1.0 && x.im == 0.0)) emit_phase(nullptr, 0, c.data(), int(c.size()), &x);
+    };
+    std::vector<int> cb(cbits, cbits + nc);
+    if (nt == 1 && nreg_t == 1) {  // diag(a, b) on the register bit under lane bits
+      phase(cb, d[0]);
+      cb.push_back(tbits[0]);
+      phase(cb, over(d[1], d[0]));
+      return;
+    }
+    if (nt == 1 && nreg_c == 1) {  // diag(a, b) on a lane bit, the register bit among the conditions
+      phase(cb, d[0]);
+      cb.push_back(tbits[0]);
+      phase(cb, over(d[1], d[0]));
+      return;
+    }
+    if (nt == 2 && nreg_t == 1 && nc == 0) {
+      const int jr = jt, jl = 1 - jt;
+      auto at = [&](int r, int l) { return d[(r << (1 - jr)) | (l << (1 - jl))]; };
+      const C lane[2] = {at(0, 0), at(0, 1)};
+      emit_phase(&tbits[jl], 1, nullptr, 0, lane);
+      const C up[1] = {over(at(1, 0), at(0, 0))};
+      emit_phase(nullptr, 0, &tbits[jr], 1, up);
+      phase({tbits[jr], tbits[jl]}, over(over(at(1, 1), at(0, 1)), up[0]));
+      return;
+    }
+  }
+  int enc[kMaxTargets];
+  for (int k = 0; k < nt; ++k) enc[k] = reg(tbits[k]) >= 0 ? int(kRegFlag | uint32_t(reg(tbits[k]))) : tbits[k];
+  emit(kRDiag, 0, cm, nt, enc, nt, d, 1 << nt, rreq, 0, true);
+}
+
+void Compiler::emit_diag(const Op& o) {
+  int tb[kMaxTargets], cb[kMaxControls];
+  for (int k = 0; k < o.nt; ++k) tb[k] = n_ - 1 - o.t[k];
+  for (int k = 0; k < o.nc; ++k) cb[k] = n_ - 1 - o.c[k];
+  emit_phase(tb, o.nt, cb, o.nc, o.data);
+}
+
+void Compiler::emit_dense1(const Op& o, int j) {
+  flush_reg(j);
+  qflush(j);
+  uint64_t cm = 0;
+  int rreq = 0;
+  for (int k = 0; k < o.nc; ++k) {
+    const int b = n_ - 1 - o.c[k];
+    const int r = local_[b] >= 0 ? lay_.reg_of(local_[b]) : -1;
+    if (r >= 0)
+      rreq |= 1 << r;
+    else
+      cm |= uint64_t(1) << b;
+  }
+  const C* m = o.data;
+  int mode;
+  double t, s;
+  bool neg;
+  if (cm == 0 && rreq == 0 && rotation_form(m, w_.itemsize == 16 ? 1e-14 : 4e-7, &mode, &t, &s, &neg)) {
+    double c = std::fabs(m[0].re);
+    const double norm = std::hypot(c, s);  // (complex64 entries: the rotation by atan2(s, c))
+    Event e;
+    e.kind = 0;
+    e.off = long(w_.len);
+    e.t = t;
+    e.s = s;
+    e.c = c / norm;
+    e.tan = c > 0 ? s / c : 0;
+    events_.push_back(e);
+    w_.emit_rot(j | (mode << 2), t, s);  // fold_cosines turns it into ROTS
+    sign_ ^= neg;
+    return;
+  }
+  const bool x = m[0].re == 0 && m[0].im == 0 && m[3].re == 0 && m[3].im == 0 && m[1].re == 1 && m[1].im == 0 &&
+                 m[2].re == 1 && m[2].im == 0;
+  if (x) {
+    emit(kRFlip, j, cm, 0, nullptr, 0, nullptr, 0, rreq);
+    return;
+  }
+  bool real = true;
+  for (int k = 0; k < 4 && real; ++k) real = m[k].im == 0;
+  emit(real ? kRDense1Real : kRDense1, j, cm, 0, nullptr, 0, m, 4, rreq);
+}
+
+void Compiler::emit_dense2(const Op& o) {
+  const int j0 = lay_.reg_of(local_[n_ - 1 - o.t[0]]), j1 = lay_.reg_of(local_[n_ - 1 - o.t[1]]);
+  flush_reg(j0);
+  flush_reg(j1);
+  qflush(j0);
+  qflush(j1);
+  C m[16];
+  auto role = [&](int c) { return j0 > j1 ? c : ((c & 1) << 1) | (c >> 1); };
+  for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < 4; ++c) m[4 * role(r) + role(c)] = o.data[4 * r + c];
+  bool real = true, cross = true;
+  for (int r = 0; r < 4; ++r)
+    for (int c = 0; c < 4; ++c) {
+      const C x = m[4 * r + c];
+      real = real && x.im == 0;
+      if (c != r && c != 3 - r) cross = cross && x.re == 0 && x.im == 0;
+    }
+  const int hi = std::max(j0, j1), lo = std::min(j0, j1);
+  static const int kPair[4][4] = {{-1, -1, -1, -1}, {0, -1, -1, -1}, {1, 3, -1, -1}, {2, 4, 5, -1}};
+  const int kind = (cross ? 2 : 0) + (real ? 1 : 0);
+  emit(kRDense2, kPair[hi][lo] | (kind << 3), 0, 0, nullptr, 0, m, 16);
+}
+
+void Compiler::emit_lds(const Op& o) {
+  static const C kSwapMat[16] = {{1, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1, 0}, {0, 0},
+                                 {0, 0}, {1, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 0}, {1, 0}};
+  flush_reg(-1);
+  qflush(-1);
+  const C* mat = o.kind == kSwap ? kSwapMat : o.data;
+  const int k = o.nt;
+  int bits[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  int lb[3] = {0, 0, 0};
+  for (int q = 0; q < k; ++q) bits[q] = lb[q] = local_[n_ - 1 - o.t[q]];
+  std::sort(lb, lb + k);
+  for (int q = 0; q < k; ++q) bits[4 + q] = lb[q];
+  uint64_t cm = 0;
+  for (int q = 0; q < o.nc; ++q) cm |= uint64_t(1) << (n_ - 1 - o.c[q]);
+  // (its amplitudes go through LDS under the layout the kernel holds)
+  if (relabelled_unseen_) {
+    stale_ = relabelled_unseen_ = false;
+    w_.emit(kRMap, kMapRelabel, lay_.word(), 0, nullptr, 0, nullptr, 0);
+  }
+  w_.emit(kRDenseLds, k, cm, 0, bits, 8, mat, (1 << k) * (1 << k));
+}
+
+// Rotations become ROTS records: each cosine goes to the last record before
+// it that multiplies the whole state (or to the first one). complex64 keeps
+// such runs short, so that the state stays in range: after 8 rotations the
+// next table is made one of all registers.
+void Compiler::fold_cosines() {
+  const bool single = w_.itemsize == 8;
+  const double floor = single ? 0x1p-64 : 0x1p-400;
+  const int longest = single ? 8 : 1 << 30;
+  int nrot = 0;
+  bool any = false;
+  for (const Event& e : events_) {
+    nrot += e.kind == 0;
+    any = any || e.kind == 1;
+  }
+  if (nrot == 0) return;
+  if (!any && nrot >= 5) {  // a table of its own: 64 operations against 16 saved per rotation
+    C one[16];
+    for (int r = 0; r < 16; ++r) one[r] = {1.0, 0.0};
+    emit(kRRegPhase, 0, 0, 0, nullptr, 0, one, 16);
+    any = true;
+  }
+  if (!any) return;
+  size_t target = 0;  // the record that takes the next cosines
+  while (events_[target].kind != 1) ++target;
+  const size_t first = target;
+  std::vector<double> factor(events_.size(), 1.0);
+  bool before = true;  // rotations before the first such record go to it
+  int run = 0;
+  for (size_t i = 0; i < events_.size(); ++i) {
+    Event& e = events_[i];
+    if (e.kind == 1) {
+      if (!(before && i == first)) run = 0;
+      before = before && i != first;
+      target = i;
+      continue;
+    }
+    if (e.kind == 2) {
+      if (!before && run >= longest) {
+        e.kind = 1;
+        const uint8_t all = 0;
+        std::memcpy(w_.out + e.off - kHeader + 1, &all, 1);
+        target = i;
+        run = 0;
+      }
+      continue;
+    }
+    if (!(e.c > 0) || factor[target] * e.c < floor) continue;  // stays three shears
+    factor[target] *= e.c;
+    ++run;
+    uint8_t* h = w_.out + e.off;
+    h[0] = kRRotS;
+    std::memset(h + 8, 0, 16);
+    if (single) {
+      const float t = float(e.tan);
+      std::memcpy(h + 8, &t, 4);
+    } else {
+      std::memcpy(h + 8, &e.tan, 8);
+    }
+  }
+  for (size_t i = 0; i < events_.size(); ++i) {
+    Event& e = events_[i];
+    if (e.kind != 1 || factor[i] == 1.0) continue;
+    for (C& x : e.entries) x.re *= factor[i], x.im *= factor[i];
+    w_.rewrite(e.off, e.entries.data(), int(e.entries.size()));
+  }
+}
+
+int Compiler::run(std::vector<Op>& ops, int* switches) {
+  build_items(ops);
+  dependencies();
+  lay_ = make_layout(choose_regs(true), low_);
+  w_.emit(kRMap, kMapStart, lay_.word(), 0, nullptr, 0, nullptr, 0);
+  auto runs_here = [&](int i, uint32_t R) {
+    const Item& it = items_[size_t(i)];
+    return !it.lds && !(it.need & ~R);
+  };
+  while (!ready_.empty()) {
+    std::sort(ready_.begin(), ready_.end());
+    uint32_t R = lay_.regs();
+    int pick = -1;
+    for (int i : ready_)
+      if (runs_here(i, R)) {
+        pick = i;
+        break;
+      }
+    if (pick < 0) {
+      bool reg = false;
+      for (int i : ready_) reg = reg || !items_[size_t(i)].lds;
+      if (reg) {
+        const uint32_t next = choose_regs(false);
+        change_layout(next);
+        for (int i : ready_)
+          if (runs_here(i, next)) {
+            pick = i;
+            break;
+          }
+        if (pick < 0) return -1;  // cannot happen: the layout runs a waiting gate
+      } else {
+        pick = ready_[0];
+      }
+    }
+    ready_.erase(std::find(ready_.begin(), ready_.end(), pick));
+    for (int j : succ_[size_t(pick)])
+      if (--npred_[size_t(j)] == 0) ready_.push_back(j);
+    const Item& it = items_[size_t(pick)];
+    const Op& o = it.op;
+    if (it.relabel) {
+      const int a = local_[n_ - 1 - o.t[0]], b = local_[n_ - 1 - o.t[1]];
+      for (int p = 0; p < kTileBits; ++p) {
+        if (lay_.at[p] == a)
+          lay_.at[p] = uint8_t(b);
+        else if (lay_.at[p] == b)
+          lay_.at[p] = uint8_t(a);
+        else
+          continue;
+        if (p < 8) stale_ = true;
+      }
+      relabelled_unseen_ = true;
+    } else if (it.lds) {
+      emit_lds(o);
+    } else if (o.kind == kDiag) {
+      emit_diag(o);
+    } else if (o.nt == 1) {
+      emit_dense1(o, lay_.reg_of(local_[n_ - 1 - o.t[0]]));
+    } else {
+      emit_dense2(o);
+    }
+  }
+  flush_reg(-1);
+  qflush(-1);
+  // the tile is stored in whole lines: no low bit may sit in a register
+  if (lay_.regs() & lowmask_) {
+    uint32_t R = lay_.regs() & ~lowmask_;
+    for (int b = kTileBits - 1; b >= 0 && __builtin_popcount(R) < 4; --b)
+      if (!((R >> b) & 1) && !((lowmask_ >> b) & 1)) R |= 1u << b;
+    change_layout(R);
+  } else if (relabelled_unseen_) {
+    w_.emit(kRMap, kMapRelabel, lay_.word(), 0, nullptr, 0, nullptr, 0);
+  }
+  if (w_.overflow) return 0;
+  if (reg_first_off_ >= 0 && !(gfac_.re == 1.0 && gfac_.im == 0.0)) {
+    Event& e = events_[reg_first_ev_];
+    for (C& x : e.entries) x = cmulf(x, gfac_);
+    w_.rewrite(e.off, e.entries.data(), 16);
+  }
+  if (sign_) {
+    Event* to = nullptr;
+    for (Event& e : events_)
+      if (e.kind == 1) {
+        to = &e;
+        break;
+      }
+    if (to) {
+      for (C& x : to->entries) x.re = -x.re, x.im = -x.im;
+      w_.rewrite(to->off, to->entries.data(), int(to->entries.size()));
+    } else {
+      w_.emit(kRNeg, 0, 0, 0, nullptr, 0, nullptr, 0);
+    }
+  }
+  fold_cosines();
+  *switches = switches_;
+  return 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+size_t qsim_compile_program_capacity(int nops, int dtype) {
+  if (nops < 0) return 0;
+  const size_t item = dtype == QSIM_C64 ? 8 : 16;
+  // per op at most a layout change, a rename, table and factor flushes, three
+  // records of a split diagonal and its own record (<= 64 entries)
+  const size_t per_op = 12 * kHeader + (16 + 16 + 64) * item + 64;
+  return size_t(nops) * 2 * per_op + 16 * kHeader + 64 * item;
+}
+
+int qsim_compile_program(int nqubits, const int* tile_bits, int nops, const int* op_desc, const double* op_data,
+                         const int64_t* data_offsets, int dtype, int low_bits, uint8_t* out, size_t capacity,
+                         size_t* out_bytes, int* count, int* switches) {
+  qsim::clear_error();
+  QSIM_CHECK_ARG(nqubits >= kTileBits && nqubits <= QSIM_MAX_QUBITS, "qsim_compile_program: nqubits out of range");
+  QSIM_CHECK_ARG(tile_bits != nullptr && out_bytes != nullptr && count != nullptr && switches != nullptr,
+                 "qsim_compile_program: null pointer");
+  QSIM_CHECK_ARG(nops >= 0 && (nops == 0 || (op_desc && op_data && data_offsets)), "qsim_compile_program: bad ops");
+  QSIM_CHECK_ARG(dtype == QSIM_C128 || dtype == QSIM_C64, "qsim_compile_program: bad dtype");
+  QSIM_CHECK_ARG(low_bits >= 0 && low_bits < kTileBits, "qsim_compile_program: bad low bits");
+  QSIM_CHECK_ARG(out != nullptr && capacity >= qsim_compile_program_capacity(nops, dtype),
+                 "qsim_compile_program: output buffer smaller than qsim_compile_program_capacity");
+  std::vector<Op> ops;
+  if (parse_ops(nqubits, tile_bits, nops, op_desc, op_data, data_offsets, ops, "qsim_compile_program") != QSIM_OK)
+    return QSIM_EINVAL;
+  Writer w;
+  w.out = out;
+  w.cap = capacity;
+  w.itemsize = dtype == QSIM_C64 ? 8 : 16;
+  // bits kept out of the registers at load and store: the low index bits the
+  // tile holds in place (at least the 3 the kernels keep whole lines of, at
+  // most 8: four bits are left to the registers)
+  int low = 0;
+  while (low < kTileBits && tile_bits[low] == low && low < std::max(3, std::min(low_bits, 8))) ++low;
+  low = std::max(low, 3);
+  int sw = 0;
+  Compiler c(nqubits, tile_bits, low, w);
+  if (c.run(ops, &sw) != 0) {
+    qsim::set_error("qsim_compile_program: scheduling failed");
+    return QSIM_EINVAL;
+  }
+  QSIM_CHECK_ARG(!w.overflow, "qsim_compile_program: output buffer overflow");
+  *out_bytes = w.len;
+  *count = w.count;
+  *switches = sw;
+  return QSIM_OK;
+}
+
+}  // extern "C"

@@ -362,7 +362,7 @@ class GPUExecutor:
         code = _lib.C128 if req.dtype == "complex128" else _lib.C64
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
         plan, program = blocking.compile_circuit(ops, n, cdtype, backend._low_bits(code),
-                                                 backend.blocking_ordered)
+                                                 backend.blocking_ordered, device=True)
         return code, plan, program
 
     def _run(self, req, h):
@@ -587,7 +587,7 @@ class GPUExecutor:
         code = _lib.C128 if req.dtype == "complex128" else _lib.C64
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
         plan, program = blocking.compile_circuit(ops, blocking.TILE_BITS, cdtype, backend._low_bits(code),
-                                                 backend.blocking_ordered)
+                                                 backend.blocking_ordered, device=True)
         if len(plan) > 1 or (plan and plan[0][0] != "block"):
             return code, None  # not a single pass (e.g. a 4-qubit dense block): run it alone
         count = plan[0][3] if plan else 0

@@ -1,0 +1,101 @@
+"""The programs the backend runs on the GPU (needs an MI355X): kernels
+specialised to their records against the interpreter bit for bit, and the
+final states against the numpy interpreter of the records and the oracle --
+from a given state and from |0...0>, in both precisions, with every record
+form (layouts, renames, scaled rotations, 4x4s in registers, flips)."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import OracleBackend
+from qibo_amd import Circuit, _lib, blocking, gates, models
+from qibo_amd.backend import GatePlanner, MI355XBackend
+
+from tests.program_records import records, run_program
+from tests.specialize_programs import mixed_circuit
+from tests.test_program import _phases, _random_state, _two_qubit
+
+pytestmark = pytest.mark.gpu
+
+ALL = (1 << 64) - 1
+
+
+def _passes(circuit, n, cdt, low):
+    planner = GatePlanner("complex128" if cdt == np.complex128 else "complex64")
+    ops = [op for g in circuit.queue for op in planner.plan_ops(g)]
+    for kind, payload in blocking.partition(iter(ops), n, low, False):
+        if kind == "block":
+            yield (payload[0],) + blocking.compile_program(payload[0], payload[1], n, cdt, low)
+
+
+@pytest.mark.parametrize("cdt,tol", [(np.complex128, 1e-14), (np.complex64, 3e-6)])
+def test_passes_interpreted_and_specialised(backend, rng, cdt, tol):
+    lib = backend.lib
+    n, code, low = 14, (_lib.C128 if cdt == np.complex128 else _lib.C64), (3 if cdt == np.complex128 else 4)
+    isz = np.dtype(cdt).itemsize
+    cases = [p for c in (mixed_circuit(n, rng, 1), _phases(n, rng), _two_qubit(n, rng), models.QFT(n))
+             for p in list(_passes(c, n, cdt, low))[:3]]
+    seen = set()
+    for i, (bits, prog, count) in enumerate(cases):
+        seen |= {r[0] for r in records(prog, count, isz)}
+        dev = torch.from_numpy(np.frombuffer(prog + bytes(blocking.PAD_BYTES), dtype=np.uint8).copy()).cuda()
+        tba = _lib.int_array(bits)
+        handle = ctypes.c_uint64(0)
+        for zero in (False, True):
+            psi = _random_state(n, rng, cdt)
+            start = torch.from_numpy(psi).cuda()
+            a, b = start.clone(), start.clone()
+            launch = lib.qsim_apply_blocked_from_zero if zero else lib.qsim_apply_blocked
+            _lib.check(launch(a.data_ptr(), n, code, tba, dev.data_ptr(), len(prog), count, None), lib)
+            if zero:
+                psi = np.zeros_like(psi)
+                psi[0] = 1
+            held = next(k for k in range(13) if k == 12 or bits[k] != k)
+            want = run_program(psi, n, list(bits), prog, count, max(3, min(held, low)))
+            assert np.max(np.abs(a.cpu().numpy() - want)) < tol, (i, zero)
+            rc = lib.qsim_blocked_specialize(prog, len(prog), count, code, int(zero), ctypes.byref(handle))
+            if rc != 0:  # over the compile budget
+                continue
+            _lib.check(lib.qsim_apply_blocked_specialized(handle.value, b.data_ptr(), 1, n, code, tba, ALL,
+                                                          dev.data_ptr(), 0, len(prog), count, None), lib)
+            assert torch.equal(a, b), (i, zero)
+    assert {1, 2, 5, 6, 7, 11, 12, 13, 14, 15} <= seen
+
+
+@pytest.mark.parametrize("specialize", [False, True])
+@pytest.mark.parametrize("dtype,tol", [("complex128", 1e-12), ("complex64", 2e-5)])
+@pytest.mark.parametrize("n", [5, 13, 16])
+def test_circuits_match_the_oracle(n, dtype, tol, specialize, rng):
+    be = MI355XBackend(dtype=dtype)
+    be.specialize, be.specialize_after = specialize, 1
+    circuits = [_phases(n, rng), _two_qubit(n, rng), models.QFT(n), models.random_layered_circuit(n, 8, 3, False)]
+    for c in circuits[: 2 if specialize and n < 16 else 4]:
+        want = OracleBackend().execute(c)
+        for _ in range(2):
+            got = be.execute_circuit(c).state().cpu().numpy()
+            assert np.max(np.abs(got - want)) < tol
+            be.wait_specializations()
+
+
+@pytest.mark.parametrize("specialize", [False, True])
+def test_swaps_alone_are_stored_after_every_load(specialize, rng):
+    """A pass of renames only permutes its tiles in place without an exchange
+    through LDS: no lane may store before the others have loaded."""
+    n = 21
+    be = MI355XBackend()
+    be.specialize, be.specialize_after = specialize, 1
+    c = Circuit(n)
+    for q in range(9):
+        c.add(gates.SWAP(q, 17 - q))
+    host = _random_state(n, rng, np.complex128)
+    at = np.arange(2**n)
+    src = at & 7  # qubits 18-20 stay
+    for q in range(18):
+        src |= ((at >> (n - 1 - q)) & 1) << (n - 1 - (17 - q))
+    psi, want = torch.from_numpy(host).cuda(), torch.from_numpy(host[src]).cuda()
+    for _ in range(6):
+        assert torch.equal(be.execute_circuit(c, initial_state=psi).state(), want)
+        be.wait_specializations()
