@@ -79,7 +79,7 @@ PAD_BYTES = 1056  # readable bytes required past a record stream (QSIM_BLOCKED_P
 OP_DIAG, OP_DENSE1, OP_MAP, OP_DENSE_LDS = 0, 1, 2, 3
 OP_DENSE1_REAL, OP_REG_PHASE, OP_LANE_PHASE, OP_NEG = 4, 5, 6, 7
 OP_ROT = 10
-OP_ROTS, OP_DENSE2, OP_FLIP = 13, 14, 15  # compile_program's further forms (csrc/program.hip)
+OP_ROTS, OP_DENSE2, OP_FLIP, OP_LRPMANY = 13, 14, 15, 16  # compile_program's further forms (csrc/program.hip)
 MAP_LAYOUT, MAP_START, MAP_RELABEL = 3, 4, 5  # MAP arguments that carry layouts
 ROT_RY, ROT_H, ROT_RX = 0, 1, 2  # ROT modes (arg = register bit | mode << 2)
 OP_LANE_REGPHASE, OP_QFLUSH = 11, 12
@@ -901,6 +901,8 @@ def program_flops(program: bytes, count: int, itemsize: int) -> float:
             total += 6.0 + 8.0 * (2**arg - 1)
         elif op == OP_DENSE2:
             total += _DENSE2_FLOPS[min(arg >> 3, 3)]
+        elif op == OP_LRPMANY:
+            total += 6.0 / 16 * program[off + 2]
         elif op == OP_REG_PHASE and arg & 15:
             total += 6.0 * int(_REG_DEP[arg & 15].sum()) / 16
         else:

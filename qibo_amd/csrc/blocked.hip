@@ -32,7 +32,7 @@
 //                   that stays inside the lane's registers)
 //   NEG (7)         v = -v (the -1 phase of CZ-like gates)
 //   ROT (10), ROTS (13)  rotations as three shears, or divided by their cosine
-//   LANE_REGPHASE (11), QFLUSH (12)  controlled phases of a register bit
+//   LANE_REGPHASE (11), LRPMANY (16), QFLUSH (12)  controlled phases of a register bit
 //   DENSE2 (14)     4x4 on two register bits; FLIP (15) X under conditions
 // MAP may also name any layout of the local bits (blocked_dev.h).
 // Conditions: `tmask` = condition bits outside the tile (the same for the
@@ -145,6 +145,9 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
         q_lds[threadIdx.x] = csel(lane_ok(), cmul(me[0], q), q);
         break;
       }
+      case kOpLrpMany:
+        q_lds[threadIdx.x] = lane_phases(q_lds[threadIdx.x], m, h.nt < 48u ? h.nt : 48u, lane_idx, tile_base_s);
+        break;
       case kOpQFlush: {
         const cplx<R> q = q_lds[threadIdx.x];
         q_lds[threadIdx.x] = cplx<R>{R(1), R(0)};
@@ -272,12 +275,15 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
         if (h.arg == kMapRelabel) {
           relabel_fence(v);
           layout = h.cmask;
+        } else if (h.arg == kMapLayout) {
+          flush_lane_phase(v, P, pdirty);
+          lane_idx = tile_base | lay_remap_words(lds, v, reinterpret_cast<const uint32_t*>(m));
+          layout = h.cmask;
+          break;
         } else {
           flush_lane_phase(v, P, pdirty);
-          const bool given = h.arg == kMapLayout;
-          const uint64_t from = given ? (uint64_t(h.b0) | (uint64_t(h.b1) << 32)) : layout;
-          const uint64_t to = given ? h.cmask : map_layout(h.arg);
-          lay_remap(lds, v, from, to);
+          const uint64_t to = map_layout(h.arg);
+          lay_remap(lds, v, layout, to);
           layout = to;
         }
         lane_idx = tile_base | lay_lane_index(a, layout);

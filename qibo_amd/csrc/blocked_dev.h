@@ -33,6 +33,7 @@ enum : uint32_t {
   kOpRotS = 13,          // a rotation divided by its cosine (see rots_regs): tan in the header (cmask field)
   kOpDense2 = 14,        // 4x4 on two register bits: arg = pair (kPairHi/Lo) | kind << 3, 16 entries
   kOpFlip = 15,          // X on register bit arg under conditions
+  kOpLrpMany = 16,       // nt controlled phases between register bit arg and one bit each (see lane_phases)
   kOpNop = 0xFF          // no effect (pads the programs of a batched launch to one record count)
 };
 
@@ -181,7 +182,9 @@ __device__ __forceinline__ uint32_t swz(uint32_t u) { return u ^ ((u >> 4) & 15u
 // 12 nibbles, nibble p = the local bit at position p. Mappings 0-2 are three
 // of them; a compiled program may use any (MAP records with the arguments
 // below carry the layouts in their header):
-//   kMapLayout   from the layout in `bits` to the one in `cmask`, through LDS
+//   kMapLayout   from the layout in `bits` to the one in `cmask`, through LDS;
+//                its entries hold what the interpreter would otherwise derive
+//                from them bit by bit (kMapWords dwords, see lay_remap_words)
 //   kMapStart    the layout the tile is loaded in (first record of a program)
 //   kMapRelabel  the local bits at the positions change names (a SWAP gate on
 //                them: no data moves), the layout from then on in `cmask`
@@ -209,11 +212,15 @@ __device__ __forceinline__ bool lay_low_in_regs(uint64_t L) {
 // are 1, 2, 4, 8, 16, 1, 2, 4, 16, 8, 31, 30 (the residues of the additive
 // layout's weights below), so a half-wave hits 32 distinct pairs of banks in
 // every layout whose lane positions 0-4 hold bits of five different kinds
-// {0,5,10} {1,6,11} {2,7} {3,9} {4,8}; the compiler orders them so. Linear over
-// GF(2) and a bijection (bits 5-11 are kept).
+// {0,5,10} {1,6,11} {2,7} {3,9} {4,8}; the compiler orders them so. 4-byte
+// components, which a whole wave spreads over 64 banks, also flip slot bit 5
+// with each of the local bits 6-11. Linear over GF(2) and a bijection (bits
+// 6-11 are kept, and bits 5 and 0-4 follow from them).
+template <typename R>
 __device__ __forceinline__ uint32_t swl(uint32_t u) {
-  return u ^ ((u >> 5) & 7u) ^ (((u >> 8) & 1u) << 4) ^ (((u >> 9) & 1u) << 3) ^ (((u >> 10) & 1u) * 31u) ^
-         (((u >> 11) & 1u) * 30u);
+  const uint32_t s = u ^ ((u >> 5) & 7u) ^ (((u >> 8) & 1u) << 4) ^ (((u >> 9) & 1u) << 3) ^
+                     (((u >> 10) & 1u) * 31u) ^ (((u >> 11) & 1u) * 30u);
+  return sizeof(R) == 4 ? s ^ ((uint32_t(__popc(u >> 6)) & 1u) << 5) : s;
 }
 
 // LDS slots of 8-byte components: an additive layout, slot(u) = the sum of
@@ -271,7 +278,7 @@ struct LdsSlots {
 // the swizzle `swl` otherwise.
 template <typename R>
 __device__ __forceinline__ uint32_t lay_slot(uint32_t u) {
-  return LdsSlots<R>::kAdd ? slot_f64(u) : swl(u);
+  return LdsSlots<R>::kAdd ? slot_f64(u) : swl<R>(u);
 }
 
 // All-ones where bit p of the lane number is set.
@@ -481,63 +488,118 @@ __device__ __forceinline__ void remap(R* lds, cplx<R>* v, int from, int to) {
 // `from` to its place in `to`. In the kernels specialised to one sequence the
 // layouts are constants and every access is the lane's base plus an immediate.
 template <typename R>
-__device__ __forceinline__ void lay_put(R* lds, const R* x, uint64_t L) {
+__device__ __forceinline__ void lay_put(R* lds, const R* x, uint32_t lane_slot, uint64_t L) {
   if constexpr (LdsSlots<R>::kAdd) {
-    R* base = lds + lay_lane_slot<R>(L);
+    R* base = lds + lane_slot;
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r) base[lay_reg_slot<R>(L, uint32_t(r))] = x[r];
   } else {
-    const uint32_t s = lay_lane_slot<R>(L) * uint32_t(sizeof(R));
     char* base = reinterpret_cast<char*>(lds);
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r)
-      *reinterpret_cast<R*>(base + slot_bytes(s, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R)))) = x[r];
+      *reinterpret_cast<R*>(base + slot_bytes(lane_slot, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R)))) = x[r];
   }
 }
 
 template <typename R>
-__device__ __forceinline__ void lay_get(const R* lds, R* x, uint64_t L) {
+__device__ __forceinline__ void lay_get(const R* lds, R* x, uint32_t lane_slot, uint64_t L) {
   if constexpr (LdsSlots<R>::kAdd) {
-    const R* base = lds + lay_lane_slot<R>(L);
+    const R* base = lds + lane_slot;
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r) x[r] = base[lay_reg_slot<R>(L, uint32_t(r))];
   } else {
-    const uint32_t s = lay_lane_slot<R>(L) * uint32_t(sizeof(R));
     const char* base = reinterpret_cast<const char*>(lds);
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r)
-      x[r] = *reinterpret_cast<const R*>(base + slot_bytes(s, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R))));
+      x[r] = *reinterpret_cast<const R*>(
+          base + slot_bytes(lane_slot, lay_reg_slot<R>(L, uint32_t(r)) * uint32_t(sizeof(R))));
   }
+}
+
+// The lane's slot of a layout as lay_put and lay_get take it (a slot in the
+// additive layout, bytes in the swizzled one), formed once per exchange.
+template <typename R>
+__device__ __forceinline__ uint32_t lay_base(uint64_t L) {
+  uint32_t s = lay_lane_slot<R>(L) * (LdsSlots<R>::kAdd ? 1u : uint32_t(sizeof(R)));
+  asm volatile("" : "+v"(s));
+  return s;
 }
 
 template <typename R>
 __device__ __forceinline__ void lay_remap(R* lds, cplx<R>* v, uint64_t from, uint64_t to) {
   if constexpr (LdsSlots<R>::kPair) {
-    cplx<R>* l = reinterpret_cast<cplx<R>*>(lds);  // 8-byte aligned (the buffer is 16-byte aligned)
-    lay_put(l, v, from);
+    using W = cplx<R>;
+    W* l = reinterpret_cast<W*>(lds);  // 8-byte aligned (the buffer is 16-byte aligned)
+    lay_put(l, v, lay_base<W>(from), from);
     __syncthreads();
-    lay_get(l, v, to);
+    lay_get(l, v, lay_base<W>(to), to);
     __syncthreads();
     return;
   }
+  const uint32_t sf = lay_base<R>(from), st = lay_base<R>(to);
   R x[kBReg];
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) x[r] = v[r].re;
-  lay_put(lds, x, from);
+  lay_put(lds, x, sf, from);
   __syncthreads();
-  lay_get(lds, x, to);
+  lay_get(lds, x, st, to);
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) {
     v[r].re = x[r];
     x[r] = v[r].im;
   }
-  lay_put(lds, x, from);
+  lay_put(lds, x, sf, from);
   __syncthreads();
-  lay_get(lds, x, to);
+  lay_get(lds, x, st, to);
   __syncthreads();
 #pragma clang loop unroll(full)
   for (int r = 0; r < kBReg; ++r) v[r].im = x[r];
+}
+
+// The exchange of a kMapLayout record in the interpreter, from the record's
+// words: [0, 16) the global index bits of lane bits 0-7 in the new layout (low,
+// high), [16, 24) and [24, 32) the slot bytes of the lane bits in the old and
+// the new one, [32, 48) and [48, 64) those of the registers. Deriving these
+// from the layouts took some 400 scalar instructions per exchange (8 % of a
+// layered pass). Returns the lane's index bits.
+constexpr uint32_t kMapWords = 64;
+
+__device__ __forceinline__ uint32_t lane_part(const uint32_t* w) {
+  uint32_t s = 0;
+#pragma clang loop unroll(full)
+  for (int p = 0; p < 8; ++p) s ^= lane_mask(p) & w[p];
+  asm volatile("" : "+v"(s));
+  return s;
+}
+
+template <typename R>
+__device__ __forceinline__ uint64_t lay_remap_words(R* lds, cplx<R>* v, const uint32_t* w) {
+  char* base = reinterpret_cast<char*>(lds);
+  const uint32_t sf = lane_part(w + 16), st = lane_part(w + 24);
+  R x[kBReg];
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) *reinterpret_cast<R*>(base + slot_bytes(sf, w[32 + r])) = v[r].re;
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) x[r] = *reinterpret_cast<const R*>(base + slot_bytes(st, w[48 + r]));
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    v[r].re = x[r];
+    *reinterpret_cast<R*>(base + slot_bytes(sf, w[32 + r])) = v[r].im;
+  }
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) v[r].im = *reinterpret_cast<const R*>(base + slot_bytes(st, w[48 + r]));
+  __syncthreads();
+  uint32_t lo = 0, hi = 0;
+#pragma clang loop unroll(full)
+  for (int p = 0; p < 8; ++p) {
+    lo |= lane_mask(p) & w[2 * p];
+    hi |= lane_mask(p) & w[2 * p + 1];
+  }
+  return uint64_t(lo) | (uint64_t(hi) << 32);
 }
 
 // Before a renamed layout is stored: amplitudes change places within the tile
@@ -949,6 +1011,37 @@ __device__ __forceinline__ void flush_lane_phase(cplx<R>* v, cplx<R>& P, bool& p
   P.re = R(1);
   P.im = R(0);
   pdirty = false;
+}
+
+// LRPMANY: the lane's factor multiplied by m[i] where bit i's index bit is 1,
+// for k phases. The bits follow the phases, a byte each: 0x80 | bit outside
+// the tile (the same for the workgroup: a scalar branch), else a bit fixed
+// per lane. One record instead of k LANE_REGPHASE records (20 per qubit of a
+// QFT), whose headers and factor loads cost more than the products.
+constexpr uint32_t kTileBitFlag = 0x80;
+
+template <typename R>
+__device__ __forceinline__ cplx<R> lane_phases(cplx<R> q, const cplx<R>* m, uint32_t k, uint64_t lane_idx,
+                                               uint64_t tile_base_s) {
+  const uint32_t* bw = reinterpret_cast<const uint32_t*>(m + k);
+#if QSIM_LDS_ADDITIVE  // (k is a constant in the specialised kernels)
+#pragma clang loop unroll(full)
+#endif
+  for (uint32_t i0 = 0; i0 < k; i0 += 4) {
+    const uint32_t b4 = bw[i0 / 4];
+    const cplx<R> c[4] = {m[i0], m[i0 + 1], m[i0 + 2], m[i0 + 3]};  // (past the phases: the bits and the padding)
+#pragma clang loop unroll(full)
+    for (uint32_t t = 0; t < 4; ++t) {
+      if (i0 + t >= k) continue;
+      const uint32_t b = (b4 >> (8 * t)) & 255u;
+      if (b & kTileBitFlag) {
+        if ((tile_base_s >> (b & 63u)) & 1) q = cmul(c[t], q);
+      } else {
+        q = csel(((lane_idx >> (b & 63u)) & 1) != 0, cmul(c[t], q), q);
+      }
+    }
+  }
+  return q;
 }
 
 // Multiply the registers whose bit J is set by the per-lane factor q.

@@ -46,6 +46,7 @@ struct RecView {
   uint32_t nent;  // entries (at most kMaxEntries): fixes the next record's offset
   uint32_t off;
   uint64_t to, from;  // MAP with a layout: the header's layouts
+  uint32_t nt;        // LRPMANY: phases (at most 48)
 };
 
 // What a specialised kernel does: a pass (k_blocked), a pass whose input is
@@ -61,7 +62,8 @@ bool decode(const uint8_t* prog, size_t nbytes, int ninstr, int dtype, std::vect
     BlkHdr h;
     std::memcpy(&h, prog + off, sizeof(BlkHdr));
     const uint32_t nent = h.nent < kMaxEntries ? h.nent : kMaxEntries;
-    RecView r{h.op, h.arg, h.tmask != 0, nent, off, 0, 0};
+    RecView r{h.op, h.arg, h.tmask != 0, nent, off, 0, 0, 0};
+    if (h.op == kOpLrpMany) r.nt = h.nt < 48 ? h.nt : 48;
     if (h.op == kOpMap && h.arg >= kMapLayout && h.arg <= kMapRelabel) {
       r.to = h.cmask;
       if (h.arg == kMapLayout) std::memcpy(&r.from, h.bits, 8);
@@ -89,7 +91,7 @@ uint64_t spec_cost_ms(const std::vector<RecView>& recs) {
   for (const RecView& r : recs) {
     switch (r.op) {
       case kOpRot: case kOpRotS: case kOpRegPhase: case kOpNeg: case kOpFlip: c += 15; break;
-      case kOpLanePhase: case kOpLaneRegPhase: case kOpQFlush: c += 30; break;
+      case kOpLanePhase: case kOpLaneRegPhase: case kOpQFlush: case kOpLrpMany: c += 30; break;
       case kOpMap: case kOpDense1: case kOpDense1Real: c += 100; break;
       case kOpDiag: case kOpDense2: c += 120; break;
       case kOpDenseLds: c += 300; break;
@@ -110,6 +112,7 @@ std::string structure_key(const std::vector<RecView>& recs, int dtype, int varia
     key.push_back(char(r.arg));
     key.push_back(char(r.cond ? 1 : 0));
     key.push_back(char(r.nent));  // <= 64
+    key.push_back(char(r.nt));
     if (r.op == kOpMap && r.arg >= kMapLayout && r.arg <= kMapRelabel)  // the layouts are constants of the kernel
       for (int i = 0; i < 6; ++i) {
         key.push_back(char((r.to >> (8 * i)) & 255));
@@ -144,6 +147,9 @@ void emit_record(std::string& s, const RecView& r, bool dbl, uint64_t& layout) {
   switch (r.op) {
     case kOpLaneRegPhase:
       s += "      Q = csel(lane_ok(), cmul(me[0], Q), Q);\n";
+      break;
+    case kOpLrpMany:
+      s += "      Q = lane_phases(Q, m, " + std::to_string(r.nt) + "u, lane_idx, tile_base_s);\n";
       break;
     case kOpQFlush:
       s += "      flush_q_bit<R, " + J + ">(v, Q);\n"

@@ -17,7 +17,7 @@
 //  * a diagonal gate between one register bit and lane bits is split into a
 //    table, a per-lane phase and a controlled phase (0.30 CU-cycles as DIAG);
 //  * phases whose conditions lie outside the tile are skipped by whole
-//    workgroups;
+//    workgroups; the controlled phases of one register bit share a record;
 //  * conditional X gates exchange registers instead of multiplying.
 
 #include <algorithm>
@@ -28,7 +28,8 @@
 
 namespace {
 
-constexpr uint8_t kRRotS = 13, kRDense2 = 14, kRFlip = 15;
+constexpr uint8_t kRRotS = 13, kRDense2 = 14, kRFlip = 15, kRLrpMany = 16;
+constexpr int kMaxPhases = 48;  // of one LRPMANY record
 constexpr int kMapLayout = 3, kMapStart = 4, kMapRelabel = 5;
 
 // Local bits of one kind share the low bits of their LDS slot (blocked_dev.h:
@@ -90,6 +91,15 @@ Layout make_layout(uint32_t R, int low) {
   return l;
 }
 
+// LDS slot of a local index in the interpreter's exchanges (swl in
+// blocked_dev.h: linear, so the slots of single bits are combined by XOR).
+uint32_t slot_of(uint32_t u, int itemsize) {
+  uint32_t s = u ^ ((u >> 5) & 7u) ^ (((u >> 8) & 1u) << 4) ^ (((u >> 9) & 1u) << 3) ^ (((u >> 10) & 1u) * 31u) ^
+               (((u >> 11) & 1u) * 30u);
+  if (itemsize == 8) s ^= uint32_t(__builtin_popcount(u >> 6) & 1) << 5;
+  return s * uint32_t(itemsize / 2);
+}
+
 class Compiler {
  public:
   Compiler(int n, const int* tile_bits, int low, Writer& w) : n_(n), tb_(tile_bits), low_(low), w_(w) {
@@ -122,6 +132,7 @@ class Compiler {
   C gfac_ = {1.0, 0.0};
   bool sign_ = false;
   int qpend_ = -1;
+  std::vector<std::pair<int, C>> phases_;  // controlled phases of register qpend_ not emitted yet: (bit, phase)
   int switches_ = 0;
 
   // rotations and the records that can take their cosines, in order
@@ -143,6 +154,7 @@ class Compiler {
   void change_layout(uint32_t R);
   void flush_reg(int j);
   void qflush(int j);
+  void emit_phases();
   void emit_diag(const Op& o);
   void emit_phase(const int* tbits, int nt, const int* cbits, int nc, const C* d);
   void emit_dense1(const Op& o, int j);
@@ -379,14 +391,61 @@ void Compiler::change_layout(uint32_t R) {
   const uint64_t from = lay_.word();
   int bytes[8];
   for (int i = 0; i < 8; ++i) bytes[i] = int((from >> (8 * i)) & 255);
-  w_.emit(kRMap, kMapLayout, to.word(), 0, bytes, 8, nullptr, 0);
+  // the interpreter's words (lay_remap_words)
+  uint32_t words[64];
+  auto slot = [&](const Layout& l, int p) { return slot_of(1u << l.at[p], w_.itemsize); };
+  for (int p = 0; p < 8; ++p) {
+    const uint64_t g = uint64_t(1) << gbit(to.at[p]);
+    words[2 * p] = uint32_t(g);
+    words[2 * p + 1] = uint32_t(g >> 32);
+    words[16 + p] = slot(lay_, p);
+    words[24 + p] = slot(to, p);
+  }
+  for (int r = 0; r < 16; ++r) {
+    words[32 + r] = words[48 + r] = 0;
+    for (int j = 0; j < 4; ++j)
+      if ((r >> j) & 1) words[32 + r] ^= slot(lay_, 8 + j), words[48 + r] ^= slot(to, 8 + j);
+  }
+  const C none[32] = {};
+  const size_t at = w_.len + kHeader;
+  w_.emit(kRMap, kMapLayout, to.word(), 0, bytes, 8, none, int(sizeof(words)) / w_.itemsize);
+  if (!w_.overflow) std::memcpy(w_.out + at, words, sizeof(words));
   lay_ = to;
   stale_ = relabelled_unseen_ = false;
   ++switches_;
 }
 
+// The collected phases of register qpend_, before the lanes' bits change
+// names or its factor is applied.
+void Compiler::emit_phases() {
+  const int k = int(phases_.size());
+  if (k == 0) return;
+  if (k <= 2) {
+    for (const auto& p : phases_) {
+      const uint64_t cm = uint64_t(1) << p.first, tm = outside(cm);
+      emit(kRLaneRegPhase, qpend_, cm & ~tm, 0, nullptr, 0, &p.second, 1, 0, tm);
+    }
+  } else {
+    C data[64] = {};
+    uint8_t bits[kMaxPhases] = {};
+    for (int i = 0; i < k; ++i) {
+      data[i] = phases_[size_t(i)].second;
+      const int b = phases_[size_t(i)].first;
+      bits[i] = uint8_t(local_[b] < 0 ? 0x80 | b : b);
+    }
+    const int extra = (k + w_.itemsize - 1) / w_.itemsize;
+    emit(kRLrpMany, qpend_, 0, k, nullptr, 0, data, k + extra, 0, 0, true);
+    if (!w_.overflow) {
+      const size_t raw = (size_t(k + extra) * size_t(w_.itemsize) + 15) / 16 * 16;
+      std::memcpy(w_.out + w_.len - raw + size_t(k) * size_t(w_.itemsize), bits, size_t(k));
+    }
+  }
+  phases_.clear();
+}
+
 void Compiler::qflush(int j) {
   if (qpend_ < 0 || (j >= 0 && j != qpend_)) return;
+  emit_phases();
   emit(kRQFlush, qpend_, 0, 0, nullptr, 0, nullptr, 0);
   qpend_ = -1;
 }
@@ -469,6 +528,11 @@ void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, co
       if (qpend_ != j) {
         qflush(-1);
         qpend_ = j;
+      }
+      if ((cm & (cm - 1)) == 0) {  // one condition: collected
+        if (int(phases_.size()) == kMaxPhases) emit_phases();
+        phases_.emplace_back(__builtin_ctzll(cm), d[0]);
+        return;
       }
       const uint64_t tm = outside(cm);
       emit(kRLaneRegPhase, j, cm & ~tm, 0, nullptr, 0, d, 1, 0, tm);
@@ -718,6 +782,7 @@ int Compiler::run(std::vector<Op>& ops, int* switches) {
     const Item& it = items_[size_t(pick)];
     const Op& o = it.op;
     if (it.relabel) {
+      emit_phases();  // (they name bits, which are about to change places)
       const int a = local_[n_ - 1 - o.t[0]], b = local_[n_ - 1 - o.t[1]];
       for (int p = 0; p < kTileBits; ++p) {
         if (lay_.at[p] == a)
@@ -784,8 +849,8 @@ size_t qsim_compile_program_capacity(int nops, int dtype) {
   const size_t item = dtype == QSIM_C64 ? 8 : 16;
   // per op at most a layout change, a rename, table and factor flushes, three
   // records of a split diagonal and its own record (<= 64 entries)
-  const size_t per_op = 12 * kHeader + (16 + 16 + 64) * item + 64;
-  return size_t(nops) * 2 * per_op + 16 * kHeader + 64 * item;
+  const size_t per_op = 12 * kHeader + (16 + 16 + 64) * item + 256 + 64;
+  return size_t(nops) * 2 * per_op + 16 * kHeader + 64 * item + 2 * 256;
 }
 
 int qsim_compile_program(int nqubits, const int* tile_bits, int nops, const int* op_desc, const double* op_data,

@@ -163,6 +163,14 @@ def run_program(state, n, tile_bits, program, count, low):
             assert rreq == 0 and qbit in (None, arg)
             qbit = arg
             pend = np.where(cond & ((reg >> arg) & 1)[None, :].astype(bool), pend * mat[0], pend)
+        elif op == blocking.OP_LRPMANY:
+            assert rreq == 0 and cmask == 0 and tmask == 0 and qbit in (None, arg) and 3 <= nt <= 48
+            qbit = arg
+            for k, b in enumerate(mat[nt:].tobytes()[:nt]):
+                assert bool(b & 0x80) == ((b & 63) not in tile_bits)
+                assert (b & 63) not in [tile_bits[names[8 + j]] for j in range(4)]
+                on = (((gidx >> (b & 63)) & 1) == 1) & ((reg >> arg) & 1)[None, :].astype(bool)
+                pend = np.where(on, pend * mat[k], pend)
         elif op == blocking.OP_QFLUSH:
             assert qbit == arg
             v, pend, qbit = v * pend, np.ones_like(v), None

@@ -62,7 +62,7 @@ def test_passes_interpreted_and_specialised(backend, rng, cdt, tol):
             _lib.check(lib.qsim_apply_blocked_specialized(handle.value, b.data_ptr(), 1, n, code, tba, ALL,
                                                           dev.data_ptr(), 0, len(prog), count, None), lib)
             assert torch.equal(a, b), (i, zero)
-    assert {1, 2, 5, 6, 7, 11, 12, 13, 14, 15} <= seen
+    assert {1, 2, 5, 6, 7, 11, 12, 13, 14, 15, 16} <= seen
 
 
 @pytest.mark.parametrize("specialize", [False, True])
