@@ -961,7 +961,8 @@ class MI355XBackend(GatePlanner):
                                           len(qubits), outcome, norm, self._stream(state)), self.lib)
         return state
 
-    def run_queue(self, queue, state: torch.Tensor, nqubits: int, zero_pending: bool = False) -> torch.Tensor:
+    def run_queue(self, queue, state: torch.Tensor, nqubits: int, zero_pending: bool = False,
+                  sampled: Optional[bool] = None) -> torch.Tensor:
         """Apply the gates of ``queue`` in order (the loop of abstract.py:3321-3322).
 
         With ``self.blocking`` (the default) consecutive gates are grouped into
@@ -974,8 +975,11 @@ class MI355XBackend(GatePlanner):
         no-op on the state); other special gates run in order between passes.
         With ``zero_pending`` the contents of ``state`` are not yet written and
         stand for |0...0>: a first blocked pass produces it itself, anything
-        else fills it first.
+        else fills it first. ``sampled``: shots will be drawn from the final
+        state (default: the queue holds a measurement); see ``_keeps_samples``.
         """
+        keep = self._keeps_samples(state.dtype == torch.complex64, nqubits,
+                                   lambda: any(kinds.is_measurement(g) for g in queue) if sampled is None else sampled)
         # [|0...0> still to be materialised, support, unwritten]: the support
         # is the mask of index bits that may be 1 in a nonzero amplitude (None:
         # any); the passes from |0...0> grow it by their tile bits, skip the
@@ -993,6 +997,8 @@ class MI355XBackend(GatePlanner):
         if nqubits < blocking.TILE_BITS:
             return self._run_small(queue, state, nqubits)
         key = self._queue_key(queue, nqubits, state, zero_pending) if self.program_cache else None
+        if key is not None:
+            key += (keep,)
         if key is not None:
             actions = self._cache_get(key)
             if actions is not None:
@@ -1019,7 +1025,7 @@ class MI355XBackend(GatePlanner):
                 yield from self.plan_ops(gate)
 
         while True:
-            state = self._run_blocked(segment(), state, nqubits, zero, record)
+            state = self._run_blocked(segment(), state, nqubits, zero, record, keep)
             self._complete(state, nqubits, zero)  # (no blocked pass produced |0...0>, or left it unwritten)
             if not stop:
                 if record is not None:
@@ -1276,13 +1282,25 @@ class MI355XBackend(GatePlanner):
                                                           zero[1], self._stream(state)), self.lib)
             zero[2] = False
 
-    def _run_blocked(self, ops, state: torch.Tensor, nqubits: int, zero=None, record=None) -> torch.Tensor:
+    @staticmethod
+    def _keeps_samples(single: bool, nqubits: int, sampled) -> bool:
+        """Whether a circuit's passes use compile_pass's records, whose rounding
+        fixes the shots of seeded complex64 runs. compile_program rounds each
+        gate differently, by about 6e-8 of the probability it moves in single
+        precision: above 18 qubits that is more than an entry of the cumulative
+        sum (2^-n), so seeded draws would land on other bitstrings. In double
+        precision the entry of the largest register (2^-36) is far above it."""
+        return single and nqubits > _SAMPLED_C64_QUBITS and sampled()
+
+    def _run_blocked(self, ops, state: torch.Tensor, nqubits: int, zero=None, record=None,
+                     keep: bool = False) -> torch.Tensor:
         """Partition ``ops`` (an iterable of planned gates) into passes and
         launch each pass as soon as it is compiled, so the host plans and
         compiles pass k+1 while the GPU runs pass k. ``zero`` = [True] means the
         state still stands for |0...0>: the first pass starts from it (or the
         state is filled before a one-gate launch); it is cleared once done.
-        ``record`` (a list) receives the launches for the program cache."""
+        ``record`` (a list) receives the launches for the program cache;
+        ``keep``: see ``_keeps_samples``."""
         code = self._dtype_code(state)
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
         low = self._low_bits(code)
@@ -1300,7 +1318,10 @@ class MI355XBackend(GatePlanner):
                     record.append(("single", payload))
                 continue
             tile_bits, pops = payload
-            program, count = blocking.compile_program(tile_bits, pops, nqubits, cdtype, low, ordered)
+            if keep:
+                program, count, _ = blocking.compile_pass(tile_bits, pops, nqubits, cdtype, ordered)
+            else:
+                program, count = blocking.compile_program(tile_bits, pops, nqubits, cdtype, low, ordered)
             # zero padding: the kernel may read QSIM_BLOCKED_PAD bytes past the stream
             host = torch.frombuffer(bytearray(program) + bytes(blocking.PAD_BYTES), dtype=torch.uint8).pin_memory()
             prog = host.to(state.device, non_blocking=True)
@@ -1745,6 +1766,7 @@ def _dm_pair(op: _Op, nqubits: int) -> List[_Op]:
     return [op, col]
 _BLOCK_OP = _Op("block", (), (), None)
 _ALL_BITS = (1 << 64) - 1  # support mask of a pass over every tile
+_SAMPLED_C64_QUBITS = 18  # complex64 registers above keep compile_pass's rounding when shots are drawn
 _FILL_FROM_ZERO_QUBITS = 22  # from this size on the first pass from |0...0> runs tile 0 alone
 _TILE_MASKS = {}  # tile bits -> their index mask
 

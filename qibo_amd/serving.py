@@ -361,8 +361,9 @@ class GPUExecutor:
         ops = [op for g in req.circuit.queue for op in backend.plan_ops(g)]
         code = _lib.C128 if req.dtype == "complex128" else _lib.C64
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
+        keep = backend._keeps_samples(code == _lib.C64, n, lambda: req.kind == "shots")
         plan, program = blocking.compile_circuit(ops, n, cdtype, backend._low_bits(code),
-                                                 backend.blocking_ordered, device=True)
+                                                 backend.blocking_ordered, device=not keep)
         return code, plan, program
 
     def _run(self, req, h):
@@ -384,7 +385,8 @@ class GPUExecutor:
             code = _lib.C128 if req.dtype == "complex128" else _lib.C64
             with torch.cuda.stream(stream):
                 state = backend._alloc_state(n, req.dtype)
-                state = backend.run_queue(list(req.circuit.queue), state, n, zero_pending=True)
+                state = backend.run_queue(list(req.circuit.queue), state, n, zero_pending=True,
+                                          sampled=req.kind == "shots")
                 tail = _Tail(backend, n, code, req.kind, req.nshots)
                 tail.set_uniforms(req.seed)
                 tail.launch(state, stream.cuda_stream)

@@ -99,3 +99,27 @@ def test_swaps_alone_are_stored_after_every_load(specialize, rng):
     for _ in range(6):
         assert torch.equal(be.execute_circuit(c, initial_state=psi).state(), want)
         be.wait_specializations()
+
+
+def test_sampled_complex64_keeps_its_rounding(backend64):
+    """complex64 registers above 18 qubits keep compile_pass's records when
+    shots are drawn (their rounding decides the seeded shots); the same circuit
+    without a measurement, and smaller registers, run compile_program's."""
+    for n, kept in ((18, False), (19, True)):
+        c = models.random_layered_circuit(n, 3, seed=4)
+        planner = GatePlanner("complex64")
+        ops = [op for g in c.queue if g.__class__.__name__ != "M" for op in planner.plan_ops(g)]
+        state = torch.zeros(2**n, dtype=torch.complex64, device="cuda")
+        state[0] = 1
+        for kind, payload in blocking.partition(iter(ops), n, 4, False):
+            bits, pops = payload
+            prog, count, _ = blocking.compile_pass(bits, pops, n, np.complex64)
+            dev = torch.from_numpy(np.frombuffer(prog + bytes(blocking.PAD_BYTES), dtype=np.uint8).copy()).cuda()
+            _lib.check(backend64.lib.qsim_apply_blocked(state.data_ptr(), n, _lib.C64, _lib.int_array(bits),
+                                                        dev.data_ptr(), len(prog), count, None), backend64.lib)
+        torch.cuda.synchronize()
+        start = torch.zeros_like(state)
+        start[0] = 1
+        assert torch.equal(backend64.execute_circuit(c, initial_state=start).state(), state) == kept
+        plain = models.random_layered_circuit(n, 3, seed=4, measure=False)
+        assert not torch.equal(backend64.execute_circuit(plain, initial_state=start).state(), state)
