@@ -79,6 +79,7 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
   prog += blockIdx.z * a.prog_stride;
   const uint64_t tile_base = tile_origin(a, tile);
 
+  const uint32_t fetched = prefetch_program(a, prog);
   // the layout the tile is loaded in: a program's first record may name it
   uint64_t layout = kLayout0;
   Hdr h = {};
@@ -101,6 +102,7 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
       load_lane(a, psi, lane_idx, layout, rb, v);
     }
   }
+  prefetch_done(fetched);
 
   cplx<R> P;  // pending per-lane factor of LANE_PHASE records
   P.re = R(1);
@@ -280,11 +282,13 @@ void k_blocked(const BlkArgs a, const uint8_t* __restrict__ prog,
           lane_idx = tile_base | lay_remap_words(lds, v, reinterpret_cast<const uint32_t*>(m));
           layout = h.cmask;
           break;
-        } else {
+        } else {  // one of the three mappings, from another of them
           flush_lane_phase(v, P, pdirty);
-          const uint64_t to = map_layout(h.arg);
-          lay_remap(lds, v, layout, to);
-          layout = to;
+          const int nmap = h.arg < 3 ? int(h.arg) : 0;
+          remap(lds, v, layout == kLayout1 ? 1 : (layout == kLayout2 ? 2 : 0), nmap);
+          layout = map_layout(uint32_t(nmap));
+          lane_idx = tile_base | insert_local(local_index(nmap, threadIdx.x, 0), a);
+          break;
         }
         lane_idx = tile_base | lay_lane_index(a, layout);
         break;

@@ -32,7 +32,7 @@ enum : uint32_t {
   kOpQFlush = 12,        // apply Q to the registers with bit arg set, reset it to 1
   kOpRotS = 13,          // a rotation divided by its cosine (see rots_regs): tan in the header (cmask field)
   kOpDense2 = 14,        // 4x4 on two register bits: arg = pair (kPairHi/Lo) | kind << 3, 16 entries
-  kOpFlip = 15,          // X on register bit arg under conditions
+  kOpFlip = 15,          // X on register bit arg where register bits allow it
   kOpLrpMany = 16,       // nt controlled phases between register bit arg and one bit each (see lane_phases)
   kOpNop = 0xFF          // no effect (pads the programs of a batched launch to one record count)
 };
@@ -85,6 +85,22 @@ __device__ __forceinline__ uint64_t tile_origin(const BlkArgs& a, uint64_t tile)
   for (int i = 0; i < int(a.nfree); ++i) b |= ((tile >> i) & 1) << a.fbits[i];
   return b;
 }
+
+// Launches of few tiles (small registers, the passes on a part of the tiles)
+// read their program once: the lanes fetch its lines into the L2 cache while
+// the amplitudes load, so that the records' scalar loads do not each wait for
+// memory. Consumed by prefetch_done after the amplitudes.
+constexpr uint64_t kPrefetchTiles = 512;
+
+__device__ __forceinline__ uint32_t prefetch_program(const BlkArgs& a, const uint8_t* prog) {
+  uint32_t x = 0;
+  if (a.ntiles <= kPrefetchTiles)
+    for (uint64_t o = uint64_t(threadIdx.x) * 128; o < a.nbytes; o += uint64_t(kBT) * 128)
+      x ^= *reinterpret_cast<const uint32_t*>(prog + o);
+  return x;
+}
+
+__device__ __forceinline__ void prefetch_done(uint32_t x) { asm volatile("" ::"v"(x)); }
 
 // A header decoded from its eight dwords. gfx950 has no scalar byte loads, so
 // the header is read as whole dwords (uniform address: scalar loads) and the
@@ -577,28 +593,34 @@ template <typename R>
 __device__ __forceinline__ uint64_t lay_remap_words(R* lds, cplx<R>* v, const uint32_t* w) {
   char* base = reinterpret_cast<char*>(lds);
   const uint32_t sf = lane_part(w + 16), st = lane_part(w + 24);
-  R x[kBReg];
-#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) *reinterpret_cast<R*>(base + slot_bytes(sf, w[32 + r])) = v[r].re;
-  __syncthreads();
-#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) x[r] = *reinterpret_cast<const R*>(base + slot_bytes(st, w[48 + r]));
-  __syncthreads();
-#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) {
-    v[r].re = x[r];
-    *reinterpret_cast<R*>(base + slot_bytes(sf, w[32 + r])) = v[r].im;
-  }
-  __syncthreads();
-#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) v[r].im = *reinterpret_cast<const R*>(base + slot_bytes(st, w[48 + r]));
-  __syncthreads();
   uint32_t lo = 0, hi = 0;
 #pragma clang loop unroll(full)
   for (int p = 0; p < 8; ++p) {
     lo |= lane_mask(p) & w[2 * p];
     hi |= lane_mask(p) & w[2 * p + 1];
   }
+  // all words are read before the first LDS access: scalar loads and LDS share
+  // a counter, so a load between accesses would wait for each of them
+  uint32_t f[kBReg], t[kBReg];
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) f[r] = w[32 + r], t[r] = w[48 + r];
+  __builtin_amdgcn_sched_barrier(0);
+  R x[kBReg];
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) *reinterpret_cast<R*>(base + slot_bytes(sf, f[r])) = v[r].re;
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) x[r] = *reinterpret_cast<const R*>(base + slot_bytes(st, t[r]));
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    v[r].re = x[r];
+    *reinterpret_cast<R*>(base + slot_bytes(sf, f[r])) = v[r].im;
+  }
+  __syncthreads();
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) v[r].im = *reinterpret_cast<const R*>(base + slot_bytes(st, t[r]));
+  __syncthreads();
   return uint64_t(lo) | (uint64_t(hi) << 32);
 }
 
@@ -811,34 +833,6 @@ __device__ __forceinline__ R rots_t(const Hdr& h) {
 constexpr int kPairHi[6] = {1, 2, 3, 2, 3, 3};
 constexpr int kPairLo[6] = {0, 0, 0, 1, 1, 2};
 
-template <typename R, int HI, int LO, int KIND>
-__device__ __forceinline__ void dense2_regs(cplx<R>* v, const cplx<R>* m) {
-#pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) {
-    if (((r >> HI) & 1) || ((r >> LO) & 1)) continue;
-    const int at[4] = {r, r | (1 << LO), r | (1 << HI), r | (1 << HI) | (1 << LO)};
-    const cplx<R> x[4] = {v[at[0]], v[at[1]], v[at[2]], v[at[3]]};
-#pragma clang loop unroll(full)
-    for (int i = 0; i < 4; ++i) {
-      cplx<R> y;
-      if constexpr (KIND == 0) {
-        y = cfma(m[4 * i + 3], x[3], cfma(m[4 * i + 2], x[2], cfma(m[4 * i + 1], x[1], cmul(m[4 * i], x[0]))));
-      } else if constexpr (KIND == 1) {
-        y.re = fmaR(m[4 * i + 3].re, x[3].re,
-                    fmaR(m[4 * i + 2].re, x[2].re, fmaR(m[4 * i + 1].re, x[1].re, m[4 * i].re * x[0].re)));
-        y.im = fmaR(m[4 * i + 3].re, x[3].im,
-                    fmaR(m[4 * i + 2].re, x[2].im, fmaR(m[4 * i + 1].re, x[1].im, m[4 * i].re * x[0].im)));
-      } else if constexpr (KIND == 2) {
-        y = cfma(m[4 * i + 3 - i], x[3 - i], cmul(m[4 * i + i], x[i]));
-      } else {
-        y.re = fmaR(m[4 * i + 3 - i].re, x[3 - i].re, m[4 * i + i].re * x[i].re);
-        y.im = fmaR(m[4 * i + 3 - i].re, x[3 - i].im, m[4 * i + i].re * x[i].im);
-      }
-      v[at[i]] = y;
-    }
-  }
-}
-
 // x *= d with d uniform: exactly cmul(d, x) (re = fma(d.re, x.re, -(d.im x.im)),
 // im = fma(d.re, x.im, d.im x.re)).
 __device__ __forceinline__ void cmul_inplace(cplx<double>& x, cplx<double> d) {
@@ -892,6 +886,34 @@ __device__ __forceinline__ cplx<R> csel(bool c, cplx<R> a, cplx<R> b) {
   return r;
 }
 
+template <typename R, int HI, int LO, int KIND>
+__device__ __forceinline__ void dense2_regs(cplx<R>* v, const cplx<R>* m) {
+#pragma clang loop unroll(full)
+  for (int r = 0; r < kBReg; ++r) {
+    if (((r >> HI) & 1) || ((r >> LO) & 1)) continue;
+    const int at[4] = {r, r | (1 << LO), r | (1 << HI), r | (1 << HI) | (1 << LO)};
+    const cplx<R> x[4] = {v[at[0]], v[at[1]], v[at[2]], v[at[3]]};
+#pragma clang loop unroll(full)
+    for (int i = 0; i < 4; ++i) {
+      cplx<R> y;
+      if constexpr (KIND == 0) {
+        y = cfma(m[4 * i + 3], x[3], cfma(m[4 * i + 2], x[2], cfma(m[4 * i + 1], x[1], cmul(m[4 * i], x[0]))));
+      } else if constexpr (KIND == 1) {
+        y.re = fmaR(m[4 * i + 3].re, x[3].re,
+                    fmaR(m[4 * i + 2].re, x[2].re, fmaR(m[4 * i + 1].re, x[1].re, m[4 * i].re * x[0].re)));
+        y.im = fmaR(m[4 * i + 3].re, x[3].im,
+                    fmaR(m[4 * i + 2].re, x[2].im, fmaR(m[4 * i + 1].re, x[1].im, m[4 * i].re * x[0].im)));
+      } else if constexpr (KIND == 2) {
+        y = cfma(m[4 * i + 3 - i], x[3 - i], cmul(m[4 * i + i], x[i]));
+      } else {
+        y.re = fmaR(m[4 * i + 3 - i].re, x[3 - i].re, m[4 * i + i].re * x[i].re);
+        y.im = fmaR(m[4 * i + 3 - i].re, x[3 - i].im, m[4 * i + i].re * x[i].im);
+      }
+      v[at[i]] = y;
+    }
+  }
+}
+
 // FLIP: X on register bit J where the conditions hold.
 template <typename R, int J>
 __device__ __forceinline__ void flip_regs(cplx<R>* v, const Hdr& h, uint64_t lane_idx) {
@@ -900,9 +922,17 @@ __device__ __forceinline__ void flip_regs(cplx<R>* v, const Hdr& h, uint64_t lan
   for (int r = 0; r < kBReg; ++r) {
     if ((r >> J) & 1) continue;
     if (!reg_ok(r, h.rreq)) continue;
-    const cplx<R> a = v[r], b = v[r | (1 << J)];
-    v[r] = csel(on, b, a);
-    v[r | (1 << J)] = csel(on, a, b);
+    cplx<R>&a = v[r], &b = v[r | (1 << J)];
+#if QSIM_LDS_ADDITIVE
+    const cplx<R> t = a;
+#else
+    // a value of its own: recognised as an exchange, the interpreter's loop
+    // copied all 16 amplitudes around it (0.29 against 0.13 CU-cycles per amplitude)
+    cplx<R> t = a;
+    asm volatile("" : "+v"(t.re), "+v"(t.im));
+#endif
+    a = csel(on, b, a);
+    b = csel(on, t, b);
   }
 }
 

@@ -382,6 +382,7 @@ std::string make_source(const std::vector<RecView>& recs, int dtype, int variant
   psi += blockIdx.z * a.state_stride;
   prog += blockIdx.z * a.prog_stride;
   const uint64_t tile_base = tile_origin(a, tile);
+  const uint32_t fetched = prefetch_program(a, prog);
 )";
   uint64_t layout = kLayout0;
   if (!recs.empty() && recs[0].op == kOpMap && recs[0].arg == kMapStart) layout = recs[0].to;
@@ -397,6 +398,7 @@ std::string make_source(const std::vector<RecView>& recs, int dtype, int variant
   else
     s += "    load_lane(a, psi, lane_idx, " + hex(layout) + ", rb, v);\n";
   s += R"(  }
+  prefetch_done(fetched);
   cplx<R> P;
   P.re = R(1);
   P.im = R(0);
