@@ -700,7 +700,10 @@ void Compiler::fold_cosines() {
   size_t target = 0;  // the record that takes the next cosines
   while (events_[target].kind != 1) ++target;
   const size_t first = target;
-  std::vector<double> factor(events_.size(), 1.0);
+  // 1 / sqrt(1 + t^2) of the rounded tangent, multiplied in extended precision:
+  // the rotations keep the norm, whatever their number (products of rounded
+  // cosines put a 23-qubit circuit of 400 gates 4e-15 off it)
+  std::vector<long double> factor(events_.size(), 1.0L);
   bool before = true;  // rotations before the first such record go to it
   int run = 0;
   for (size_t i = 0; i < events_.size(); ++i) {
@@ -721,14 +724,16 @@ void Compiler::fold_cosines() {
       }
       continue;
     }
-    if (!(e.c > 0) || factor[target] * e.c < floor) continue;  // stays three shears
-    factor[target] *= e.c;
+    const double tan = single ? double(float(e.tan)) : e.tan;
+    const long double cosine = 1.0L / std::sqrt(1.0L + (long double)(tan) * tan);
+    if (!(e.c > 0) || factor[target] * cosine < floor) continue;  // stays three shears
+    factor[target] *= cosine;
     ++run;
     uint8_t* h = w_.out + e.off;
     h[0] = kRRotS;
     std::memset(h + 8, 0, 16);
     if (single) {
-      const float t = float(e.tan);
+      const float t = float(tan);
       std::memcpy(h + 8, &t, 4);
     } else {
       std::memcpy(h + 8, &e.tan, 8);
@@ -736,8 +741,8 @@ void Compiler::fold_cosines() {
   }
   for (size_t i = 0; i < events_.size(); ++i) {
     Event& e = events_[i];
-    if (e.kind != 1 || factor[i] == 1.0) continue;
-    for (C& x : e.entries) x.re *= factor[i], x.im *= factor[i];
+    if (e.kind != 1 || factor[i] == 1.0L) continue;
+    for (C& x : e.entries) x.re = double(x.re * factor[i]), x.im = double(x.im * factor[i]);
     w_.rewrite(e.off, e.entries.data(), int(e.entries.size()));
   }
 }
