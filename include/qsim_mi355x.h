@@ -131,6 +131,13 @@ int qsim_apply_swap(void* state, int nqubits, int dtype, int q0, int q1, const i
 int qsim_apply_fused(void* state, int nqubits, int dtype, const int* targets, int ntargets,
                      const void* matrix_dev, void* stream);
 
+/* Two uncontrolled blocks of 4 or 5 targets each, the first one first, on a
+ * complex128 state of at least 13 qubits in one pass over it: the same
+ * arithmetic as two calls of qsim_apply_fused. */
+int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const int* targets1, int ntargets1,
+                          const void* matrix1_dev, const int* targets2, int ntargets2, const void* matrix2_dev,
+                          void* stream);
+
 /* Many gates in one pass over the state: the gate loop of
  * Backend._execute_circuit (abstract.py:3321-3322, each step an apply_gate,
  * abstract.py:2322-2361) for a run of consecutive gates that the host has

@@ -680,25 +680,56 @@ class MI355XBackend(GatePlanner):
                 raise_error(NotImplementedError, "controlled blocks on more than 3 targets")
             if len(op.targets) > 5:
                 raise_error(NotImplementedError, "dense blocks on more than 5 qubits are not supported")
-            # the block's matrix goes to the device once per op (a pinned,
-            # stream-ordered copy) and is reused when the op runs again
-            cached = op.dev
-            cur = torch.cuda.current_stream(state.device)
-            if cached is not None and cached[0] == state.device and cached[1] == npdt:
-                m = cached[2]
-                if cached[4] != cur.cuda_stream:
-                    cur.wait_event(cached[3])  # the upload ran on another stream
-            else:
-                host = torch.from_numpy(np.ascontiguousarray(op.data, dtype=npdt)).pin_memory()
-                m = host.to(state.device, non_blocking=True)
-                ev = torch.cuda.Event()
-                ev.record(cur)
-                op.dev = (state.device, npdt, m, ev, cur.cuda_stream)
+            m = self._block_matrix(op, state, npdt)
             rc = self.lib.qsim_apply_fused(state.data_ptr(), nqubits, code, tg, len(op.targets),
                                            m.data_ptr(), stream)
             _keep_alive(m, state)
         _lib.check(rc, self.lib)
         return state
+
+    @staticmethod
+    def _block_matrix(op: _Op, state: torch.Tensor, npdt) -> torch.Tensor:
+        """The matrix of a fused op in device memory, usable on the current stream."""
+        # it goes to the device once per op (a pinned, stream-ordered copy) and
+        # is reused when the op runs again
+        cached = op.dev
+        cur = torch.cuda.current_stream(state.device)
+        if cached is not None and cached[0] == state.device and cached[1] == npdt:
+            m = cached[2]
+            if cached[4] != cur.cuda_stream:
+                cur.wait_event(cached[3])  # the upload ran on another stream
+        else:
+            host = torch.from_numpy(np.ascontiguousarray(op.data, dtype=npdt)).pin_memory()
+            m = host.to(state.device, non_blocking=True)
+            ev = torch.cuda.Event()
+            ev.record(cur)
+            op.dev = (state.device, npdt, m, ev, cur.cuda_stream)
+        return m
+
+    @staticmethod
+    def _pairable(op: _Op, state: torch.Tensor, nqubits: int) -> bool:
+        """Whether two such ops in a row run as one pass over the state
+        (qsim_apply_fused_pair): uncontrolled blocks of 4 or 5 qubits,
+        complex128, a register of at least the tile's 13 qubits."""
+        return (op.kind == "fused" and not op.controls and len(op.targets) in (4, 5)
+                and state.dtype == torch.complex128 and nqubits >= 13)
+
+    def _apply_pair(self, first: _Op, second: _Op, state: torch.Tensor, nqubits: int):
+        timer = self._timer
+        timed = timer is not None and timer[0](first)
+        cur = torch.cuda.current_stream(state.device)
+        if timed:
+            ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+            ev[0].record(cur)
+        mats = [self._block_matrix(op, state, np.complex128) for op in (first, second)]
+        _lib.check(self.lib.qsim_apply_fused_pair(
+            state.data_ptr(), nqubits, _lib.C128, _lib.int_array(first.targets), len(first.targets), mats[0].data_ptr(),
+            _lib.int_array(second.targets), len(second.targets), mats[1].data_ptr(), self._stream(state)), self.lib)
+        for m in mats:
+            _keep_alive(m, state)
+        if timed:
+            ev[1].record(cur)
+            timer[1].append(ev)
 
     def apply_gate(self, gate, state, nqubits):
         if state.dim() == 2:
@@ -1140,7 +1171,10 @@ class MI355XBackend(GatePlanner):
         for act in actions:
             if act[0] == "single":
                 self._complete(state, nqubits, zero)
-                self.apply_op(act[1], state, nqubits)
+                if len(act) == 3:
+                    self._apply_pair(act[1], act[2], state, nqubits)
+                else:
+                    self.apply_op(act[1], state, nqubits)
                 if len(zero) > 1:
                     zero[1] = None
                 continue
@@ -1307,16 +1341,37 @@ class MI355XBackend(GatePlanner):
         ordered = self.blocking_ordered
         stream = self._stream(state)
         cur = torch.cuda.current_stream(state.device)
+        waiting = None  # a block that the next one may join
+
+        def one_op(*pair):
+            if zero is not None:
+                self._complete(state, nqubits, zero)
+            if len(pair) == 2:
+                self._apply_pair(*pair, state, nqubits)
+            else:
+                self.apply_op(pair[0], state, nqubits)
+            if zero is not None and len(zero) > 1:
+                zero[1] = None
+            if record is not None:
+                record.append(("single",) + pair)
+
         for kind, payload in blocking.partition(ops, nqubits, low, ordered):
             if kind == "single":
-                if zero is not None:
-                    self._complete(state, nqubits, zero)
-                self.apply_op(payload, state, nqubits)
-                if zero is not None and len(zero) > 1:
-                    zero[1] = None
-                if record is not None:
-                    record.append(("single", payload))
+                if self._pairable(payload, state, nqubits):
+                    if waiting is None:
+                        waiting = payload
+                    else:
+                        one_op(waiting, payload)
+                        waiting = None
+                    continue
+                if waiting is not None:
+                    one_op(waiting)
+                    waiting = None
+                one_op(payload)
                 continue
+            if waiting is not None:
+                one_op(waiting)
+                waiting = None
             tile_bits, pops = payload
             if keep:
                 program, count, _ = blocking.compile_pass(tile_bits, pops, nqubits, cdtype, ordered)
@@ -1329,6 +1384,8 @@ class MI355XBackend(GatePlanner):
                                  stream, cur, zero, program)
             if record is not None:
                 record.append(("block", tuple(tile_bits), prog, len(program), count, len(pops), bytes(program)))
+        if waiting is not None:
+            one_op(waiting)
         return state
 
     # -- specialised blocked passes --------------------------------------------

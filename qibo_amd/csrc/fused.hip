@@ -543,9 +543,250 @@ static int launch_fused_tile_c128(void* state, int n, const int* targets, const 
   return QSIM_OK;
 }
 
+// Two blocks of k = 4 or 5 qubits in one pass over the state. One block moves
+// 32 bytes per amplitude for 24 D FP64 operations (D = 32: half of what the
+// matrix cores do in that time), so a pass of two is still bound by HBM: a
+// tile of 8192 amplitudes holds the targets of both (at most 10 bits) and the
+// lowest other bits, and the second product reads the first one's results from
+// LDS. The tile takes 128 KB: with 4096 amplitudes only two low bits are left
+// beside 10 targets, and 64-byte segments cost 2.9 ms per pair at 28 qubits
+// (their loads and stores alone 2.4 to 3.2, with 128 bytes 1.5). The other
+// 32 KB hold Re M and Im M of both matrices; Re M + Im M is formed as read.
+// One workgroup of 16 wavefronts per CU; the next tile is in flight in
+// registers during the products. The arithmetic of each block is that of
+// k_fused_tile_c128, bit for bit.
+// 28 qubits, two 5-qubit blocks: 3.4 ms in two passes, 2.2 to 2.3 ms in this one
+// (its products alone 1.95, its loads and stores alone 1.5), 2.9 against 3.9 on
+// the ten top bits; two 4-qubit blocks 3.3 to 3.6 against 1.6 to 1.8 ms.
+constexpr int kPairBits = 13;
+constexpr int kPairThreads = 1024;
+
+struct PairBlock {
+  uint8_t rowbit[5];           // as Tile128Args
+  uint8_t colbit[kPairBits];
+};
+struct Pair128Args {
+  uint64_t ntiles;
+  uint8_t tbits[kPairBits];
+  PairBlock b[2];
+};
+
+// As swz128, of 13 bits: sixteen columns whose four index bits are distinct
+// modulo 4 land on sixteen distinct 16-byte bank groups.
+__device__ __forceinline__ uint32_t swz_pair(uint32_t u) {
+  return u ^ ((u >> 4) & 15u) ^ ((u >> 8) & 15u) ^ (u >> 12);
+}
+
+// The tile offset of matrix row bits `row` (K of them).
+template <int K>
+__device__ __forceinline__ uint32_t pair_row(const PairBlock& b, uint32_t row) {
+  uint32_t u = 0;
+#pragma clang loop unroll(full)
+  for (int t = 0; t < K; ++t)
+    if ((row >> (K - 1 - t)) & 1) u |= 1u << b.rowbit[t];
+  return u;
+}
+
+template <int K>
+__device__ __forceinline__ void pair_fragments(const c128* __restrict__ mat, double* frag) {
+  constexpr int D = 1 << K, RPL = D / 4, MB = D / 16;
+  for (int e = threadIdx.x; e < 2 * MB * RPL * 64; e += kPairThreads) {
+    const int l = e & 63, f = e >> 6;
+    const int st = f % RPL, mb = (f / RPL) % MB, p = f / (RPL * MB);
+    const c128 m = mat[(16 * mb + (l & 15)) * D + RPL * (l >> 4) + st];
+    frag[e] = p == 0 ? m.re : m.im;
+  }
+}
+
+// One block on the tile in LDS: each wavefront takes groups of 16 columns,
+// which no other one touches.
+template <int K>
+__device__ __forceinline__ void pair_product(const PairBlock& b, const double* frag, c128* tile) {
+  constexpr int D = 1 << K, RPL = D / 4, MB = D / 16;
+  constexpr int NCG = (1 << (kPairBits - K)) / 16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int j = lane & 15, q = lane >> 4;
+  // (the swizzle is linear: offsets of columns, rows per lane and rows per step add by XOR)
+  const uint32_t in = swz_pair(pair_row<K>(b, uint32_t(RPL * q))), out = swz_pair(pair_row<K>(b, uint32_t(q)));
+  for (int cg = wave; cg < NCG; cg += kPairThreads / 64) {
+    uint32_t col = 0;
+#pragma clang loop unroll(full)
+    for (int i = 0; i < kPairBits - K; ++i)
+      if (((16 * cg + j) >> i) & 1) col |= 1u << b.colbit[i];
+    col = swz_pair(col);
+    uint32_t from = in ^ col, to = out ^ col;
+    // (the addresses of the steps are formed at each one: kept over the tiles
+    // they spilled, and a reload waits for the next tile's loads as well)
+    asm volatile("" : "+v"(from), "+v"(to));
+    doublex4 acc[3][MB];
+#pragma clang loop unroll(full)
+    for (int p = 0; p < 3; ++p)
+#pragma clang loop unroll(full)
+      for (int mb = 0; mb < MB; ++mb) acc[p][mb] = doublex4(0.0);
+#pragma clang loop unroll(full)
+    for (int st = 0; st < RPL; ++st) {
+      __builtin_amdgcn_sched_barrier(0);
+      const c128 x = tile[swz_pair(pair_row<K>(b, uint32_t(st))) ^ from];
+      const double b0 = x.re, b1 = x.im, b2 = x.re + x.im;
+#pragma clang loop unroll(full)
+      for (int mb = 0; mb < MB; ++mb) {
+        const double re = frag[(mb * RPL + st) * 64 + lane], im = frag[((MB + mb) * RPL + st) * 64 + lane];
+        acc[0][mb] = __builtin_amdgcn_mfma_f64_16x16x4f64(re, b0, acc[0][mb], 0, 0, 0);
+        acc[1][mb] = __builtin_amdgcn_mfma_f64_16x16x4f64(im, b1, acc[1][mb], 0, 0, 0);
+        acc[2][mb] = __builtin_amdgcn_mfma_f64_16x16x4f64(re + im, b2, acc[2][mb], 0, 0, 0);
+      }
+    }
+#pragma clang loop unroll(full)
+    for (int mb = 0; mb < MB; ++mb)
+#pragma clang loop unroll(full)
+      for (int r = 0; r < 4; ++r) {
+        c128 y;
+        y.re = acc[0][mb][r] - acc[1][mb][r];
+        y.im = (acc[2][mb][r] - acc[0][mb][r]) - acc[1][mb][r];
+        tile[swz_pair(pair_row<K>(b, uint32_t(16 * mb + 4 * r))) ^ to] = y;
+      }
+  }
+}
+
+template <int K1, int K2>
+__global__ __launch_bounds__(kPairThreads) void k_fused_pair_c128(const Pair128Args a, const c128* __restrict__ m1,
+                                                                  const c128* __restrict__ m2, c128* psi) {
+  constexpr int PER = (1 << kPairBits) / kPairThreads, LB = 10;  // log2(kPairThreads)
+  constexpr int F1 = 2 << (2 * K1), F2 = 2 << (2 * K2);          // Re and Im of D x D entries
+  __shared__ c128 tile[1 << kPairBits];
+  __shared__ double frag1[F1], frag2[F2];
+  pair_fragments<K1>(m1, frag1);
+  pair_fragments<K2>(m2, frag2);
+  uint64_t lanebits = 0;
+#pragma clang loop unroll(full)
+  for (int i = 0; i < LB; ++i)
+    if ((threadIdx.x >> i) & 1) lanebits |= uint64_t(1) << a.tbits[i];
+  auto addr = [&](uint64_t glow, int k) {
+#pragma clang loop unroll(full)
+    for (int i = 0; i < kPairBits - LB; ++i)
+      if ((k >> i) & 1) glow |= uint64_t(1) << a.tbits[LB + i];
+    return glow;
+  };
+  const uint32_t slot = swz_pair(threadIdx.x);
+  // the 32 workgroups of an XCD take neighbouring tiles
+  const uint32_t g = gridDim.x;
+  uint64_t t = (g & 7) ? blockIdx.x : (blockIdx.x & 7) * (g >> 3) + (blockIdx.x >> 3);
+  c128 nxt[PER];
+  if (t < a.ntiles) {
+    const uint64_t glow = insert_zeros(t, a.tbits, kPairBits) | lanebits;
+#pragma clang loop unroll(full)
+    for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, addr(glow, k));
+  }
+  while (t < a.ntiles) {
+    // each thread writes (and later reads back) only its own staging slots
+#pragma clang loop unroll(full)
+    for (int k = 0; k < PER; ++k) tile[swz_pair(uint32_t(k) * kPairThreads) ^ slot] = nxt[k];
+    __syncthreads();  // (the first pass through also publishes the fragments)
+    const uint64_t tn = t + g;
+    if (tn < a.ntiles) {
+      const uint64_t gnext = insert_zeros(tn, a.tbits, kPairBits) | lanebits;
+#pragma clang loop unroll(full)
+      for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, addr(gnext, k));
+    }
+    pair_product<K1>(a.b[0], frag1, tile);
+    __syncthreads();
+    pair_product<K2>(a.b[1], frag2, tile);
+    __syncthreads();
+    const uint64_t glow = insert_zeros(t, a.tbits, kPairBits) | lanebits;
+#pragma clang loop unroll(full)
+    for (int k = 0; k < PER; ++k) st_nt(psi, addr(glow, k), tile[swz_pair(uint32_t(k) * kPairThreads) ^ slot]);
+    t = tn;
+  }
+}
+
+// The tile bits of a pair: its targets and the lowest other bits. The columns
+// of a block are numbered so that the first four index bits differ modulo 4
+// where possible (swz_pair).
+static void pair_args(Pair128Args& a, int n, const int* const targets[2], const int nt[2]) {
+  std::memset(&a, 0, sizeof(a));
+  a.ntiles = uint64_t(1) << (n - kPairBits);
+  bool taken[QSIM_MAX_QUBITS] = {false};
+  int nb = 0;
+  for (int k = 0; k < 2; ++k)
+    for (int t = 0; t < nt[k]; ++t) {
+      bool& x = taken[n - 1 - targets[k][t]];
+      nb += !x;
+      x = true;
+    }
+  for (int b = 0; b < n && nb < kPairBits; ++b) {
+    nb += !taken[b];
+    taken[b] = true;
+  }
+  for (int b = 0, i = 0; b < n; ++b)
+    if (taken[b]) a.tbits[i++] = uint8_t(b);
+  for (int k = 0; k < 2; ++k) {
+    bool row[kPairBits] = {false};
+    for (int t = 0; t < nt[k]; ++t)
+      for (int i = 0; i < kPairBits; ++i)
+        if (a.tbits[i] == n - 1 - targets[k][t]) {
+          a.b[k].rowbit[t] = uint8_t(i);
+          row[i] = true;
+        }
+    int nc = 0;
+    for (int r = 0; r < 4; ++r)
+      for (int i = r; i < kPairBits; i += 4)
+        if (!row[i]) {
+          a.b[k].colbit[nc++] = uint8_t(i);
+          row[i] = true;
+          break;
+        }
+    for (int i = 0; i < kPairBits; ++i)
+      if (!row[i]) a.b[k].colbit[nc++] = uint8_t(i);
+  }
+}
+
+template <int K1, int K2>
+static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m2, void* state, hipStream_t s) {
+  static const unsigned resident = [] {
+    int nbk = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nbk, k_fused_pair_c128<K1, K2>, kPairThreads, 0) != hipSuccess ||
+        nbk < 1)
+      nbk = 1;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+      cus = 256;
+    return unsigned(nbk) * unsigned(cus);
+  }();
+  const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
+  hipLaunchKernelGGL((k_fused_pair_c128<K1, K2>), dim3(grid), dim3(kPairThreads), 0, s, a,
+                     reinterpret_cast<const c128*>(m1), reinterpret_cast<const c128*>(m2),
+                     reinterpret_cast<c128*>(state));
+  QSIM_CHECK_LAUNCH();
+  return QSIM_OK;
+}
+
 }  // namespace qsim
 
 using namespace qsim;
+
+extern "C" int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const int* targets1, int ntargets1,
+                                     const void* matrix1_dev, const int* targets2, int ntargets2,
+                                     const void* matrix2_dev, void* stream) {
+  clear_error();
+  QSIM_CHECK_ARG(state != nullptr && matrix1_dev != nullptr && matrix2_dev != nullptr,
+                 "qsim_apply_fused_pair: null pointer");
+  QSIM_CHECK_ARG(dtype == QSIM_C128, "qsim_apply_fused_pair: complex128 states");
+  QSIM_CHECK_ARG((ntargets1 == 4 || ntargets1 == 5) && (ntargets2 == 4 || ntargets2 == 5),
+                 "qsim_apply_fused_pair: blocks of 4 or 5 targets");
+  QSIM_CHECK_ARG(nqubits >= kPairBits, "qsim_apply_fused_pair: at least 13 qubits");
+  if (!validate_qubits(nqubits, targets1, ntargets1, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
+  if (!validate_qubits(nqubits, targets2, ntargets2, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
+  Pair128Args a;
+  const int* const targets[2] = {targets1, targets2};
+  const int nt[2] = {ntargets1, ntargets2};
+  pair_args(a, nqubits, targets, nt);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (ntargets1 == 5)
+    return ntargets2 == 5 ? launch_fused_pair<5, 5>(a, matrix1_dev, matrix2_dev, state, s)
+                          : launch_fused_pair<5, 4>(a, matrix1_dev, matrix2_dev, state, s);
+  return ntargets2 == 5 ? launch_fused_pair<4, 5>(a, matrix1_dev, matrix2_dev, state, s)
+                        : launch_fused_pair<4, 4>(a, matrix1_dev, matrix2_dev, state, s);
+}
 
 extern "C" int qsim_apply_fused(void* state, int nqubits, int dtype, const int* targets, int ntargets,
                                 const void* matrix_dev, void* stream) {
