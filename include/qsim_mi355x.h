@@ -133,8 +133,9 @@ int qsim_apply_fused(void* state, int nqubits, int dtype, const int* targets, in
 
 /* Two uncontrolled blocks of 4 or 5 targets each, the first one first, on a
  * complex128 state of at least 13 qubits in one pass over it: the same
- * arithmetic as two calls of qsim_apply_fused. */
-int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const int* targets1, int ntargets1,
+ * arithmetic as two calls of qsim_apply_fused. `source`: the state that is
+ * read (NULL: `state` itself), apart from `state` otherwise. */
+int qsim_apply_fused_pair(void* state, const void* source, int nqubits, int dtype, const int* targets1, int ntargets1,
                           const void* matrix1_dev, const int* targets2, int ntargets2, const void* matrix2_dev,
                           void* stream);
 
@@ -169,6 +170,13 @@ int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const int* target
 size_t qsim_blocked_header_bytes(void);
 int qsim_apply_blocked(void* state, int nqubits, int dtype, const int* tile_bits, const void* program_dev,
                        size_t program_bytes, int ninstr, void* stream);
+
+/* qsim_apply_blocked that reads another state, `source` (16-byte aligned, not
+ * overlapping `state`), and leaves it as it is: the first pass on an initial
+ * state that the caller keeps (the cast with copy=True of
+ * Backend.execute_circuit), without the copy. */
+int qsim_apply_blocked_from(void* state, const void* source, int nqubits, int dtype, const int* tile_bits,
+                            const void* program_dev, size_t program_bytes, int ninstr, void* stream);
 
 /* qsim_apply_blocked with the input taken to be |0...0>: the buffer's old
  * contents are never read, only the result is written. The first pass of
@@ -233,6 +241,10 @@ int qsim_blocked_specialized_lookup(const void* program, size_t program_bytes, i
 int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, int nqubits, int dtype,
                                    const int* tile_bits, uint64_t support, const void* programs_dev,
                                    size_t program_stride, size_t program_bytes, int ninstr, void* stream);
+/* one state, read from `source` as in qsim_apply_blocked_from */
+int qsim_apply_blocked_specialized_from(uint64_t handle, void* state, const void* source, int nqubits, int dtype,
+                                        const int* tile_bits, const void* program_dev, size_t program_bytes,
+                                        int ninstr, void* stream);
 int qsim_adjoint_blocked_specialized(uint64_t handle, void* psi, void* lam, int nbatch, int nqubits, int dtype,
                                      const int* tile_bits, const void* programs_dev, size_t program_stride,
                                      size_t program_bytes, int ninstr, int nslots, double* partials,

@@ -41,7 +41,7 @@ SIGNATURES = {
     "qsim_apply_diag": (_i, [_vp, _i, _i, _c_int_p, _i, _c_int_p, _i, _vp, _vp]),
     "qsim_apply_swap": (_i, [_vp, _i, _i, _i, _i, _c_int_p, _i, _vp]),
     "qsim_apply_fused": (_i, [_vp, _i, _i, _c_int_p, _i, _vp, _vp]),
-    "qsim_apply_fused_pair": (_i, [_vp, _i, _i, _c_int_p, _i, _vp, _c_int_p, _i, _vp, _vp]),
+    "qsim_apply_fused_pair": (_i, [_vp, _vp, _i, _i, _c_int_p, _i, _vp, _c_int_p, _i, _vp, _vp]),
     "qsim_probabilities_workspace": (_sz, [_i, _i]),
     "qsim_probabilities": (_i, [_vp, _i, _i, _c_int_p, _i, _vp, _vp, _sz, _vp]),
     "qsim_cumsum_workspace": (_sz, [_i64]),
@@ -66,6 +66,8 @@ SIGNATURES = {
     "qsim_inner_matrix": (_i, [_vp, _vp, _i, _i, _c_int_p, _i, _c_int_p, _i, _vp, _vp, _vp, _sz, _vp]),
     "qsim_blocked_header_bytes": (_sz, []),
     "qsim_apply_blocked": (_i, [_vp, _i, _i, _c_int_p, _vp, _sz, _i, _vp]),
+    "qsim_apply_blocked_from": (_i, [_vp, _vp, _i, _i, _c_int_p, _vp, _sz, _i, _vp]),
+    "qsim_apply_blocked_specialized_from": (_i, [ctypes.c_uint64, _vp, _vp, _i, _i, _c_int_p, _vp, _sz, _i, _vp]),
     "qsim_apply_blocked_from_zero": (_i, [_vp, _i, _i, _c_int_p, _vp, _sz, _i, _vp]),
     "qsim_apply_blocked_batched": (_i, [_vp, _i, _i, _i, _c_int_p, _vp, _sz, _sz, _i, _vp]),
     "qsim_blocked_specialize": (_i, [_vp, _sz, _i, _i, _i, _vp]),

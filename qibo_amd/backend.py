@@ -714,7 +714,10 @@ class MI355XBackend(GatePlanner):
         return (op.kind == "fused" and not op.controls and len(op.targets) in (4, 5)
                 and state.dtype == torch.complex128 and nqubits >= 13)
 
-    def _apply_pair(self, first: _Op, second: _Op, state: torch.Tensor, nqubits: int):
+    def _apply_pair(self, first: _Op, second: _Op, state: torch.Tensor, nqubits: int, zero=None):
+        source = zero[3] if zero is not None and len(zero) > 3 else None
+        if source is None and zero is not None:
+            self._complete(state, nqubits, zero)
         timer = self._timer
         timed = timer is not None and timer[0](first)
         cur = torch.cuda.current_stream(state.device)
@@ -723,8 +726,11 @@ class MI355XBackend(GatePlanner):
             ev[0].record(cur)
         mats = [self._block_matrix(op, state, np.complex128) for op in (first, second)]
         _lib.check(self.lib.qsim_apply_fused_pair(
-            state.data_ptr(), nqubits, _lib.C128, _lib.int_array(first.targets), len(first.targets), mats[0].data_ptr(),
+            state.data_ptr(), 0 if source is None else source.data_ptr(), nqubits, _lib.C128,
+            _lib.int_array(first.targets), len(first.targets), mats[0].data_ptr(),
             _lib.int_array(second.targets), len(second.targets), mats[1].data_ptr(), self._stream(state)), self.lib)
+        if source is not None:
+            zero[3] = None
         for m in mats:
             _keep_alive(m, state)
         if timed:
@@ -835,8 +841,12 @@ class MI355XBackend(GatePlanner):
         if isinstance(initial_state, Circuit):
             return self.execute_circuit(initial_state + circuit, None, nshots)
         source = (circuit, initial_state)  # for accuracy reports (re-execution at complex128)
+        kept = None  # an initial state in place: the first pass reads it and writes a new one
         if initial_state is not None:
-            initial_state = self.cast(initial_state, dtype=self.dtype, copy=True)
+            if self._readable(initial_state, circuit):
+                kept, initial_state = initial_state, torch.empty_like(initial_state)
+            else:
+                initial_state = self.cast(initial_state, dtype=self.dtype, copy=True)
             valid = (2**nqubits, 2**nqubits) if dm else (2**nqubits,)
             if tuple(initial_state.shape) != valid:
                 raise_error(
@@ -855,7 +865,7 @@ class MI355XBackend(GatePlanner):
                 )
             return self.execute_circuit_repeated(circuit, nshots, initial_state)
         try:
-            result = self._execute_circuit(circuit, initial_state=initial_state, nshots=nshots)
+            result = self._execute_circuit(circuit, initial_state=initial_state, nshots=nshots, source=kept)
         except self.oom_error:
             raise_error(
                 RuntimeError,
@@ -880,7 +890,17 @@ class MI355XBackend(GatePlanner):
             self._reference = ref
         return ref
 
-    def _execute_circuit(self, circuit, initial_state=None, nshots: int = 1000):
+    def _readable(self, state, circuit) -> bool:
+        """Whether a circuit's first pass can read ``state`` where it is: a plain
+        tensor of this device and dtype that the kernels can address, under a
+        state-vector circuit run once in blocked passes."""
+        return (type(state) is torch.Tensor and not circuit.density_matrix and not circuit.repeated_execution
+                and self.blocking and circuit.nqubits >= blocking.TILE_BITS
+                and state.device == self.torch_device and state.dtype == _torch_dtype(self.dtype)
+                and state.shape == (2**circuit.nqubits,) and state.is_contiguous() and not state.requires_grad
+                and not state.is_conj() and not state.is_neg() and state.data_ptr() % 16 == 0)
+
+    def _execute_circuit(self, circuit, initial_state=None, nshots: int = 1000, source=None):
         from .result import CircuitResult, QuantumState
 
         nqubits = circuit.nqubits
@@ -894,7 +914,7 @@ class MI355XBackend(GatePlanner):
             state = self.run_queue(circuit.queue, state, nqubits, zero_pending=True)
         else:
             state = self.zero_state(nqubits) if initial_state is None else initial_state
-            state = self.run_queue(circuit.queue, state, nqubits)
+            state = self.run_queue(circuit.queue, state, nqubits, source=source)
         if circuit.measurements:
             circuit._final_state = CircuitResult(state, circuit.measurements, backend=self, nshots=nshots)
         else:
@@ -993,7 +1013,7 @@ class MI355XBackend(GatePlanner):
         return state
 
     def run_queue(self, queue, state: torch.Tensor, nqubits: int, zero_pending: bool = False,
-                  sampled: Optional[bool] = None) -> torch.Tensor:
+                  sampled: Optional[bool] = None, source: Optional[torch.Tensor] = None) -> torch.Tensor:
         """Apply the gates of ``queue`` in order (the loop of abstract.py:3321-3322).
 
         With ``self.blocking`` (the default) consecutive gates are grouped into
@@ -1008,6 +1028,8 @@ class MI355XBackend(GatePlanner):
         stand for |0...0>: a first blocked pass produces it itself, anything
         else fills it first. ``sampled``: shots will be drawn from the final
         state (default: the queue holds a measurement); see ``_keeps_samples``.
+        ``source``: the amplitudes to start from (``state`` is not yet written); the
+        first pass reads them there, and they stay as they are.
         """
         keep = self._keeps_samples(state.dtype == torch.complex64, nqubits,
                                    lambda: any(kinds.is_measurement(g) for g in queue) if sampled is None else sampled)
@@ -1017,10 +1039,13 @@ class MI355XBackend(GatePlanner):
         # tiles outside it (all zero) and read only the amplitudes inside it.
         # unwritten: the amplitudes outside the support are not in memory yet
         # (written as zeros before anything else reads the state)
-        zero = [zero_pending, 0 if zero_pending else None, False]
+        # source: the tensor that still holds the state's amplitudes
+        zero = [zero_pending, 0 if zero_pending else None, False, source]
         if zero_pending and (not self.blocking or nqubits < blocking.TILE_BITS):
             self._fill_zero(state, nqubits)
             zero[0] = False
+        if not self.blocking or nqubits < blocking.TILE_BITS:
+            self._complete(state, nqubits, zero)
         if not self.blocking:
             for gate in queue:
                 state = gate.apply(self, state, nqubits)
@@ -1170,10 +1195,10 @@ class MI355XBackend(GatePlanner):
         cur = torch.cuda.current_stream(state.device)
         for act in actions:
             if act[0] == "single":
-                self._complete(state, nqubits, zero)
                 if len(act) == 3:
-                    self._apply_pair(act[1], act[2], state, nqubits)
+                    self._apply_pair(act[1], act[2], state, nqubits, zero)
                 else:
+                    self._complete(state, nqubits, zero)
                     self.apply_op(act[1], state, nqubits)
                 if len(zero) > 1:
                     zero[1] = None
@@ -1307,7 +1332,10 @@ class MI355XBackend(GatePlanner):
     def _complete(self, state: torch.Tensor, nqubits: int, zero):
         """Write every amplitude of a state that passes from |0...0> have left
         partly unwritten (``zero`` as in run_queue), before an operation that
-        may read any of them."""
+        may read any of them, or copies it from where it still is."""
+        if len(zero) > 3 and zero[3] is not None:
+            state.copy_(zero[3])
+            zero[3] = None
         if zero[0]:
             self._fill_zero(state, nqubits)
             zero[0] = False
@@ -1344,11 +1372,11 @@ class MI355XBackend(GatePlanner):
         waiting = None  # a block that the next one may join
 
         def one_op(*pair):
-            if zero is not None:
-                self._complete(state, nqubits, zero)
             if len(pair) == 2:
-                self._apply_pair(*pair, state, nqubits)
+                self._apply_pair(*pair, state, nqubits, zero)
             else:
+                if zero is not None:
+                    self._complete(state, nqubits, zero)
                 self.apply_op(pair[0], state, nqubits)
             if zero is not None and len(zero) > 1:
                 zero[1] = None
@@ -1466,10 +1494,19 @@ class MI355XBackend(GatePlanner):
         # is read only inside the support (the rest may be unwritten)
         partial = not from_zero and support != full
         sparse = partial and (support | tmask) != full
+        source = zero[3] if zero is not None and len(zero) > 3 else None
         variant = _lib.SPEC_PASS_FROM_ZERO if from_zero else _lib.SPEC_PASS
         handle = self._specialized(host, count, code, variant, state.device)
         tba = _lib.int_array(list(tile_bits))
-        if handle:
+        if source is not None:  # (every tile: a state in hand has no known support)
+            args = (state.data_ptr(), source.data_ptr(), nqubits, code, tba, prog.data_ptr(), nbytes, count, stream)
+            if handle:
+                rc = self.lib.qsim_apply_blocked_specialized_from(handle, *args)
+                self.specialized_launches += 1
+            else:
+                rc = self.lib.qsim_apply_blocked_from(*args)
+            zero[3] = None
+        elif handle:
             rc = self.lib.qsim_apply_blocked_specialized(handle, state.data_ptr(), 1, nqubits, code, tba,
                                                          support if partial else _ALL_BITS, prog.data_ptr(), 0,
                                                          nbytes, count, stream)

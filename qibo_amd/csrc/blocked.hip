@@ -351,9 +351,10 @@ void set_tiles(BlkArgs& a, int n, const int* tbits, uint64_t support) {
 template <typename R>
 static int launch_blocked(void* state, int n, const int* tbits, const void* prog, size_t nbytes, int ninstr,
                           int nbatch, size_t prog_stride, hipStream_t s, bool from_zero = false,
-                          uint64_t support = ~uint64_t(0)) {
+                          uint64_t support = ~uint64_t(0), const void* source = nullptr) {
   BlkArgs a;
   std::memset(&a, 0, sizeof(a));
+  if (source) a.source = static_cast<const char*>(source) - static_cast<const char*>(state);
   a.nbytes = nbytes;
   a.state_stride = uint64_t(1) << n;
   a.prog_stride = prog_stride;
@@ -604,6 +605,17 @@ int check_blocked_args(int nqubits, int dtype, const int* tile_bits, const void*
   }
   return QSIM_OK;
 }
+
+int check_blocked_source(const void* state, const void* source, int nqubits, int dtype, const char* what) {
+  QSIM_CHECK_ARG(state != nullptr && source != nullptr, what);
+  QSIM_CHECK_ARG(nqubits >= kBTileBits && nqubits <= QSIM_MAX_QUBITS && (dtype == QSIM_C128 || dtype == QSIM_C64), what);
+  QSIM_CHECK_ARG((reinterpret_cast<uintptr_t>(source) & 15) == 0, what);
+  // the same state, or one that shares no byte with it
+  const uintptr_t s = reinterpret_cast<uintptr_t>(state), f = reinterpret_cast<uintptr_t>(source);
+  const uintptr_t bytes = uintptr_t(dtype == QSIM_C128 ? 16 : 8) << nqubits;
+  QSIM_CHECK_ARG(s == f || s + bytes <= f || f + bytes <= s, what);
+  return QSIM_OK;
+}
 }  // namespace qsim
 
 extern "C" {
@@ -731,6 +743,21 @@ int qsim_apply_blocked(void* state, int nqubits, int dtype, const int* tile_bits
   if (dtype == QSIM_C128)
     return launch_blocked<double>(state, nqubits, tile_bits, program_dev, program_bytes, ninstr, 1, 0, s);
   return launch_blocked<float>(state, nqubits, tile_bits, program_dev, program_bytes, ninstr, 1, 0, s);
+}
+
+int qsim_apply_blocked_from(void* state, const void* source, int nqubits, int dtype, const int* tile_bits,
+                            const void* program_dev, size_t program_bytes, int ninstr, void* stream) {
+  clear_error();
+  if (qsim::check_blocked_source(state, source, nqubits, dtype, "qsim_apply_blocked_from: bad states") != QSIM_OK ||
+      qsim::check_blocked_args(nqubits, dtype, tile_bits, program_dev, program_bytes, ninstr,
+                               "qsim_apply_blocked_from: bad arguments") != QSIM_OK)
+    return QSIM_EINVAL;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (dtype == QSIM_C128)
+    return launch_blocked<double>(state, nqubits, tile_bits, program_dev, program_bytes, ninstr, 1, 0, s, false,
+                                  ~uint64_t(0), source);
+  return launch_blocked<float>(state, nqubits, tile_bits, program_dev, program_bytes, ninstr, 1, 0, s, false,
+                               ~uint64_t(0), source);
 }
 
 }  // extern "C"

@@ -76,6 +76,10 @@ struct BlkArgs {
   // has one of them set is zero and is not read (its memory may hold
   // anything); 0 reads the whole tile.
   uint32_t zload;
+  // Byte distance from the state to the amplitudes that are read (0: the state
+  // itself). The first pass on a state that has to be kept reads it and writes
+  // another: a copy before it took 1.8 ms at 28 qubits, more than the pass.
+  int64_t source;
 };
 
 // Global index of the first amplitude of tile number `tile`.
@@ -381,6 +385,7 @@ __device__ __forceinline__ uint64_t deposit(uint32_t u, const uint64_t* gbit) {
 template <typename R>
 __device__ __forceinline__ void load_lane(const BlkArgs& a, const cplx<R>* psi, uint64_t lane_idx, uint64_t L,
                                           const uint64_t* rb, cplx<R>* v) {
+  psi = reinterpret_cast<const cplx<R>*>(reinterpret_cast<const char*>(psi) + a.source);
   if (a.zload == 0) {
 #pragma clang loop unroll(full)
     for (int r = 0; r < kBReg; ++r) v[r] = ld_nt(psi, lane_idx | reg_index(rb, r));

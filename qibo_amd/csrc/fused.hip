@@ -648,9 +648,10 @@ __device__ __forceinline__ void pair_product(const PairBlock& b, const double* f
   }
 }
 
+// (src may be psi: a tile is read before it is written, by one workgroup)
 template <int K1, int K2>
 __global__ __launch_bounds__(kPairThreads) void k_fused_pair_c128(const Pair128Args a, const c128* __restrict__ m1,
-                                                                  const c128* __restrict__ m2, c128* psi) {
+                                                                  const c128* __restrict__ m2, const c128* src, c128* psi) {
   constexpr int PER = (1 << kPairBits) / kPairThreads, LB = 10;  // log2(kPairThreads)
   constexpr int F1 = 2 << (2 * K1), F2 = 2 << (2 * K2);          // Re and Im of D x D entries
   __shared__ c128 tile[1 << kPairBits];
@@ -675,7 +676,7 @@ __global__ __launch_bounds__(kPairThreads) void k_fused_pair_c128(const Pair128A
   if (t < a.ntiles) {
     const uint64_t glow = insert_zeros(t, a.tbits, kPairBits) | lanebits;
 #pragma clang loop unroll(full)
-    for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, addr(glow, k));
+    for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(src, addr(glow, k));
   }
   while (t < a.ntiles) {
     // each thread writes (and later reads back) only its own staging slots
@@ -686,7 +687,7 @@ __global__ __launch_bounds__(kPairThreads) void k_fused_pair_c128(const Pair128A
     if (tn < a.ntiles) {
       const uint64_t gnext = insert_zeros(tn, a.tbits, kPairBits) | lanebits;
 #pragma clang loop unroll(full)
-      for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, addr(gnext, k));
+      for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(src, addr(gnext, k));
     }
     pair_product<K1>(a.b[0], frag1, tile);
     __syncthreads();
@@ -741,7 +742,8 @@ static void pair_args(Pair128Args& a, int n, const int* const targets[2], const 
 }
 
 template <int K1, int K2>
-static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m2, void* state, hipStream_t s) {
+static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m2, void* state, const void* source,
+                             hipStream_t s) {
   static const unsigned resident = [] {
     int nbk = 0, dev = 0, cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nbk, k_fused_pair_c128<K1, K2>, kPairThreads, 0) != hipSuccess ||
@@ -755,7 +757,7 @@ static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_pair_c128<K1, K2>), dim3(grid), dim3(kPairThreads), 0, s, a,
                      reinterpret_cast<const c128*>(m1), reinterpret_cast<const c128*>(m2),
-                     reinterpret_cast<c128*>(state));
+                     reinterpret_cast<const c128*>(source), reinterpret_cast<c128*>(state));
   QSIM_CHECK_LAUNCH();
   return QSIM_OK;
 }
@@ -764,7 +766,7 @@ static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m
 
 using namespace qsim;
 
-extern "C" int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const int* targets1, int ntargets1,
+extern "C" int qsim_apply_fused_pair(void* state, const void* source, int nqubits, int dtype, const int* targets1, int ntargets1,
                                      const void* matrix1_dev, const int* targets2, int ntargets2,
                                      const void* matrix2_dev, void* stream) {
   clear_error();
@@ -776,16 +778,21 @@ extern "C" int qsim_apply_fused_pair(void* state, int nqubits, int dtype, const 
   QSIM_CHECK_ARG(nqubits >= kPairBits, "qsim_apply_fused_pair: at least 13 qubits");
   if (!validate_qubits(nqubits, targets1, ntargets1, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
   if (!validate_qubits(nqubits, targets2, ntargets2, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
+  if (source == nullptr) source = state;
+  const uintptr_t to = reinterpret_cast<uintptr_t>(state), from = reinterpret_cast<uintptr_t>(source);
+  const uintptr_t bytes = uintptr_t(16) << nqubits;
+  QSIM_CHECK_ARG((from & 15) == 0 && (to == from || to + bytes <= from || from + bytes <= to),
+                 "qsim_apply_fused_pair: bad source");
   Pair128Args a;
   const int* const targets[2] = {targets1, targets2};
   const int nt[2] = {ntargets1, ntargets2};
   pair_args(a, nqubits, targets, nt);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (ntargets1 == 5)
-    return ntargets2 == 5 ? launch_fused_pair<5, 5>(a, matrix1_dev, matrix2_dev, state, s)
-                          : launch_fused_pair<5, 4>(a, matrix1_dev, matrix2_dev, state, s);
-  return ntargets2 == 5 ? launch_fused_pair<4, 5>(a, matrix1_dev, matrix2_dev, state, s)
-                        : launch_fused_pair<4, 4>(a, matrix1_dev, matrix2_dev, state, s);
+    return ntargets2 == 5 ? launch_fused_pair<5, 5>(a, matrix1_dev, matrix2_dev, state, source, s)
+                          : launch_fused_pair<5, 4>(a, matrix1_dev, matrix2_dev, state, source, s);
+  return ntargets2 == 5 ? launch_fused_pair<4, 5>(a, matrix1_dev, matrix2_dev, state, source, s)
+                        : launch_fused_pair<4, 4>(a, matrix1_dev, matrix2_dev, state, source, s);
 }
 
 extern "C" int qsim_apply_fused(void* state, int nqubits, int dtype, const int* targets, int ntargets,

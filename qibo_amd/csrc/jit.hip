@@ -33,6 +33,7 @@ namespace qsim {
 
 int check_blocked_args(int nqubits, int dtype, const int* tile_bits, const void* program_dev, size_t program_bytes,
                        int ninstr, const char* what);
+int check_blocked_source(const void* state, const void* source, int nqubits, int dtype, const char* what);
 void set_tiles(BlkArgs& a, int n, const int* tbits, uint64_t support);
 
 namespace {
@@ -617,10 +618,9 @@ int qsim_blocked_specialized_lookup(const void* program, size_t program_bytes, i
   return QSIM_OK;
 }
 
-int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, int nqubits, int dtype,
-                                   const int* tile_bits, uint64_t support, const void* programs_dev,
-                                   size_t program_stride, size_t program_bytes, int ninstr, void* stream) {
-  clear_error();
+static int apply_specialized(uint64_t handle, void* states, const void* source, int nbatch, int nqubits, int dtype,
+                             const int* tile_bits, uint64_t support, const void* programs_dev, size_t program_stride,
+                             size_t program_bytes, int ninstr, void* stream) {
   QSIM_CHECK_ARG(states != nullptr && nbatch >= 1 && nbatch <= 65535, "qsim_apply_blocked_specialized: bad batch");
   QSIM_CHECK_ARG(program_stride % 16 == 0 && (nbatch == 1 || program_stride >= program_bytes),
                  "qsim_apply_blocked_specialized: bad program stride");
@@ -638,6 +638,8 @@ int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, in
   if (spec_for(handle, dtype, sp.variant, program_bytes, ninstr, sp,
                "qsim_apply_blocked_specialized: kernel for another device, dtype or program") != QSIM_OK)
     return QSIM_EINVAL;
+  QSIM_CHECK_ARG(source == nullptr || sp.variant != kVariantFromZero,
+                 "qsim_apply_blocked_specialized_from: handle of a from-zero pass");
   if (sp.variant == kVariantFromZero) {
     // as qsim_apply_blocked_from_zero: a large state filled with |0...0> and
     // the pass run on tile 0, a small one run on every tile
@@ -651,6 +653,7 @@ int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, in
   }
   BlkArgs a;
   std::memset(&a, 0, sizeof(a));
+  if (source) a.source = static_cast<const char*>(source) - static_cast<const char*>(states);
   a.nbytes = program_bytes;
   a.state_stride = uint64_t(1) << nqubits;
   a.prog_stride = program_stride;
@@ -663,6 +666,24 @@ int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, in
   QSIM_CHECK_HIP(hipModuleLaunchKernel(sp.fn, grid.x, grid.y, unsigned(nbatch), kBT, 1, 1, 0,
                                        reinterpret_cast<hipStream_t>(stream), args, nullptr));
   return QSIM_OK;
+}
+
+int qsim_apply_blocked_specialized(uint64_t handle, void* states, int nbatch, int nqubits, int dtype,
+                                   const int* tile_bits, uint64_t support, const void* programs_dev,
+                                   size_t program_stride, size_t program_bytes, int ninstr, void* stream) {
+  clear_error();
+  return apply_specialized(handle, states, nullptr, nbatch, nqubits, dtype, tile_bits, support, programs_dev,
+                           program_stride, program_bytes, ninstr, stream);
+}
+
+int qsim_apply_blocked_specialized_from(uint64_t handle, void* state, const void* source, int nqubits, int dtype,
+                                        const int* tile_bits, const void* program_dev, size_t program_bytes,
+                                        int ninstr, void* stream) {
+  clear_error();
+  if (check_blocked_source(state, source, nqubits, dtype, "qsim_apply_blocked_specialized_from: bad states") != QSIM_OK)
+    return QSIM_EINVAL;
+  return apply_specialized(handle, state, source, 1, nqubits, dtype, tile_bits, ~uint64_t(0), program_dev, 0,
+                           program_bytes, ninstr, stream);
 }
 
 int qsim_adjoint_blocked_specialized(uint64_t handle, void* psi, void* lam, int nbatch, int nqubits, int dtype,

@@ -34,7 +34,7 @@ def test_pair_is_bitwise_two_blocks(backend, n, first, second):
     stream = torch.cuda.current_stream().cuda_stream
     for m, t in zip(mats, (first, second)):
         _lib.check(lib.qsim_apply_fused(two.data_ptr(), n, _lib.C128, _lib.int_array(t), len(t), m.data_ptr(), stream), lib)
-    _lib.check(lib.qsim_apply_fused_pair(one.data_ptr(), n, _lib.C128, _lib.int_array(first), len(first),
+    _lib.check(lib.qsim_apply_fused_pair(one.data_ptr(), None, n, _lib.C128, _lib.int_array(first), len(first),
                                          mats[0].data_ptr(), _lib.int_array(second), len(second), mats[1].data_ptr(),
                                          stream), lib)
     assert torch.equal(torch.view_as_real(one), torch.view_as_real(two))
@@ -47,8 +47,8 @@ def test_pair_refuses_what_it_does_not_cover(backend):
     m = torch.eye(32, dtype=torch.complex128, device="cuda")
     lib = backend.lib
 
-    def call(n, code, t1, t2):
-        return lib.qsim_apply_fused_pair(psi.data_ptr(), n, code, _lib.int_array(t1), len(t1), m.data_ptr(),
+    def call(n, code, t1, t2, source=None):
+        return lib.qsim_apply_fused_pair(psi.data_ptr(), source, n, code, _lib.int_array(t1), len(t1), m.data_ptr(),
                                          _lib.int_array(t2), len(t2), m.data_ptr(), 0)
 
     five = (0, 1, 2, 3, 4)
@@ -57,6 +57,7 @@ def test_pair_refuses_what_it_does_not_cover(backend):
     assert call(13, _lib.C128, five, (0, 1, 2)) != 0
     assert call(13, _lib.C128, (0, 1, 2, 3, 3), five) != 0
     assert call(13, _lib.C128, five, (0, 1, 2, 3, 13)) != 0
+    assert call(13, _lib.C128, five, five, psi.data_ptr() + 4096) != 0  # overlaps the state
 
 
 @pytest.mark.parametrize("count", [1, 2, 3, 5])
