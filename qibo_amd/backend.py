@@ -1032,7 +1032,7 @@ class MI355XBackend(GatePlanner):
         first pass reads them there, and they stay as they are.
         """
         keep = self._keeps_samples(state.dtype == torch.complex64, nqubits,
-                                   lambda: any(kinds.is_measurement(g) for g in queue) if sampled is None else sampled)
+                                   lambda: any(kinds.is_measurement(g) for g in reversed(queue)) if sampled is None else sampled)
         # [|0...0> still to be materialised, support, unwritten]: the support
         # is the mask of index bits that may be 1 in a nonzero amplitude (None:
         # any); the passes from |0...0> grow it by their tile bits, skip the
