@@ -131,6 +131,12 @@ int qsim_apply_swap(void* state, int nqubits, int dtype, int q0, int q1, const i
 int qsim_apply_fused(void* state, int nqubits, int dtype, const int* targets, int ntargets,
                      const void* matrix_dev, void* stream);
 
+/* qsim_apply_fused for 4 or 5 targets that reads `source` (16-byte aligned,
+ * apart from `state`) and leaves it as it is; registers of at least the
+ * kernels' tile (11 qubits in complex128, 12 in complex64). */
+int qsim_apply_fused_from(void* state, const void* source, int nqubits, int dtype, const int* targets, int ntargets,
+                          const void* matrix_dev, void* stream);
+
 /* Two uncontrolled blocks of 4 or 5 targets each, the first one first, on a
  * complex128 state of at least 13 qubits in one pass over it: the same
  * arithmetic as two calls of qsim_apply_fused. `source`: the state that is

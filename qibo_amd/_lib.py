@@ -41,6 +41,7 @@ SIGNATURES = {
     "qsim_apply_diag": (_i, [_vp, _i, _i, _c_int_p, _i, _c_int_p, _i, _vp, _vp]),
     "qsim_apply_swap": (_i, [_vp, _i, _i, _i, _i, _c_int_p, _i, _vp]),
     "qsim_apply_fused": (_i, [_vp, _i, _i, _c_int_p, _i, _vp, _vp]),
+    "qsim_apply_fused_from": (_i, [_vp, _vp, _i, _i, _c_int_p, _i, _vp, _vp]),
     "qsim_apply_fused_pair": (_i, [_vp, _vp, _i, _i, _c_int_p, _i, _vp, _c_int_p, _i, _vp, _vp]),
     "qsim_probabilities_workspace": (_sz, [_i, _i]),
     "qsim_probabilities": (_i, [_vp, _i, _i, _c_int_p, _i, _vp, _vp, _sz, _vp]),

@@ -706,13 +706,21 @@ class MI355XBackend(GatePlanner):
             op.dev = (state.device, npdt, m, ev, cur.cuda_stream)
         return m
 
-    @staticmethod
-    def _pairable(op: _Op, state: torch.Tensor, nqubits: int) -> bool:
-        """Whether two such ops in a row run as one pass over the state
-        (qsim_apply_fused_pair): uncontrolled blocks of 4 or 5 qubits,
-        complex128, a register of at least the tile's 13 qubits."""
-        return (op.kind == "fused" and not op.controls and len(op.targets) in (4, 5)
-                and state.dtype == torch.complex128 and nqubits >= 13)
+    def _apply_single(self, op: _Op, state: torch.Tensor, nqubits: int, zero):
+        """One op between passes; a dense block reads a state still elsewhere in place."""
+        if zero is not None:
+            if (len(zero) > 3 and zero[3] is not None and op.kind == "fused" and not op.controls
+                    and len(op.targets) in (4, 5) and nqubits >= blocking.TILE_BITS and self._timer is None):
+                code = self._dtype_code(state)
+                m = self._block_matrix(op, state, np.complex128 if code == _lib.C128 else np.complex64)
+                _lib.check(self.lib.qsim_apply_fused_from(
+                    state.data_ptr(), zero[3].data_ptr(), nqubits, code, _lib.int_array(op.targets), len(op.targets),
+                    m.data_ptr(), self._stream(state)), self.lib)
+                _keep_alive(m, state)
+                zero[3] = None
+                return
+            self._complete(state, nqubits, zero)
+        self.apply_op(op, state, nqubits)
 
     def _apply_pair(self, first: _Op, second: _Op, state: torch.Tensor, nqubits: int, zero=None):
         source = zero[3] if zero is not None and len(zero) > 3 else None
@@ -896,7 +904,7 @@ class MI355XBackend(GatePlanner):
         state-vector circuit run once in blocked passes."""
         return (type(state) is torch.Tensor and not circuit.density_matrix and not circuit.repeated_execution
                 and self.blocking and circuit.nqubits >= blocking.TILE_BITS
-                and state.device == self.torch_device and state.dtype == _torch_dtype(self.dtype)
+                and state.dtype == _torch_dtype(self.dtype) and state.device == self.torch_device
                 and state.shape == (2**circuit.nqubits,) and state.is_contiguous() and not state.requires_grad
                 and not state.is_conj() and not state.is_neg() and state.data_ptr() % 16 == 0)
 
@@ -1198,8 +1206,7 @@ class MI355XBackend(GatePlanner):
                 if len(act) == 3:
                     self._apply_pair(act[1], act[2], state, nqubits, zero)
                 else:
-                    self._complete(state, nqubits, zero)
-                    self.apply_op(act[1], state, nqubits)
+                    self._apply_single(act[1], state, nqubits, zero)
                 if len(zero) > 1:
                     zero[1] = None
                 continue
@@ -1369,15 +1376,17 @@ class MI355XBackend(GatePlanner):
         ordered = self.blocking_ordered
         stream = self._stream(state)
         cur = torch.cuda.current_stream(state.device)
+        # uncontrolled blocks of 4 or 5 qubits in a row run two to a pass
+        # (qsim_apply_fused_pair: complex128, registers of at least its tile's 13
+        # qubits): 28 qubits 1.7 ms alone, 2.2 (k = 5) and 1.6 ms (k = 4) for two
+        pairs = code == _lib.C128 and nqubits >= 13
         waiting = None  # a block that the next one may join
 
         def one_op(*pair):
             if len(pair) == 2:
                 self._apply_pair(*pair, state, nqubits, zero)
             else:
-                if zero is not None:
-                    self._complete(state, nqubits, zero)
-                self.apply_op(pair[0], state, nqubits)
+                self._apply_single(pair[0], state, nqubits, zero)
             if zero is not None and len(zero) > 1:
                 zero[1] = None
             if record is not None:
@@ -1385,7 +1394,7 @@ class MI355XBackend(GatePlanner):
 
         for kind, payload in blocking.partition(ops, nqubits, low, ordered):
             if kind == "single":
-                if self._pairable(payload, state, nqubits):
+                if pairs and payload.kind == "fused" and not payload.controls and len(payload.targets) in (4, 5):
                     if waiting is None:
                         waiting = payload
                     else:

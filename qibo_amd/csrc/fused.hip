@@ -158,7 +158,7 @@ __device__ __forceinline__ void st_pair(c64* psi, uint64_t i, floatx4 v) {
 // latency is hidden inside each workgroup (tiles t = blockIdx.x + i gridDim.x).
 template <int K>
 __global__ __launch_bounds__(256) void k_fused_mfma_c64(const MfmaArgs a, const c64* __restrict__ mat,
-                                                       c64* __restrict__ psi) {
+                                                       const c64* src, c64* psi) {
   constexpr int D = 1 << K;             // complex rows
   constexpr int MB = (2 * D) / 32;      // 32-row blocks of the real embedding (1 or 2)
   constexpr int KS = (2 * D) / 2;       // K = 2 steps over the 2D real inner dimension
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void k_fused_mfma_c64(const MfmaArgs a, const 
   if (t < a.ntiles) {
     const uint64_t glow = insert_zeros(t, a.tbits, kMfmaTileBits) | lanebits;
 #pragma clang loop unroll(full)
-    for (int k = 0; k < 8; ++k) nxt[k] = ld_pair(psi, mfma_addr(a, glow, k));
+    for (int k = 0; k < 8; ++k) nxt[k] = ld_pair(src, mfma_addr(a, glow, k));
   }
   while (t < a.ntiles) {
     const uint64_t glow = insert_zeros(t, a.tbits, kMfmaTileBits) | lanebits;
@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_fused_mfma_c64(const MfmaArgs a, const 
     if (tn < a.ntiles) {  // next tile's loads overlap this tile's product
       const uint64_t gnext = insert_zeros(tn, a.tbits, kMfmaTileBits) | lanebits;
 #pragma clang loop unroll(full)
-      for (int k = 0; k < 8; ++k) nxt[k] = ld_pair(psi, mfma_addr(a, gnext, k));
+      for (int k = 0; k < 8; ++k) nxt[k] = ld_pair(src, mfma_addr(a, gnext, k));
     }
     // one 32-column group per wave at a time; the groups are disjoint, so each
     // wave reads and writes only its own columns of the tile
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(256) void k_fused_mfma_c64(const MfmaArgs a, const 
 }
 
 template <int K>
-static int launch_fused_mfma(void* state, int n, const int* targets, const void* mat, hipStream_t s) {
+static int launch_fused_mfma(void* state, const void* source, int n, const int* targets, const void* mat, hipStream_t s) {
   MfmaArgs a;
   std::memset(&a, 0, sizeof(a));
   a.ntiles = uint64_t(1) << (n - kMfmaTileBits);
@@ -330,7 +330,7 @@ static int launch_fused_mfma(void* state, int n, const int* targets, const void*
   const uint64_t resident = uint64_t(cus) * uint64_t(per_cu[K - 4]);
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_mfma_c64<K>), dim3(grid), dim3(256), 0, s, a, reinterpret_cast<const c64*>(mat),
-                     reinterpret_cast<c64*>(state));
+                     reinterpret_cast<const c64*>(source), reinterpret_cast<c64*>(state));
   QSIM_CHECK_LAUNCH();
   return QSIM_OK;
 }
@@ -404,7 +404,7 @@ __device__ __forceinline__ uint64_t tile128_addr(const Tile128Args& a, uint64_t 
 
 template <int K>
 __global__ __launch_bounds__(256) void k_fused_tile_c128(const Tile128Args a, const c128* __restrict__ mat,
-                                                        c128* __restrict__ psi) {
+                                                        const c128* src, c128* psi) {
   constexpr int D = 1 << K;          // complex rows
   constexpr int RPL = D / 4;         // rows per lane = K-steps per product
   constexpr int MB = D / 16;         // 16-row output blocks per product
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256) void k_fused_tile_c128(const Tile128Args a, co
   if (t < a.ntiles) {
     const uint64_t glow = insert_zeros(t, a.tbits, kT128Bits) | lanebits;
 #pragma clang loop unroll(full)
-    for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, tile128_addr(a, glow, k));
+    for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(src, tile128_addr(a, glow, k));
   }
   while (t < a.ntiles) {
     const uint64_t glow = insert_zeros(t, a.tbits, kT128Bits) | lanebits;
@@ -450,7 +450,7 @@ __global__ __launch_bounds__(256) void k_fused_tile_c128(const Tile128Args a, co
     if (tn < a.ntiles) {  // the next tile's loads overlap this tile's products
       const uint64_t gnext = insert_zeros(tn, a.tbits, kT128Bits) | lanebits;
 #pragma clang loop unroll(full)
-      for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(psi, tile128_addr(a, gnext, k));
+      for (int k = 0; k < PER; ++k) nxt[k] = ld_nt(src, tile128_addr(a, gnext, k));
     }
     // one 16-column group per wave at a time; the groups are disjoint, so each
     // wave reads and writes only its own columns of the tile
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256) void k_fused_tile_c128(const Tile128Args a, co
 }
 
 template <int K>
-static int launch_fused_tile_c128(void* state, int n, const int* targets, const void* mat, hipStream_t s) {
+static int launch_fused_tile_c128(void* state, const void* source, int n, const int* targets, const void* mat, hipStream_t s) {
   Tile128Args a;
   std::memset(&a, 0, sizeof(a));
   a.ntiles = uint64_t(1) << (n - kT128Bits);
@@ -538,7 +538,7 @@ static int launch_fused_tile_c128(void* state, int n, const int* targets, const 
   }();
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_tile_c128<K>), dim3(grid), dim3(256), 0, s, a, reinterpret_cast<const c128*>(mat),
-                     reinterpret_cast<c128*>(state));
+                     reinterpret_cast<const c128*>(source), reinterpret_cast<c128*>(state));
   QSIM_CHECK_LAUNCH();
   return QSIM_OK;
 }
@@ -766,6 +766,30 @@ static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m
 
 using namespace qsim;
 
+// A source to read instead of the state: aligned, the state itself or clear of it.
+static bool apart(const void* state, const void* source, uintptr_t bytes) {
+  const uintptr_t to = reinterpret_cast<uintptr_t>(state), from = reinterpret_cast<uintptr_t>(source);
+  return (from & 15) == 0 && (to == from || to + bytes <= from || from + bytes <= to);
+}
+
+extern "C" int qsim_apply_fused_from(void* state, const void* source, int nqubits, int dtype, const int* targets,
+                                     int ntargets, const void* matrix_dev, void* stream) {
+  clear_error();
+  QSIM_CHECK_ARG(state != nullptr && source != nullptr && matrix_dev != nullptr, "qsim_apply_fused_from: null pointer");
+  QSIM_CHECK_ARG(dtype == QSIM_C128 || dtype == QSIM_C64, "qsim_apply_fused_from: bad dtype");
+  QSIM_CHECK_ARG(ntargets == 4 || ntargets == 5, "qsim_apply_fused_from: blocks of 4 or 5 targets");
+  if (!validate_qubits(nqubits, targets, ntargets, nullptr, 0, "qsim_apply_fused_from")) return QSIM_EINVAL;
+  QSIM_CHECK_ARG(nqubits >= (dtype == QSIM_C128 ? kT128Bits : kMfmaTileBits), "qsim_apply_fused_from: register below a tile");
+  QSIM_CHECK_ARG(apart(state, source, uintptr_t(dtype == QSIM_C128 ? 16 : 8) << nqubits),
+                 "qsim_apply_fused_from: bad source");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (dtype == QSIM_C128)
+    return ntargets == 5 ? launch_fused_tile_c128<5>(state, source, nqubits, targets, matrix_dev, s)
+                         : launch_fused_tile_c128<4>(state, source, nqubits, targets, matrix_dev, s);
+  return ntargets == 5 ? launch_fused_mfma<5>(state, source, nqubits, targets, matrix_dev, s)
+                       : launch_fused_mfma<4>(state, source, nqubits, targets, matrix_dev, s);
+}
+
 extern "C" int qsim_apply_fused_pair(void* state, const void* source, int nqubits, int dtype, const int* targets1, int ntargets1,
                                      const void* matrix1_dev, const int* targets2, int ntargets2,
                                      const void* matrix2_dev, void* stream) {
@@ -779,10 +803,7 @@ extern "C" int qsim_apply_fused_pair(void* state, const void* source, int nqubit
   if (!validate_qubits(nqubits, targets1, ntargets1, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
   if (!validate_qubits(nqubits, targets2, ntargets2, nullptr, 0, "qsim_apply_fused_pair")) return QSIM_EINVAL;
   if (source == nullptr) source = state;
-  const uintptr_t to = reinterpret_cast<uintptr_t>(state), from = reinterpret_cast<uintptr_t>(source);
-  const uintptr_t bytes = uintptr_t(16) << nqubits;
-  QSIM_CHECK_ARG((from & 15) == 0 && (to == from || to + bytes <= from || from + bytes <= to),
-                 "qsim_apply_fused_pair: bad source");
+  QSIM_CHECK_ARG(apart(state, source, uintptr_t(16) << nqubits), "qsim_apply_fused_pair: bad source");
   Pair128Args a;
   const int* const targets[2] = {targets1, targets2};
   const int nt[2] = {ntargets1, ntargets2};
@@ -805,11 +826,11 @@ extern "C" int qsim_apply_fused(void* state, int nqubits, int dtype, const int* 
   QSIM_CHECK_ARG(nqubits >= ntargets, "qsim_apply_fused: more targets than qubits");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (dtype == QSIM_C128) {
-    if (nqubits >= kT128Bits && ntargets == 5) return launch_fused_tile_c128<5>(state, nqubits, targets, matrix_dev, s);
-    if (nqubits >= kT128Bits && ntargets == 4) return launch_fused_tile_c128<4>(state, nqubits, targets, matrix_dev, s);
+    if (nqubits >= kT128Bits && ntargets == 5) return launch_fused_tile_c128<5>(state, state, nqubits, targets, matrix_dev, s);
+    if (nqubits >= kT128Bits && ntargets == 4) return launch_fused_tile_c128<4>(state, state, nqubits, targets, matrix_dev, s);
     return dispatch_fused<double>(state, nqubits, targets, ntargets, matrix_dev, s);
   }
-  if (nqubits >= kMfmaTileBits && ntargets == 5) return launch_fused_mfma<5>(state, nqubits, targets, matrix_dev, s);
-  if (nqubits >= kMfmaTileBits && ntargets == 4) return launch_fused_mfma<4>(state, nqubits, targets, matrix_dev, s);
+  if (nqubits >= kMfmaTileBits && ntargets == 5) return launch_fused_mfma<5>(state, state, nqubits, targets, matrix_dev, s);
+  if (nqubits >= kMfmaTileBits && ntargets == 4) return launch_fused_mfma<4>(state, state, nqubits, targets, matrix_dev, s);
   return dispatch_fused<float>(state, nqubits, targets, ntargets, matrix_dev, s);
 }
