@@ -171,7 +171,10 @@ class Compiler {
 };
 
 // Remembers a record that multiplies the whole state, or a table of some
-// registers, as a place for the cosines.
+// registers, as a place for the cosines. (Not LANE_PHASE: it multiplies the
+// lane's pending factor, which would gather the cosines of several runs of
+// rotations while the state already holds their secants: complex64 RX(pi)
+// four times beside RZ ended as inf * 0.)
 void Compiler::note(uint8_t op, int arg, uint64_t cmask, uint64_t tmask, int rreq, const C* data, int ndata) {
   if (cmask || tmask || rreq || !data) return;
   Event e;
@@ -180,8 +183,7 @@ void Compiler::note(uint8_t op, int arg, uint64_t cmask, uint64_t tmask, int rre
   if (op == kRRegPhase && arg != 0) {
     e.kind = 2;
     e.dep = arg;
-  } else if (op == kRDense1 || op == kRDense1Real || op == kRRegPhase || op == kRLanePhase || op == kRDiag ||
-             op == kRDense2) {
+  } else if (op == kRDense1 || op == kRDense1Real || op == kRRegPhase || op == kRDiag || op == kRDense2) {
     e.kind = 1;
   } else {
     return;

@@ -1,5 +1,8 @@
 """A numpy interpreter of the records of blocking.compile_program (layouts,
-scaled rotations, two-qubit gates in registers), for the tests on the CPU."""
+scaled rotations, two-qubit gates in registers), for the tests on the CPU.
+Factors are held as the kernels hold them: a LANE_PHASE multiplies the lane's
+pending factor, which reaches the amplitudes at the next change of layout,
+DENSE_LDS or store, so a range that the kernels leave is left here too."""
 
 import numpy as np
 
@@ -53,6 +56,7 @@ def run_program(state, n, tile_bits, program, count, low):
     gidx = index(lay)
     v = state[gidx].copy()
     pend = np.ones_like(v)
+    lane = np.ones_like(v)  # the pending factor of LANE_PHASE records: the same on all registers of a lane
     qbit = None
     for op, arg, nt, rreq, raw, mat in recs[1:]:
         cmask = int.from_bytes(raw[:8], "little")
@@ -68,6 +72,7 @@ def run_program(state, n, tile_bits, program, count, low):
                 names = _nibbles(cmask)
                 continue
             assert arg == blocking.MAP_LAYOUT
+            v, lane = v * lane, np.ones_like(v)
             frm, to = _nibbles(int.from_bytes(raw[8:16], "little")), _nibbles(cmask)
             full = np.empty_like(v)
 
@@ -82,6 +87,7 @@ def run_program(state, n, tile_bits, program, count, low):
             continue
         if op == blocking.OP_DENSE_LDS:
             k = arg
+            v, lane = v * lane, np.ones_like(v)
             tb = [tile_bits[b] for b in bits[:k]]
             assert sorted(bits[:k]) == bits[4: 4 + k]
             full = state.copy()
@@ -158,7 +164,11 @@ def run_program(state, n, tile_bits, program, count, low):
                 else:
                     assert tb not in [tile_bits[names[8 + j]] for j in range(4)]
                     di = (di << 1) | ((gidx >> tb) & 1)
-            v = np.where(cond, v * mat[di], v)
+            if op == blocking.OP_LANE_PHASE:
+                assert rreq == 0
+                lane = np.where(cond, lane * mat[di], lane)
+            else:
+                v = np.where(cond, v * mat[di], v)
         elif op == blocking.OP_LANE_REGPHASE:
             assert rreq == 0 and qbit in (None, arg)
             qbit = arg
@@ -177,6 +187,7 @@ def run_program(state, n, tile_bits, program, count, low):
         else:
             raise AssertionError(f"record {op}")
     assert qbit is None
+    v = v * lane
     assert not set(names[8:]) & set(range(low)), "a low bit is stored from a register"
     out = state.copy()
     out[index(names)] = v

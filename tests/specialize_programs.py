@@ -49,6 +49,23 @@ def mixed_circuit(n, rng, depth=6):
     return c
 
 
+# (angle, repeats) of steep_circuit: cosines of 6e-17 to 0.32, often enough that their product leaves a type's range
+STEEP = [(np.pi, 4), (np.pi, 24), (3.14, 13), (3.0, 35), (2.5, 80)]
+
+
+def steep_circuit(n, angle, repeats, pad=0, **kwargs):
+    """Pulses by ``angle`` with phases on other qubits between them, as
+    decoupling sequences on idle qubits have them (on the last n of n + pad)."""
+    c = Circuit(n + pad, **kwargs)
+    for _ in range(repeats):
+        c.add(gates.RX(pad, angle))
+        c.add(gates.RZ(pad + (4 if n > 4 else n - 1), 0.3))
+        for k in range(1, n - 6):
+            c.add(gates.RY(pad + k, angle))
+            c.add(gates.RZ(pad + k + 6, 0.2))
+    return c
+
+
 def programs(n, cdtype, seed=0, depth=6, ordered=False):
     """(tile_bits, program bytes, record count) of every blocked pass of the
     mixed circuit."""

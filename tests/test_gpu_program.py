@@ -15,7 +15,7 @@ from qibo_amd import Circuit, _lib, blocking, gates, models
 from qibo_amd.backend import GatePlanner, MI355XBackend
 
 from tests.program_records import records, run_program
-from tests.specialize_programs import mixed_circuit
+from tests.specialize_programs import STEEP, mixed_circuit, steep_circuit
 from tests.test_program import _phases, _random_state, _two_qubit
 
 pytestmark = pytest.mark.gpu
@@ -78,6 +78,26 @@ def test_circuits_match_the_oracle(n, dtype, tol, specialize, rng):
             got = be.execute_circuit(c).state().cpu().numpy()
             assert np.max(np.abs(got - want)) < tol
             be.wait_specializations()
+
+
+@pytest.mark.parametrize("specialize", [False, True])
+@pytest.mark.parametrize("dtype,tol", [("complex128", 1e-12), ("complex64", 2e-5)])
+@pytest.mark.parametrize("n", [5, 12, 16])
+def test_steep_rotations_beside_lane_phases(n, dtype, tol, specialize):
+    """Pulses and phases whose cosines must not gather in the lanes' pending
+    factor, as state vectors and (up to 6 qubits) density matrices."""
+    be = MI355XBackend(dtype=dtype)
+    be.specialize, be.specialize_after = specialize, 1
+    for angle, repeats in STEEP:
+        want = OracleBackend().execute(steep_circuit(n, angle, min(repeats, 30)))
+        c = steep_circuit(n, angle, min(repeats, 30))
+        for _ in range(2):
+            got = be.execute_circuit(c).state().cpu().numpy()
+            assert np.max(np.abs(got - want)) < tol
+            be.wait_specializations()
+        if n <= 6 and not specialize:
+            got = be.execute_circuit(steep_circuit(n, angle, min(repeats, 30), density_matrix=True)).state().cpu().numpy()
+            assert np.max(np.abs(got - np.outer(want, want.conj()))) < 2 * tol
 
 
 @pytest.mark.parametrize("specialize", [False, True])

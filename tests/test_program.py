@@ -17,7 +17,7 @@ from qibo_amd import Circuit, blocking, gates, models
 from qibo_amd.backend import GatePlanner, _dm_pair, plan_matrix
 
 from tests.program_records import PAIRS, records, run_program
-from tests.specialize_programs import mixed_circuit
+from tests.specialize_programs import STEEP, mixed_circuit, steep_circuit
 
 
 def _compiled(ops, n, cdt, low):
@@ -157,6 +157,28 @@ def test_steep_rotations(cdt, tol, rng):
         got, _ = _run(circuit, n, cdt, psi)
         assert np.all(np.isfinite(got))
         assert np.max(np.abs(got - _oracle(circuit, n, psi))) < tol
+
+
+@pytest.mark.parametrize("cdt,tol", [(np.complex128, 1e-13), (np.complex64, 2e-5)])
+@pytest.mark.parametrize("angle,repeats", STEEP)
+@pytest.mark.parametrize("n", [2, 5, 8, 12, 13, 16])
+def test_steep_rotations_beside_lane_phases(n, angle, repeats, cdt, tol, rng):
+    """Pulses on one qubit with phases on another between them: the phases wait
+    in the lane's factor while the rotations run, so no cosine may wait there
+    with them. From |0...0> and from a dense state; registers below a tile run
+    as the low end of one."""
+    if n > 13 and repeats > 30:
+        repeats = 30  # (the interpreter's time)
+    pad = max(0, 12 - n)
+    circuit = steep_circuit(n, angle, repeats, pad)
+    first = np.zeros(2 ** (n + pad), dtype=cdt)
+    first[0] = 1
+    second = np.zeros_like(first)
+    second[: 2**n] = _random_state(n, rng, cdt)
+    for psi in (first, second):
+        got, _ = _run(circuit, n + pad, cdt, psi)
+        assert np.all(np.isfinite(got))
+        assert np.max(np.abs(got - _oracle(circuit, n + pad, psi))) < tol
 
 
 @pytest.mark.parametrize("nrot", [1, 4, 5])
