@@ -677,60 +677,82 @@ void Compiler::emit_lds(const Op& o) {
   w_.emit(kRDenseLds, k, cm, 0, bits, 8, mat, (1 << k) * (1 << k));
 }
 
-// Rotations become ROTS records: each cosine goes to the last record before
-// it that multiplies the whole state (or to the first one). complex64 keeps
-// such runs short, so that the state stays in range: after 8 rotations the
-// next table is made one of all registers.
+// Rotations become ROTS records (and the sign of the pass goes to the first
+// record that can take it): each cosine goes to the last record before it
+// that multiplies the whole state (rotations before the first such record:
+// to that one). At most kRunDouble or kRunSingle of them share a record, so
+// that the state stays in range between its cosines and its secants; a longer
+// run goes on with the next table of some registers, made one of all, or with
+// a table of its own where that pays (64 operations against 16 saved per
+// rotation). Structure alone decides this, so that a kernel specialised to the
+// records serves other angles too: over uniform angles the product of a full
+// run's cosines is below the floor once in 10^7 runs or less (the Chernoff
+// bound over E |cos|^-0.69 is 9e-8 in complex64, 1e-34 in complex128). Several
+// angles near pi in one run pass it: those rotations stay three shears.
+constexpr int kRunDouble = 128, kRunSingle = 16, kTablePays = 5;
+
 void Compiler::fold_cosines() {
   const bool single = w_.itemsize == 8;
   const double floor = single ? 0x1p-64 : 0x1p-400;
-  const int longest = single ? 8 : 1 << 30;
-  int nrot = 0;
+  const int longest = single ? kRunSingle : kRunDouble;
+  const size_t n = events_.size();
+  // rotations from each event to the next record that takes cosines or could
+  std::vector<int> ahead(n + 1, 0);
+  int lead = 0, nrot = 0;  // rotations before the first such record, in all
   bool any = false;
+  for (size_t i = n; i-- > 0;) ahead[i] = events_[i].kind == 0 ? ahead[i + 1] + 1 : 0;
   for (const Event& e : events_) {
     nrot += e.kind == 0;
     any = any || e.kind == 1;
+    lead += e.kind == 0 && !any;
   }
-  if (nrot == 0) return;
-  if (!any && nrot >= 5) {  // a table of its own: 64 operations against 16 saved per rotation
-    C one[16];
-    for (int r = 0; r < 16; ++r) one[r] = {1.0, 0.0};
-    emit(kRRegPhase, 0, 0, 0, nullptr, 0, one, 16);
-    any = true;
+  if (!any && nrot < kTablePays) {
+    if (sign_) w_.emit(kRNeg, 0, 0, 0, nullptr, 0, nullptr, 0);
+    return;
   }
-  if (!any) return;
-  size_t target = 0;  // the record that takes the next cosines
-  while (events_[target].kind != 1) ++target;
-  const size_t first = target;
-  // 1 / sqrt(1 + t^2) of the rounded tangent, multiplied in extended precision:
-  // the rotations keep the norm, whatever their number (products of rounded
-  // cosines put a 23-qubit circuit of 400 gates 4e-15 off it)
-  std::vector<long double> factor(events_.size(), 1.0L);
-  bool before = true;  // rotations before the first such record go to it
+  struct Target {
+    long off;  // of the added table; -1: the entries of `event`
+    size_t event;
+    long double factor = 1.0L;
+  };
+  std::vector<Target> targets;
   int run = 0;
-  for (size_t i = 0; i < events_.size(); ++i) {
+  if (any && lead <= longest) {
+    size_t first = 0;
+    while (events_[first].kind != 1) ++first;
+    targets.push_back({-1, first});
+  } else {
+    size_t first = 0;
+    while (events_[first].kind != 0) ++first;
+    targets.push_back({events_[first].off, 0});
+    lead = 0;
+  }
+  for (size_t i = 0; i < n; ++i) {
     Event& e = events_[i];
+    if (e.kind == 2 && run + ahead[i + 1] > longest) {
+      e.kind = 1;
+      w_.out[e.off - kHeader + 1] = 0;  // a table of all registers
+    }
     if (e.kind == 1) {
-      if (!(before && i == first)) run = 0;
-      before = before && i != first;
-      target = i;
-      continue;
+      if (targets.back().off < 0 && targets.back().event == i) continue;  // the lead's: its run goes on
+      targets.push_back({-1, i});
+      run = 0;
     }
-    if (e.kind == 2) {
-      if (!before && run >= longest) {
-        e.kind = 1;
-        const uint8_t all = 0;
-        std::memcpy(w_.out + e.off - kHeader + 1, &all, 1);
-        target = i;
-        run = 0;
-      }
-      continue;
+    if (e.kind != 0) continue;
+    if (run == longest) {
+      if (ahead[i] < kTablePays) continue;
+      targets.push_back({e.off, 0});
+      run = 0;
     }
+    ++run;
+    // 1 / sqrt(1 + t^2) of the rounded tangent, multiplied in extended precision:
+    // the rotations keep the norm, whatever their number (products of rounded
+    // cosines put a 23-qubit circuit of 400 gates 4e-15 off it)
     const double tan = single ? double(float(e.tan)) : e.tan;
     const long double cosine = 1.0L / std::sqrt(1.0L + (long double)(tan) * tan);
-    if (!(e.c > 0) || factor[target] * cosine < floor) continue;  // stays three shears
-    factor[target] *= cosine;
-    ++run;
+    long double& factor = targets.back().factor;
+    if (!(e.c > 0) || factor * cosine < floor) continue;  // stays three shears
+    factor *= cosine;
     uint8_t* h = w_.out + e.off;
     h[0] = kRRotS;
     std::memset(h + 8, 0, 16);
@@ -741,11 +763,22 @@ void Compiler::fold_cosines() {
       std::memcpy(h + 8, &e.tan, 8);
     }
   }
-  for (size_t i = 0; i < events_.size(); ++i) {
-    Event& e = events_[i];
-    if (e.kind != 1 || factor[i] == 1.0L) continue;
-    for (C& x : e.entries) x.re = double(x.re * factor[i]), x.im = double(x.im * factor[i]);
-    w_.rewrite(e.off, e.entries.data(), int(e.entries.size()));
+  if (sign_) targets[0].factor = -targets[0].factor;
+  for (size_t k = targets.size(); k-- > 0;) {  // from the end: added tables move what follows them
+    const Target& t = targets[k];
+    if (t.off < 0) {
+      if (t.factor == 1.0L) continue;
+      Event& e = events_[t.event];
+      for (C& x : e.entries) x.re = double(x.re * t.factor), x.im = double(x.im * t.factor);
+      w_.rewrite(e.off, e.entries.data(), int(e.entries.size()));
+      continue;
+    }
+    C table[16];
+    for (C& x : table) x = {double(t.factor), 0.0};
+    const size_t tail = w_.len;
+    w_.emit(kRRegPhase, 0, 0, 0, nullptr, 0, table, 16);
+    if (w_.overflow) return;
+    std::rotate(w_.out + t.off, w_.out + tail, w_.out + w_.len);
   }
 }
 
@@ -827,20 +860,6 @@ int Compiler::run(std::vector<Op>& ops, int* switches) {
     Event& e = events_[reg_first_ev_];
     for (C& x : e.entries) x = cmulf(x, gfac_);
     w_.rewrite(e.off, e.entries.data(), 16);
-  }
-  if (sign_) {
-    Event* to = nullptr;
-    for (Event& e : events_)
-      if (e.kind == 1) {
-        to = &e;
-        break;
-      }
-    if (to) {
-      for (C& x : to->entries) x.re = -x.re, x.im = -x.im;
-      w_.rewrite(to->off, to->entries.data(), int(to->entries.size()));
-    } else {
-      w_.emit(kRNeg, 0, 0, 0, nullptr, 0, nullptr, 0);
-    }
   }
   fold_cosines();
   *switches = switches_;

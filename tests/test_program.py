@@ -193,17 +193,50 @@ def test_rotations_alone(nrot, rng):
     assert ((blocking.OP_ROTS, 0) in kinds) == (nrot >= 5)
 
 
+def _rotations(n, layers, rng, kinds=("RX", "RY"), diagonals=1):
+    """Layers of rotations with few diagonals between them."""
+    c = Circuit(n)
+    for layer in range(layers):
+        for kind in kinds:
+            for q in range(n):
+                c.add(getattr(gates, kind)(q, float(rng.uniform(0, 2 * np.pi))))
+        if layer < diagonals:
+            c.add(gates.CZ(layer, layer + 1))
+    return c
+
+
 @pytest.mark.parametrize("cdt", [np.complex128, np.complex64])
-def test_other_angles_give_the_same_records(cdt):
-    n, low = 15, 3 if cdt == np.complex128 else 4
-    seqs = []
-    for seed in range(6):
+@pytest.mark.parametrize("circuit", ["layered", "rotations12", "rotations14", "diagonals", "none"])
+def test_other_angles_give_the_same_records(circuit, cdt):
+    """Which rotations are scaled, and where tables are added for them, follows
+    from the structure: kernels specialised to it serve every parameter set."""
+    make = {"layered": lambda r: models.random_layered_circuit(15, 10, seed=int(r.integers(1000)), measure=False),
+            "rotations12": lambda r: _rotations(12, 10, r), "rotations14": lambda r: _rotations(14, 20, r),
+            "diagonals": lambda r: _rotations(13, 9, r, ("RX", "RY", "RZ"), 9),
+            "none": lambda r: _rotations(12, 12, r, diagonals=0)}[circuit]
+    low = 3 if cdt == np.complex128 else 4
+    seqs, scaled, sheared = [], 0, 0
+    for seed in range(10):
         planner = GatePlanner("complex128" if cdt == np.complex128 else "complex64")
-        ops = [op for g in models.random_layered_circuit(n, 10, seed=seed, measure=False).queue
-               for op in planner.plan_ops(g)]
+        c = make(np.random.default_rng(seed))
+        ops = [op for g in c.queue for op in planner.plan_ops(g)]
         seqs.append([[(r[0], r[1], len(r[5])) for r in records(prog, count, np.dtype(cdt).itemsize)]
-                     for _, _, prog, count in _compiled(ops, n, cdt, low)])
+                     for _, _, prog, count in _compiled(ops, c.nqubits, cdt, low)])
+        scaled += sum(r[0] == blocking.OP_ROTS for s in seqs[-1] for r in s)
+        sheared += sum(r[0] == blocking.OP_ROT for s in seqs[-1] for r in s)
     assert all(s == seqs[0] for s in seqs[1:])
+    assert sheared <= 0.02 * scaled  # (the last few before a table that would not pay)
+
+
+@pytest.mark.parametrize("cdt,tol", [(np.complex128, 1e-13), (np.complex64, 2e-5)])
+@pytest.mark.parametrize("diagonals", [0, 1, 7])
+def test_long_runs_of_rotations(diagonals, cdt, tol, rng):
+    """Runs past the limit of one table, before and after the first record
+    that takes cosines."""
+    circuit = _rotations(13, 14, rng, diagonals=diagonals)
+    psi = _random_state(13, rng, cdt)
+    got, _ = _run(circuit, 13, cdt, psi)
+    assert np.max(np.abs(got - _oracle(circuit, 13, psi))) < tol
 
 
 def test_density_ops(rng):
