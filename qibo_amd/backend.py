@@ -1039,8 +1039,7 @@ class MI355XBackend(GatePlanner):
         ``source``: the amplitudes to start from (``state`` is not yet written); the
         first pass reads them there, and they stay as they are.
         """
-        keep = self._keeps_samples(state.dtype == torch.complex64, nqubits,
-                                   lambda: any(kinds.is_measurement(g) for g in reversed(queue)) if sampled is None else sampled)
+        keep = self._keeps_samples(state.dtype, queue, sampled)
         # [|0...0> still to be materialised, support, unwritten]: the support
         # is the mask of index bits that may be 1 in a nonzero amplitude (None:
         # any); the passes from |0...0> grow it by their tile bits, skip the
@@ -1059,7 +1058,7 @@ class MI355XBackend(GatePlanner):
                 state = gate.apply(self, state, nqubits)
             return state
         if nqubits < blocking.TILE_BITS:
-            return self._run_small(queue, state, nqubits)
+            return self._run_small(queue, state, nqubits, keep)
         key = self._queue_key(queue, nqubits, state, zero_pending) if self.program_cache else None
         if key is not None:
             key += (keep,)
@@ -1215,7 +1214,7 @@ class MI355XBackend(GatePlanner):
         self._complete(state, nqubits, zero)
         return state
 
-    def _run_small(self, queue, state: torch.Tensor, nqubits: int) -> torch.Tensor:
+    def _run_small(self, queue, state: torch.Tensor, nqubits: int, keep: bool = False) -> torch.Tensor:
         """Circuits on fewer than 12 qubits: run as one blocked pass on a
         12-qubit buffer whose extra (most significant) qubits stay |0>.
 
@@ -1236,9 +1235,9 @@ class MI355XBackend(GatePlanner):
             if gate.symbolic_parameters:
                 gate.substitute_symbols()
             ops.extend(self.plan_ops(gate))
-        return self._run_ops(ops, state, nqubits)
+        return self._run_ops(ops, state, nqubits, keep)
 
-    def _run_ops(self, ops, state: torch.Tensor, nqubits: int) -> torch.Tensor:
+    def _run_ops(self, ops, state: torch.Tensor, nqubits: int, keep: bool = False) -> torch.Tensor:
         """Planned ops on an nqubits register, in blocked passes; below 12
         qubits the register is the low end of a 12-qubit buffer whose extra
         (most significant) qubits stay |0> (qubit q becomes qubit q + p)."""
@@ -1249,13 +1248,13 @@ class MI355XBackend(GatePlanner):
                 self.apply_op(op, state, nqubits)
             return state
         if nqubits >= blocking.TILE_BITS:
-            return self._run_blocked(ops, state, nqubits)
+            return self._run_blocked(ops, state, nqubits, keep=keep)
         pad = blocking.TILE_BITS - nqubits
         shifted = [_Op(op.kind, tuple(q + pad for q in op.targets), tuple(q + pad for q in op.controls), op.data)
                    for op in ops]
         big = torch.zeros(2**blocking.TILE_BITS, dtype=state.dtype, device=state.device)
         big[: state.numel()].copy_(state)
-        big = self._run_blocked(shifted, big, blocking.TILE_BITS)
+        big = self._run_blocked(shifted, big, blocking.TILE_BITS, keep=keep)
         state.copy_(big[: state.numel()])
         return state
 
@@ -1284,7 +1283,8 @@ class MI355XBackend(GatePlanner):
             ops.extend(_dm_pair(self.plan_gate(gate), nqubits))
         for gate in mgates:
             gate.result.backend = self
-        key = ("density", nqubits, str(state.dtype), str(state.device), bool(self.blocking_ordered),
+        keep = self._keeps_samples(state.dtype, mgates)
+        key = ("density", nqubits, str(state.dtype), str(state.device), bool(self.blocking_ordered), keep,
                self._low_bits(self._dtype_code(state)),
                tuple((op.kind, op.targets, op.controls,
                       None if op.data is None else (op.data.dtype.str, op.data.shape, op.data.tobytes()))
@@ -1295,7 +1295,7 @@ class MI355XBackend(GatePlanner):
             self._replay(actions, [], flat, 2 * nqubits, [False])
             return True
         record = []
-        self._run_blocked(ops, flat, 2 * nqubits, None, record)
+        self._run_blocked(ops, flat, 2 * nqubits, None, record, keep)
         self._cache_put(key, record)
         return True
 
@@ -1310,6 +1310,7 @@ class MI355XBackend(GatePlanner):
         self._dm_check(state, nqubits, "run_queue_density_matrix")
         if self._run_dm_cached(queue, state, nqubits):
             return state
+        keep = self._keeps_samples(state.dtype, queue)
         ops = []
         for gate in queue:
             if kinds.is_measurement(gate) and not gate.collapse:
@@ -1322,14 +1323,14 @@ class MI355XBackend(GatePlanner):
                     ops.append(plan_matrix(sop, t + tuple(q + nqubits for q in t), ()))
                     continue
             if kinds.runs_outside_passes(gate):
-                self._run_ops(ops, state.view(-1), 2 * nqubits)
+                self._run_ops(ops, state.view(-1), 2 * nqubits, keep)
                 ops = []
                 state = gate.apply(self, state, nqubits).contiguous()
                 continue
             if gate.symbolic_parameters:  # conditioned on an earlier collapse
                 gate.substitute_symbols()
             ops.extend(_dm_pair(self.plan_gate(gate), nqubits))
-        self._run_ops(ops, state.view(-1), 2 * nqubits)
+        self._run_ops(ops, state.view(-1), 2 * nqubits, keep)
         return state
 
     def _fill_zero(self, state: torch.Tensor, nqubits: int):
@@ -1352,14 +1353,18 @@ class MI355XBackend(GatePlanner):
             zero[2] = False
 
     @staticmethod
-    def _keeps_samples(single: bool, nqubits: int, sampled) -> bool:
+    def _keeps_samples(dtype, queue, sampled: Optional[bool] = None) -> bool:
         """Whether a circuit's passes use compile_pass's records, whose rounding
-        fixes the shots of seeded complex64 runs. compile_program rounds each
-        gate differently, by about 6e-8 of the probability it moves in single
-        precision: above 18 qubits that is more than an entry of the cumulative
-        sum (2^-n), so seeded draws would land on other bitstrings. In double
-        precision the entry of the largest register (2^-36) is far above it."""
-        return single and nqubits > _SAMPLED_C64_QUBITS and sampled()
+        fixes the shots of seeded complex64 runs (``sampled``: shots will be
+        drawn; None: where the queue holds a measurement). compile_program
+        rounds each gate differently. In single precision that moves entries of
+        the cumulative sum by about 1e-6, and seeded draws beside them land on
+        other bitstrings: of 100000 shots 0.007 % at 11 qubits, 0.2 % at 16 and
+        0.55 % at 18 (20 layers of RY, RZ, CZ), so no register is small enough.
+        In double precision entries move 10^9 times less."""
+        if dtype != torch.complex64:
+            return False
+        return any(kinds.is_measurement(g) for g in reversed(queue)) if sampled is None else sampled
 
     def _run_blocked(self, ops, state: torch.Tensor, nqubits: int, zero=None, record=None,
                      keep: bool = False) -> torch.Tensor:
@@ -1869,7 +1874,6 @@ def _dm_pair(op: _Op, nqubits: int) -> List[_Op]:
     return [op, col]
 _BLOCK_OP = _Op("block", (), (), None)
 _ALL_BITS = (1 << 64) - 1  # support mask of a pass over every tile
-_SAMPLED_C64_QUBITS = 18  # complex64 registers above keep compile_pass's rounding when shots are drawn
 _FILL_FROM_ZERO_QUBITS = 22  # from this size on the first pass from |0...0> runs tile 0 alone
 _TILE_MASKS = {}  # tile bits -> their index mask
 

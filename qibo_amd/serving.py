@@ -361,7 +361,7 @@ class GPUExecutor:
         ops = [op for g in req.circuit.queue for op in backend.plan_ops(g)]
         code = _lib.C128 if req.dtype == "complex128" else _lib.C64
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
-        keep = backend._keeps_samples(code == _lib.C64, n, lambda: req.kind == "shots")
+        keep = code == _lib.C64 and req.kind == "shots"  # (as the backend's _keeps_samples)
         plan, program = blocking.compile_circuit(ops, n, cdtype, backend._low_bits(code),
                                                  backend.blocking_ordered, device=not keep)
         return code, plan, program
@@ -549,7 +549,7 @@ class GPUExecutor:
             sptr = stream.cuda_stream
             if compiled is None:
                 state = backend.zero_state(n)
-                state = backend.run_queue(list(req.circuit.queue), state, n)
+                state = backend.run_queue(list(req.circuit.queue), state, n, sampled=req.kind == "shots")
                 keep = (state,)
             else:
                 program, count = compiled
@@ -588,8 +588,9 @@ class GPUExecutor:
                                op.data))
         code = _lib.C128 if req.dtype == "complex128" else _lib.C64
         cdtype = np.complex128 if code == _lib.C128 else np.complex64
+        keep = code == _lib.C64 and req.kind == "shots"  # (as the backend's _keeps_samples)
         plan, program = blocking.compile_circuit(ops, blocking.TILE_BITS, cdtype, backend._low_bits(code),
-                                                 backend.blocking_ordered, device=True)
+                                                 backend.blocking_ordered, device=not keep)
         if len(plan) > 1 or (plan and plan[0][0] != "block"):
             return code, None  # not a single pass (e.g. a 4-qubit dense block): run it alone
         count = plan[0][3] if plan else 0
@@ -613,7 +614,8 @@ class GPUExecutor:
                 backend = self.backends[req.dtype]
                 with torch.cuda.stream(self.batch_stream):
                     state = backend.zero_state(req.nqubits)
-                    state = backend.run_queue(list(req.circuit.queue), state, req.nqubits)
+                    state = backend.run_queue(list(req.circuit.queue), state, req.nqubits,
+                                              sampled=req.kind == "shots")
                     tail = _Tail(backend, req.nqubits, code, req.kind, req.nshots)
                     tail.set_uniforms(req.seed)
                     tail.launch(state, self.batch_stream.cuda_stream)

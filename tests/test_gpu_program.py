@@ -12,7 +12,8 @@ import torch
 
 from oracle import OracleBackend
 from qibo_amd import Circuit, _lib, blocking, gates, models
-from qibo_amd.backend import GatePlanner, MI355XBackend
+from qibo_amd.backend import GatePlanner, MI355XBackend, _dm_pair, _Op
+from qibo_amd.serving import GPUExecutor, Request
 
 from tests.program_records import records, run_program
 from tests.specialize_programs import STEEP, mixed_circuit, steep_circuit
@@ -121,25 +122,70 @@ def test_swaps_alone_are_stored_after_every_load(specialize, rng):
         be.wait_specializations()
 
 
-def test_sampled_complex64_keeps_its_rounding(backend64):
-    """complex64 registers above 18 qubits keep compile_pass's records when
-    shots are drawn (their rounding decides the seeded shots); the same circuit
-    without a measurement, and smaller registers, run compile_program's."""
-    for n, kept in ((18, False), (19, True)):
-        c = models.random_layered_circuit(n, 3, seed=4)
-        planner = GatePlanner("complex64")
-        ops = [op for g in c.queue if g.__class__.__name__ != "M" for op in planner.plan_ops(g)]
-        state = torch.zeros(2**n, dtype=torch.complex64, device="cuda")
-        state[0] = 1
-        for kind, payload in blocking.partition(iter(ops), n, 4, False):
-            bits, pops = payload
-            prog, count, _ = blocking.compile_pass(bits, pops, n, np.complex64)
-            dev = torch.from_numpy(np.frombuffer(prog + bytes(blocking.PAD_BYTES), dtype=np.uint8).copy()).cuda()
-            _lib.check(backend64.lib.qsim_apply_blocked(state.data_ptr(), n, _lib.C64, _lib.int_array(bits),
-                                                        dev.data_ptr(), len(prog), count, None), backend64.lib)
+def _compile_pass_state(lib, ops, n):
+    """|0...0> through compile_pass's records, registers below a tile as its low end."""
+    pad = max(0, 12 - n)
+    ops = [_Op(op.kind, tuple(q + pad for q in op.targets), tuple(q + pad for q in op.controls), op.data) for op in ops]
+    state = torch.zeros(2 ** (n + pad), dtype=torch.complex64, device="cuda")
+    state[0] = 1
+    for kind, payload in blocking.partition(iter(ops), n + pad, 4, False):
+        bits, pops = payload
+        prog, count, _ = blocking.compile_pass(bits, pops, n + pad, np.complex64)
+        dev = torch.from_numpy(np.frombuffer(prog + bytes(blocking.PAD_BYTES), dtype=np.uint8).copy()).cuda()
+        _lib.check(lib.qsim_apply_blocked(state.data_ptr(), n + pad, _lib.C64, _lib.int_array(bits),
+                                          dev.data_ptr(), len(prog), count, None), lib)
         torch.cuda.synchronize()
-        start = torch.zeros_like(state)
-        start[0] = 1
-        assert torch.equal(backend64.execute_circuit(c, initial_state=start).state(), state) == kept
-        plain = models.random_layered_circuit(n, 3, seed=4, measure=False)
-        assert not torch.equal(backend64.execute_circuit(plain, initial_state=start).state(), state)
+    return state[: 2**n]
+
+
+@pytest.mark.parametrize("n", [5, 11, 12, 16, 18, 19])
+def test_sampled_complex64_keeps_its_rounding(backend64, n):
+    """complex64 registers keep compile_pass's records when shots are drawn
+    (their rounding decides the seeded shots), whatever their size; the same
+    circuit without a measurement runs compile_program's."""
+    c = models.random_layered_circuit(n, 5, seed=4)
+    planner = GatePlanner("complex64")
+    ops = [op for g in c.queue if g.__class__.__name__ != "M" for op in planner.plan_ops(g)]
+    state = _compile_pass_state(backend64.lib, ops, n)
+    start = torch.zeros_like(state)
+    start[0] = 1
+    for _ in range(2):  # (compiled, then replayed)
+        assert torch.equal(backend64.execute_circuit(c, initial_state=start).state(), state)
+    backend64.set_seed(5)
+    shots = backend64.execute_circuit(c, nshots=2000).samples()
+    backend64.set_seed(5)
+    want = backend64.sample_shots(backend64.calculate_probabilities(state, list(range(n)), n), 2000)
+    got = (torch.as_tensor(shots).cpu().long() << torch.arange(n - 1, -1, -1)).sum(1)
+    assert torch.equal(got, torch.as_tensor(want).cpu().long())
+    plain = models.random_layered_circuit(n, 5, seed=4, measure=False)
+    assert not torch.equal(backend64.execute_circuit(plain, initial_state=start).state(), state)
+
+
+@pytest.mark.parametrize("cached", [True, False])
+def test_sampled_complex64_density_matrices(cached):
+    n = 7
+    c = Circuit(n, density_matrix=True)
+    for g in models.random_layered_circuit(n, 3, seed=4).queue:
+        c.add(g)
+    planner = GatePlanner("complex64")
+    ops = [op for g in c.queue if g.__class__.__name__ != "M" for op in _dm_pair(planner.plan_gate(g), n)]
+    be = MI355XBackend(dtype="complex64")
+    be.program_cache = cached
+    want = _compile_pass_state(be.lib, ops, 2 * n).view(2**n, 2**n)
+    assert torch.equal(be.execute_circuit(c).state(), want)
+
+
+@pytest.mark.parametrize("small", [False, True])
+@pytest.mark.parametrize("n", [6, 13])
+def test_sampled_complex64_served(backend64, n, small):
+    """A served request for shots draws them from the state of a sampled run."""
+    c = models.random_layered_circuit(n, 5, seed=9, measure=False)
+    planner = GatePlanner("complex64")
+    state = _compile_pass_state(backend64.lib, [op for g in c.queue for op in planner.plan_ops(g)], n)
+    np.random.seed(3)
+    want = backend64.sample_shots(backend64.calculate_probabilities(state, list(range(n)), n), 5000).cpu().numpy()
+    executor = GPUExecutor({"complex64": backend64}, nstreams=2, batch_small=small)
+    h = executor.start(Request(0, c, "complex64", "shots", 5000, seed=3))
+    while not executor.done(h):
+        executor.idle()
+    np.testing.assert_array_equal(executor.result(h), want)
