@@ -429,9 +429,12 @@ int qsim_apply_pauli_sum(const void* state, int nqubits, int dtype, int nterms,
 /* qsim_apply_pauli_sum for nbatch states of 2^nqubits amplitudes each, one
  * after the other in `states` and in `out`, and energies[b] = Re <psi_b|out_b>
  * (device doubles, from the products before they are rounded to the state's
- * type): the seed of the adjoint sweep over a batch of parameter sets, in one
- * launch for Hamiltonians of at most 40 X masks and 96 terms. `workspace` must
- * hold qsim_apply_pauli_sum_batched_workspace(nbatch, nterms) bytes. */
+ * type): the seed of the adjoint sweep over a batch of parameter sets. A launch
+ * takes at least 64 terms: up to 64 diagonal ones (an even number of Y on no X
+ * mask) beside 64 items (48 beside more than 32 diagonal terms), where a mask
+ * takes an item for two terms of even numbers of Y and one for two of odd ones.
+ * More launches add to `out`, each rounding it to the state's type. `workspace`
+ * must hold qsim_apply_pauli_sum_batched_workspace(nbatch, nterms) bytes. */
 size_t qsim_apply_pauli_sum_batched_workspace(int nbatch, int nterms);
 int qsim_apply_pauli_sum_batched(const void* states, int nbatch, int nqubits, int dtype, int nterms,
                                  const uint64_t* xmasks, const uint64_t* zmasks, const int* ny,

@@ -110,7 +110,7 @@ constexpr int kPTileBits = 12;
 constexpr int kPReg = 16;
 constexpr int kPLaneBits = 8;     // local bits 0-7: the lane; 8-11: the register
 constexpr int kPLowBits = 3;      // index bits in every tile
-constexpr int kPMaxItems = 48;
+constexpr int kPMaxItems = 64;      // 48 beside more than 32 x = 0 terms (see PauliZ)
 constexpr int kPMaxDiag = 64;
 
 enum : uint32_t { kPImag = 1u << 16, kPFar = 1u << 17, kPTwo = 1u << 18 };
@@ -138,16 +138,19 @@ struct PauliTileArgs {
   PauliItem item[kPMaxItems];
   double dk[kPMaxDiag];
 };
-static_assert(sizeof(PauliTileArgs) <= 2304, "kernel arguments");
 
-// z masks of the terms in bit order of the sign words: words 0 and 1 the
-// x = 0 terms, 2-4 the items' terms (two bits per item).
+// z masks of the terms in bit order of the sign words: the items' terms from
+// word 0 on (two bits per item), the first 32 x = 0 terms in word 4, the next 32
+// in word 3, which the items past the 48th would take. So 64 terms of any kind
+// fit one launch (kernel arguments end at 4 KB) and a complex64 product of 64
+// terms is rounded once. The mask inside the lane bits sits in the top byte.
 constexpr int kPWords = 5;
+constexpr int kPZLaneShift = 56;
 struct PauliZ {
-  uint64_t zout[32 * kPWords];  // outside the tile
-  uint16_t zl[32 * kPWords];    // local lane bits
+  uint64_t z[32 * kPWords];
 };
-static_assert(kPMaxDiag <= 64 && 2 * kPMaxItems <= 96, "sign words");
+static_assert(QSIM_MAX_QUBITS <= kPZLaneShift && kPLaneBits <= 64 - kPZLaneShift, "masks of a term share a word");
+static_assert(sizeof(PauliTileArgs) + sizeof(PauliZ) + 3 * sizeof(void*) <= 4096, "kernel arguments");
 
 template <typename R>
 __device__ __forceinline__ cplx<double> widen(cplx<R> v) {
@@ -257,14 +260,15 @@ __global__ __launch_bounds__(kET, 2) void k_pauli_tile(const cplx<R>* __restrict
 #pragma unroll
   for (int w = 0; w < kPWords; ++w) {
     lane_sign[w] = 0;
-    const int cnt = w < 2 ? (a.ndiag - 32 * w) : (2 * a.nitems - 32 * (w - 2));
+    const int items = 2 * a.nitems - 32 * w, diags = a.ndiag - 32 * (4 - w);
+    const int cnt = w == 4 ? a.ndiag : (w == 3 && diags > items ? diags : items);
     for (int t = 0; t < 32 && t < cnt; ++t)
-      lane_sign[w] |= uint32_t(__popc(lane & zz.zl[32 * w + t]) & 1) << t;
+      lane_sign[w] |= uint32_t(__popc(lane & uint32_t(zz.z[32 * w + t] >> kPZLaneShift)) & 1) << t;
   }
 #pragma unroll
   for (int h = 0; h < (kPWords + 1) / 2; ++h) {
     const int t = 64 * h + int(lane & 63);
-    zo[h] = t < 32 * kPWords ? zz.zout[t] : 0;
+    zo[h] = t < 32 * kPWords ? zz.z[t] : 0;
   }
   double acc = 0.0;
   cplx<R> v[kPReg];
@@ -291,13 +295,13 @@ __global__ __launch_bounds__(kET, 2) void k_pauli_tile(const cplx<R>* __restrict
       // transform: w on the lane's 16 amplitudes
       double w[kPReg];
       int t = 0;
-      uint32_t word = sign[0];
+      uint32_t word = sign[4];
 #pragma unroll
       for (int k = 0; k < kPReg; ++k) {
         w[k] = 0.0;
         for (int left = a.dcount[k]; left > 0; --left) {
           w[k] += xor_sign(a.dk[t], word << 31);
-          word = ++t == 32 ? sign[1] : word >> 1;
+          word = ++t == 32 ? sign[3] : word >> 1;
         }
       }
 #pragma unroll
@@ -321,17 +325,20 @@ __global__ __launch_bounds__(kET, 2) void k_pauli_tile(const cplx<R>* __restrict
       }
     }
     PauliItem next = a.item[i0 < i1 ? i0 : 0];
-    uint32_t word = sign[2];
-    if (i0 >= 32)
-      word = sign[4];
-    else if (i0 >= 16)
+    uint32_t word = sign[0];
+    if (i0 >= 48)
       word = sign[3];
+    else if (i0 >= 32)
+      word = sign[2];
+    else if (i0 >= 16)
+      word = sign[1];
     word >>= 2 * (i0 & 15);
     for (int i = i0; i < i1; ++i) {
       const PauliItem g = next;  // read one item ahead
       next = a.item[i + 1 < i1 ? i + 1 : i];
       const uint32_t s0 = word << 31, s1 = (word << 30) & 0x80000000u;
-      word = (i + 1) == 16 ? sign[3] : ((i + 1) == 32 ? sign[4] : word >> 2);
+      word >>= 2;
+      if (((i + 1) & 15) == 0) word = i == 15 ? sign[1] : (i == 31 ? sign[2] : sign[3]);
       // (products of the lane's own amplitudes are formed where they are used,
       // not kept in registers from one item to the next)
 #pragma unroll
@@ -423,8 +430,9 @@ struct PauliBatch {
     int odd = 0;
     for (int i = 0; i < p.nterms; ++i) odd += p.ny[i] & 1;
     const int even = p.nterms - odd;
-    if (p.x == 0) return a.ndiag + even <= kPMaxDiag && a.nitems + (odd + 1) / 2 <= kPMaxItems;
-    return a.nitems + (odd + 1) / 2 + (even + 1) / 2 <= kPMaxItems;
+    const int diags = a.ndiag + (p.x == 0 ? even : 0);
+    const int items = a.nitems + (odd + 1) / 2 + (p.x == 0 ? 0 : (even + 1) / 2);
+    return diags <= kPMaxDiag && items <= (diags > 32 ? kPMaxItems - 16 : kPMaxItems);
   }
 
   void append(const PauliGroupArgs& p) {
@@ -479,8 +487,7 @@ struct PauliBatch {
       return uint16_t(p);
     };
     auto put = [&](int bit, uint64_t z) {
-      zz.zout[bit] = z & ~tmask;
-      zz.zl[bit] = uint16_t(localize(z) & ((1u << kPLaneBits) - 1));
+      zz.z[bit] = (z & ~tmask) | uint64_t(localize(z) & ((1u << kPLaneBits) - 1)) << kPZLaneShift;
     };
     int d = 0;
     for (int c = 0; c < kPReg; ++c) {
@@ -488,7 +495,8 @@ struct PauliBatch {
       for (int i = 0; i < a.ndiag; ++i)
         if ((localize(diag_z[i]) >> kPLaneBits) == uint32_t(c)) {
           a.dk[d] = diag_k[i];
-          put(d++, diag_z[i]);
+          put(d < 32 ? 128 + d : 64 + d, diag_z[i]);
+          ++d;
         }
       a.dcount[c] = uint8_t(d - first);
     }
@@ -500,7 +508,7 @@ struct PauliBatch {
         g.xl |= localize(g.x);
       for (int t = 0; t < 2; ++t) {
         g.pat[t] = pattern(item_z[i][t]);
-        put(64 + 2 * i + t, item_z[i][t]);
+        put(2 * i + t, item_z[i][t]);
       }
     }
   }
@@ -677,9 +685,9 @@ __global__ __launch_bounds__(kET) void k_pauli_apply(const cplx<R>* __restrict__
 // ---------------------------------------------------------------------------
 // out = sum_t c_t P_t psi for a batch of states, and <psi|out> beside it
 // ---------------------------------------------------------------------------
-// Launches of a term table (the groups of for_each_group, as many as fit one
-// launch's arguments): at most this many.
-static int apply_launches(int nterms) { return 1 + nterms / 16; }
+// Launches of a term table: at most this many (a launch that is full holds 64
+// terms or more, see PauliBatch::fits).
+static int apply_launches(int nterms) { return 1 + nterms / 64; }
 
 template <typename R>
 static int apply_impl(const void* state, int nbatch, int n, int nterms, const uint64_t* xm, const uint64_t* zm,
@@ -707,10 +715,22 @@ static int apply_impl(const void* state, int nbatch, int n, int nterms, const ui
     cur.clear();
   };
   for_each_group(nterms, xm, zm, ny, c, [&](const PauliGroupArgs& g) {
-    if (rc != QSIM_OK) return;
-    if (!cur.fits(g)) flush();
-    if (rc != QSIM_OK) return;
-    cur.append(g);
+    // a group is split where a launch is full: each launch rounds the product
+    // to the state's type, so no launch leaves with fewer terms than it can hold
+    for (int from = 0; from < g.nterms && rc == QSIM_OK;) {
+      PauliGroupArgs part = g;
+      for (part.nterms = g.nterms - from; part.nterms > 0; --part.nterms) {
+        std::copy(g.z + from, g.z + from + part.nterms, part.z);
+        std::copy(g.c + from, g.c + from + part.nterms, part.c);
+        std::copy(g.ny + from, g.ny + from + part.nterms, part.ny);
+        if (cur.fits(part)) break;
+      }
+      if (part.nterms == 0)
+        flush();
+      else
+        cur.append(part);
+      from += part.nterms;
+    }
   });
   if (rc == QSIM_OK) flush();
   if (rc != QSIM_OK || !energies) return rc;

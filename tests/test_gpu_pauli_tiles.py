@@ -83,6 +83,54 @@ def test_pauli_tables_by_tiles(request, n, dtype, rng):
     assert np.max(np.abs(one - want[0])) <= tol
 
 
+def _one_launch(kind, n, rng):
+    """At most 64 terms: distinct X masks, diagonal terms, both, and terms of
+    one mask with even and odd numbers of Y (an item each)."""
+    full = (1 << n) - 1
+    masks = [int(x) for x in rng.choice(np.arange(1, full), 64, replace=False)]
+    xm = {"masks": masks, "diagonal": [0] * 64, "both": [0] * 32 + masks[:32], "more_diagonal": [0] * 48 + masks[:16],
+          "parities": [m for m in masks[:32] for _ in range(2)], "one_mask": [5] * 64,
+          "singles_then_one_mask": sorted(masks)[:48] + [full] * 16}[kind]
+    zm = [int(z) for z in rng.integers(0, full + 1, size=len(xm))]
+    if kind == "parities":  # the number of common bits even, then odd
+        zm = [z ^ ((bin(x & z).count("1") + i) % 2) * (x & -x) for i, (x, z) in enumerate(zip(xm, zm))]
+    ny = [bin(x & z).count("1") for x, z in zip(xm, zm)]
+    return (np.array(xm, dtype=np.uint64), np.array(zm, dtype=np.uint64), np.array(ny, dtype=np.int32),
+            rng.normal(size=len(xm)))
+
+
+@pytest.mark.parametrize("n", [12, 20])
+@pytest.mark.parametrize("kind", ["masks", "diagonal", "both", "more_diagonal", "parities", "one_mask",
+                                  "singles_then_one_mask"])
+def test_complex64_products_of_64_terms_round_once(backend64, kind, n, rng):
+    """Sums of up to 64 terms are formed in double precision and rounded to
+    complex64 once: half a unit in the last place of each component, 2^-24 of
+    it, beside the 1e-13 of double-precision sums of 64 terms."""
+    be, lib = backend64, backend64.lib
+    xm, zm, ny, c = _one_launch(kind, n, rng)
+    nb = 2 if n < 20 else 1
+    psi = rng.normal(size=(nb, 2**n)) + 1j * rng.normal(size=(nb, 2**n))
+    psi = (psi / np.linalg.norm(psi, axis=1)[:, None]).astype(np.complex64)
+    want = np.array([_apply(p.astype(np.complex128), n, xm, zm, ny, c) for p in psi])
+    dev = torch.from_numpy(psi).cuda()
+    ws = torch.empty(lib.qsim_apply_pauli_sum_batched_workspace(nb, len(c)), dtype=torch.uint8, device="cuda")
+    out, es = torch.empty_like(dev), torch.empty(nb, dtype=torch.float64, device="cuda")
+    _lib.check(lib.qsim_apply_pauli_sum_batched(dev.data_ptr(), nb, n, be._dtype_code(dev), len(c), xm.ctypes.data,
+                                                zm.ctypes.data, ny.ctypes.data, c.ctypes.data, out.data_ptr(),
+                                                es.data_ptr(), ws.data_ptr(), ws.numel(), be._stream(dev)), lib)
+    one = be.apply_pauli_sum(dev[0].clone(), n, xm, zm, ny, c).cpu().numpy()
+    scale = float(np.sum(np.abs(c)))
+    for b in range(nb):
+        energy = float(np.real(np.vdot(psi[b].astype(np.complex128), want[b])))
+        assert abs(float(es[b]) - energy) <= 1e-12 * scale
+        assert abs(float(be.expectation_pauli(dev[b].clone(), n, xm, zm, ny, c)) - energy) <= 1e-12 * scale
+    slack = 1e-13 * scale * float(np.max(np.abs(psi)))
+    for got, ref in [(out.cpu().numpy(), want), (one, want[0])]:
+        for part in ("real", "imag"):
+            g, w = getattr(got, part).astype(np.float64), getattr(ref, part)
+            assert np.all(np.abs(g - w) <= 2.0**-24 * np.abs(w) + slack)
+
+
 def test_batched_pauli_sum_refuses_bad_arguments(backend):
     lib = backend.lib
     n, nb = 5, 2
