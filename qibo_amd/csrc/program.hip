@@ -15,7 +15,10 @@
 //    pair instead of three), the cosines multiplied into the entries of one
 //    unconditional record of the run;
 //  * a diagonal gate between one register bit and lane bits is split into a
-//    table, a per-lane phase and a controlled phase (0.30 CU-cycles as DIAG);
+//    table, a per-lane phase and a controlled phase (0.30 CU-cycles as DIAG).
+//    Factors of one table or phase are multiplied in extended precision, a
+//    lane's diag(a, b) is a factor a of the whole state and b / a on half the
+//    lanes, so that an amplitude is rounded no more often than gate by gate;
 //  * phases whose conditions lie outside the tile are skipped by whole
 //    workgroups; the controlled phases of one register bit share a record;
 //  * X gates without a condition on a lane bit exchange registers.
@@ -35,6 +38,25 @@ constexpr int kMapLayout = 3, kMapStart = 4, kMapRelabel = 5;
 // Local bits of one kind share the low bits of their LDS slot (blocked_dev.h:
 // swl, kSlotW): the first five lane positions take bits of five kinds.
 constexpr int kBankKind[kTileBits] = {0, 1, 2, 3, 4, 0, 1, 2, 4, 3, 0, 1};
+
+// Factors that the compiler multiplies together are kept in extended precision
+// and rounded where a record takes them: each record then costs an amplitude
+// the one rounding of its own product.
+struct L {
+  long double re = 1, im = 0;
+
+  L() = default;
+  L(long double r, long double i) : re(r), im(i) {}
+  L(const C& c) : re(c.re), im(c.im) {}
+  C rounded() const { return {double(re), double(im)}; }
+  long double norm2() const { return re * re + im * im; }
+  bool one() const { return re == 1 && im == 0; }
+};
+inline L operator*(const L& a, const L& b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
+inline L operator/(const L& a, const L& b) {
+  const long double m = b.norm2();
+  return a * L{b.re / m, -b.im / m};
+}
 
 struct Item {
   Op op;
@@ -126,13 +148,13 @@ class Compiler {
   bool stale_ = false;  // lane positions were renamed since the kernel formed the lane's index
   bool relabelled_unseen_ = false;  // any position was renamed since the kernel last saw a layout
   bool have_pending_ = false;
-  C pending_[16];
+  L pending_[16];
   long reg_first_off_ = -1;
   size_t reg_first_ev_ = 0;
-  C gfac_ = {1.0, 0.0};
+  L gfac_;  // a factor of the whole state, taken by the first record that can
   bool sign_ = false;
   int qpend_ = -1;
-  std::vector<std::pair<int, C>> phases_;  // controlled phases of register qpend_ not emitted yet: (bit, phase)
+  std::vector<std::pair<int, L>> phases_;  // controlled phases of register qpend_ not emitted yet: (bit, phase)
   int switches_ = 0;
 
   // rotations and the records that can take their cosines, in order
@@ -141,7 +163,7 @@ class Compiler {
     long off;  // rotation: header; others: first entry
     double t = 0, s = 0, tan = 0, c = 0;
     int dep = 0;
-    std::vector<C> entries;
+    std::vector<L> entries;
   };
   std::vector<Event> events_;
 
@@ -156,7 +178,9 @@ class Compiler {
   void qflush(int j);
   void emit_phases();
   void emit_diag(const Op& o);
-  void emit_phase(const int* tbits, int nt, const int* cbits, int nc, const C* d);
+  void emit_table(int dep, const L* table);
+  void rewrite(Event& e);
+  void emit_phase(const int* tbits, int nt, const int* cbits, int nc, const L* d);
   void emit_dense1(const Op& o, int j);
   void emit_dense2(const Op& o);
   void emit_lds(const Op& o);
@@ -425,13 +449,14 @@ void Compiler::emit_phases() {
   if (k <= 2) {
     for (const auto& p : phases_) {
       const uint64_t cm = uint64_t(1) << p.first, tm = outside(cm);
-      emit(kRLaneRegPhase, qpend_, cm & ~tm, 0, nullptr, 0, &p.second, 1, 0, tm);
+      const C x = p.second.rounded();
+      emit(kRLaneRegPhase, qpend_, cm & ~tm, 0, nullptr, 0, &x, 1, 0, tm);
     }
   } else {
     C data[64] = {};
     uint8_t bits[kMaxPhases] = {};
     for (int i = 0; i < k; ++i) {
-      data[i] = phases_[size_t(i)].second;
+      data[i] = phases_[size_t(i)].second.rounded();
       const int b = phases_[size_t(i)].first;
       bits[i] = uint8_t(local_[b] < 0 ? 0x80 | b : b);
     }
@@ -460,35 +485,47 @@ void Compiler::flush_reg(int j) {
   if (!have_pending_) return;
   auto depends_on = [&](int k) {
     for (int r = 0; r < 16; ++r)
-      if (!ceq(pending_[r], pending_[r ^ (1 << k)])) return true;
+      if (!ceq(pending_[r].rounded(), pending_[r ^ (1 << k)].rounded())) return true;
     return false;
   };
   if (j >= 0 && !depends_on(j)) return;
   have_pending_ = false;
-  const C t0 = pending_[0];
-  const double mag = t0.re * t0.re + t0.im * t0.im;
-  if (reg_first_off_ < 0 || std::fabs(mag - 1.0) > 1e-12) {
+  const L t0 = pending_[0];
+  if (reg_first_off_ < 0 || std::fabs(double(t0.norm2() - 1)) > 1e-12) {
     if (reg_first_off_ < 0) {
       reg_first_off_ = long(w_.len) + kHeader;
       reg_first_ev_ = events_.size();
     }
-    emit(kRRegPhase, 0, 0, 0, nullptr, 0, pending_, 16);
+    emit_table(0, pending_);
     return;
   }
   int dep = 0;
   for (int k = 0; k < 4; ++k)
     if (depends_on(k)) dep |= 1 << k;
-  gfac_ = cmulf(gfac_, t0);
+  gfac_ = gfac_ * t0;
   if (!dep) return;
-  const C inv = {t0.re / mag, -t0.im / mag};
-  C table[16];
-  for (int r = 0; r < 16; ++r) table[r] = (r & dep) ? cmulf(pending_[r], inv) : C{1.0, 0.0};
-  emit(kRRegPhase, dep, 0, 0, nullptr, 0, table, 16);
+  L table[16];
+  for (int r = 0; r < 16; ++r) table[r] = (r & dep) ? pending_[r] / t0 : L{};
+  emit_table(dep, table);
+}
+
+// A REG_PHASE record of the registers whose bits are in `dep` (0: of all).
+void Compiler::emit_table(int dep, const L* table) {
+  C data[16];
+  for (int r = 0; r < 16; ++r) data[r] = table[r].rounded();
+  emit(kRRegPhase, dep, 0, 0, nullptr, 0, data, 16);
+  events_.back().entries.assign(table, table + 16);
+}
+
+void Compiler::rewrite(Event& e) {
+  C data[16];
+  for (size_t i = 0; i < e.entries.size(); ++i) data[i] = e.entries[i].rounded();
+  w_.rewrite(e.off, data, int(e.entries.size()));
 }
 
 // A diagonal on the global bits tbits (first = most significant index bit)
 // under the bits cbits.
-void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, const C* d) {
+void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, const L* d) {
   auto reg = [&](int b) { return local_[b] >= 0 ? lay_.reg_of(local_[b]) : -1; };
   int nreg_t = 0, nreg_c = 0, jt = -1;
   for (int k = 0; k < nt; ++k)
@@ -502,26 +539,35 @@ void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, co
     else
       cm |= uint64_t(1) << cbits[k];
   }
+  auto unit = [](const L& x) { return std::fabs(double(x.norm2() - 1)) <= 1e-6; };
+  C rounded[1 << kMaxTargets];
+  for (int i = 0; i < (1 << nt); ++i) rounded[i] = d[i].rounded();
   if (nreg_t == 0 && nreg_c == 0) {
+    if (nt == 1 && nc == 0 && unit(d[0]) && unit(d[1])) {  // half the lanes are multiplied instead of all
+      gfac_ = gfac_ * d[0];
+      const L up = d[1] / d[0];
+      if (!up.one()) emit_phase(nullptr, 0, tbits, 1, &up);
+      return;
+    }
     const uint64_t tm = outside(cm);
-    emit(kRLanePhase, 0, cm & ~tm, nt, tbits, nt, d, 1 << nt, 0, tm, true);
+    emit(kRLanePhase, 0, cm & ~tm, nt, tbits, nt, rounded, 1 << nt, 0, tm, true);
     return;
   }
   if (nreg_t == nt && nreg_c == nc) {
     if (!have_pending_) {
-      for (int r = 0; r < 16; ++r) pending_[r] = {1.0, 0.0};
+      for (L& x : pending_) x = L{};
       have_pending_ = true;
     }
     for (int r = 0; r < 16; ++r) {
       if ((r & rreq) != rreq) continue;
       int di = 0;
       for (int k = 0; k < nt; ++k) di = (di << 1) | ((r >> reg(tbits[k])) & 1);
-      pending_[r] = cmulf(pending_[r], d[di]);
+      pending_[r] = pending_[r] * d[di];
     }
     return;
   }
   if (nt == 0) {
-    if (d[0].re == -1.0 && d[0].im == 0.0) {
+    if (d[0].re == -1 && d[0].im == 0) {
       emit(kRNeg, 0, cm, 0, nullptr, 0, nullptr, 0, rreq);
       return;
     }
@@ -532,61 +578,63 @@ void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, co
         qpend_ = j;
       }
       if ((cm & (cm - 1)) == 0) {  // one condition: collected
+        for (auto& p : phases_)
+          if (p.first == __builtin_ctzll(cm)) {
+            p.second = p.second * d[0];
+            return;
+          }
         if (int(phases_.size()) == kMaxPhases) emit_phases();
         phases_.emplace_back(__builtin_ctzll(cm), d[0]);
         return;
       }
       const uint64_t tm = outside(cm);
-      emit(kRLaneRegPhase, j, cm & ~tm, 0, nullptr, 0, d, 1, 0, tm);
+      emit(kRLaneRegPhase, j, cm & ~tm, 0, nullptr, 0, rounded, 1, 0, tm);
       return;
     }
   }
   // one register bit and lane bits: f(0, lanes) f(1, lanes) / f(0, lanes)
-  auto unit = [](C x) { return std::fabs(x.re * x.re + x.im * x.im - 1.0) <= 1e-6; };
-  auto over = [](C x, C y) {  // x / y
-    const double m = y.re * y.re + y.im * y.im;
-    return cmulf(x, C{y.re / m, -y.im / m});
-  };
   bool units = true;
   for (int i = 0; i < (1 << nt); ++i) units = units && unit(d[i]);
   if (units && nreg_t + nreg_c == 1) {
-    auto phase = [&](std::vector<int> c, C x) {  // x where every bit of c is 1
-      if (!(x.re == 1.0 && x.im == 0.0)) emit_phase(nullptr, 0, c.data(), int(c.size()), &x);
+    auto phase = [&](std::vector<int> c, L x) {  // x where every bit of c is 1
+      if (!x.one()) emit_phase(nullptr, 0, c.data(), int(c.size()), &x);
     };
     std::vector<int> cb(cbits, cbits + nc);
     if (nt == 1 && nreg_t == 1) {  // diag(a, b) on the register bit under lane bits
       phase(cb, d[0]);
       cb.push_back(tbits[0]);
-      phase(cb, over(d[1], d[0]));
+      phase(cb, d[1] / d[0]);
       return;
     }
     if (nt == 1 && nreg_c == 1) {  // diag(a, b) on a lane bit, the register bit among the conditions
       phase(cb, d[0]);
       cb.push_back(tbits[0]);
-      phase(cb, over(d[1], d[0]));
+      phase(cb, d[1] / d[0]);
       return;
     }
     if (nt == 2 && nreg_t == 1 && nc == 0) {
       const int jr = jt, jl = 1 - jt;
       auto at = [&](int r, int l) { return d[(r << (1 - jr)) | (l << (1 - jl))]; };
-      const C lane[2] = {at(0, 0), at(0, 1)};
+      const L lane[2] = {at(0, 0), at(0, 1)};
       emit_phase(&tbits[jl], 1, nullptr, 0, lane);
-      const C up[1] = {over(at(1, 0), at(0, 0))};
-      emit_phase(nullptr, 0, &tbits[jr], 1, up);
-      phase({tbits[jr], tbits[jl]}, over(over(at(1, 1), at(0, 1)), up[0]));
+      const L up = at(1, 0) / at(0, 0);
+      phase({tbits[jr]}, up);
+      phase({tbits[jr], tbits[jl]}, at(1, 1) / at(0, 1) / up);
       return;
     }
   }
   int enc[kMaxTargets];
   for (int k = 0; k < nt; ++k) enc[k] = reg(tbits[k]) >= 0 ? int(kRegFlag | uint32_t(reg(tbits[k]))) : tbits[k];
-  emit(kRDiag, 0, cm, nt, enc, nt, d, 1 << nt, rreq, 0, true);
+  emit(kRDiag, 0, cm, nt, enc, nt, rounded, 1 << nt, rreq, 0, true);
 }
 
 void Compiler::emit_diag(const Op& o) {
   int tb[kMaxTargets], cb[kMaxControls];
   for (int k = 0; k < o.nt; ++k) tb[k] = n_ - 1 - o.t[k];
   for (int k = 0; k < o.nc; ++k) cb[k] = n_ - 1 - o.c[k];
-  emit_phase(tb, o.nt, cb, o.nc, o.data);
+  L d[1 << kMaxTargets];
+  std::copy(o.data, o.data + o.ndata, d);
+  emit_phase(tb, o.nt, cb, o.nc, d);
 }
 
 void Compiler::emit_dense1(const Op& o, int j) {
@@ -769,8 +817,8 @@ void Compiler::fold_cosines() {
     if (t.off < 0) {
       if (t.factor == 1.0L) continue;
       Event& e = events_[t.event];
-      for (C& x : e.entries) x.re = double(x.re * t.factor), x.im = double(x.im * t.factor);
-      w_.rewrite(e.off, e.entries.data(), int(e.entries.size()));
+      for (L& x : e.entries) x.re *= t.factor, x.im *= t.factor;
+      rewrite(e);
       continue;
     }
     C table[16];
@@ -856,11 +904,19 @@ int Compiler::run(std::vector<Op>& ops, int* switches) {
     w_.emit(kRMap, kMapRelabel, lay_.word(), 0, nullptr, 0, nullptr, 0);
   }
   if (w_.overflow) return 0;
-  if (reg_first_off_ >= 0 && !(gfac_.re == 1.0 && gfac_.im == 0.0)) {
-    Event& e = events_[reg_first_ev_];
-    for (C& x : e.entries) x = cmulf(x, gfac_);
-    w_.rewrite(e.off, e.entries.data(), 16);
+  if (!gfac_.one()) {
+    Event* to = reg_first_off_ >= 0 ? &events_[reg_first_ev_] : nullptr;
+    for (Event& e : events_)
+      if (!to && e.kind == 1) to = &e;
+    if (to) {
+      for (L& x : to->entries) x = x * gfac_;
+      rewrite(*to);
+    } else {
+      const C x = gfac_.rounded();
+      emit(kRLanePhase, 0, 0, 0, nullptr, 0, &x, 1);
+    }
   }
+  if (w_.overflow) return 0;
   fold_cosines();
   *switches = switches_;
   return 0;

@@ -239,6 +239,47 @@ def test_long_runs_of_rotations(diagonals, cdt, tol, rng):
     assert np.max(np.abs(got - _oracle(circuit, 13, psi))) < tol
 
 
+def _extended(circuit, n, state):
+    """RX, RZZ and CRZ circuits in extended precision, angles included."""
+    state = state.astype(np.clongdouble)
+    idx = np.arange(2**n)
+    for g in circuit.queue:
+        half = np.longdouble(g.parameters[0]) / 2
+        c, s = np.cos(half), np.sin(half)
+        bit = [(idx >> (n - 1 - q)) & 1 for q in g.qubits]
+        if g.name == "rx":
+            state = c * state - 1j * s * state[idx ^ (1 << (n - 1 - g.qubits[0]))]
+        else:  # the sign of the phase: by parity, or by the target under the control
+            sign = np.where(bit[0] ^ bit[1], 1, -1) if g.name == "rzz" else np.where(bit[0] == 1, 2 * bit[1] - 1, 0)
+            state = np.where(sign == 0, 1, c + 1j * s * sign) * state
+    return state
+
+
+def test_phases_cost_no_precision():
+    """Diagonal gates between register and lane bits, split into a table, a
+    lane's phase and a controlled phase, together round an amplitude no more
+    often than gate by gate: the error against extended precision is at most the
+    oracle's, which rounds once per gate (with a tenth for their scatter over
+    four circuits; entries of split gates rounded one by one gave 1.4 times)."""
+    n, ours, oracle = 14, 0.0, 0.0
+    for seed in range(4):
+        rng = np.random.default_rng(seed)
+        c = Circuit(n)
+        for _ in range(8):
+            for q in range(n):
+                c.add(gates.RX(q, float(rng.uniform(0, 6))))
+            for _ in range(n):
+                for kind in (gates.CRZ, gates.RZZ):
+                    a, b = (int(x) for x in rng.choice(n, 2, replace=False))
+                    c.add(kind(a, b, float(rng.uniform(0, 6))))
+        psi = _random_state(n, rng, np.complex128)
+        want = _extended(c, n, psi)
+        got, _ = _run(c, n, np.complex128, psi)
+        ours += float(np.linalg.norm((got - want).astype(np.complex128)))
+        oracle += float(np.linalg.norm((_oracle(c, n, psi) - want).astype(np.complex128)))
+    assert ours <= 1.1 * oracle
+
+
 def test_density_ops(rng):
     """Conjugate pairs and real transfer matrices on (row, column) qubits run
     in registers (the channel's 4x4 touches the pairs (00, 11) and (01, 10))."""
