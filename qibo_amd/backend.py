@@ -912,17 +912,18 @@ class MI355XBackend(GatePlanner):
         from .result import CircuitResult, QuantumState
 
         nqubits = circuit.nqubits
+        sampled = bool(circuit.measurements) or circuit.has_collapse
         if circuit.density_matrix:
             state = self.zero_state(nqubits, density_matrix=True) if initial_state is None else initial_state
-            state = self.run_queue_density_matrix(circuit.queue, state, nqubits)
+            state = self.run_queue_density_matrix(circuit.queue, state, nqubits, sampled)
         elif initial_state is None and self.blocking and nqubits >= blocking.TILE_BITS:
             # |0...0> is produced by the first blocked pass itself (no zero fill)
             self._validate_nqubits(nqubits)
             state = self._alloc_state(nqubits)  # budget check and MemoryError as zero_state
-            state = self.run_queue(circuit.queue, state, nqubits, zero_pending=True)
+            state = self.run_queue(circuit.queue, state, nqubits, zero_pending=True, sampled=sampled)
         else:
             state = self.zero_state(nqubits) if initial_state is None else initial_state
-            state = self.run_queue(circuit.queue, state, nqubits, source=source)
+            state = self.run_queue(circuit.queue, state, nqubits, sampled=sampled, source=source)
         if circuit.measurements:
             circuit._final_state = CircuitResult(state, circuit.measurements, backend=self, nshots=nshots)
         else:
@@ -958,13 +959,13 @@ class MI355XBackend(GatePlanner):
         for _ in range(nshots):
             state = state_copy.clone()
             if dm:
-                state = self.run_queue_density_matrix(circuit.queue, state, nqubits)
+                state = self.run_queue_density_matrix(circuit.queue, state, nqubits, True)
                 if total is None:
                     total = self.dm_axpy(torch.empty_like(state), state, 1.0, accumulate=False)
                 else:
                     self.dm_axpy(total, state, 1.0)
             else:
-                state = self.run_queue(circuit.queue, state, nqubits)
+                state = self.run_queue(circuit.queue, state, nqubits, sampled=True)
             if circuit.measurements:
                 result = CircuitResult(state, circuit.measurements, backend=self, nshots=1)
                 sample = result.samples()[0]
@@ -1258,7 +1259,7 @@ class MI355XBackend(GatePlanner):
         state.copy_(big[: state.numel()])
         return state
 
-    def _run_dm_cached(self, queue, state: torch.Tensor, nqubits: int) -> bool:
+    def _run_dm_cached(self, queue, state: torch.Tensor, nqubits: int, sampled: Optional[bool] = None) -> bool:
         """Run a density-matrix queue whose every element is a unitary gate, a
         non-collapsing measurement or a channel with a transfer matrix as one
         op list, reusing the compiled passes of an identical op list (the
@@ -1283,7 +1284,7 @@ class MI355XBackend(GatePlanner):
             ops.extend(_dm_pair(self.plan_gate(gate), nqubits))
         for gate in mgates:
             gate.result.backend = self
-        keep = self._keeps_samples(state.dtype, mgates)
+        keep = self._keeps_samples(state.dtype, mgates, sampled)
         key = ("density", nqubits, str(state.dtype), str(state.device), bool(self.blocking_ordered), keep,
                self._low_bits(self._dtype_code(state)),
                tuple((op.kind, op.targets, op.controls,
@@ -1299,7 +1300,8 @@ class MI355XBackend(GatePlanner):
         self._cache_put(key, record)
         return True
 
-    def run_queue_density_matrix(self, queue, state: torch.Tensor, nqubits: int) -> torch.Tensor:
+    def run_queue_density_matrix(self, queue, state: torch.Tensor, nqubits: int,
+                                 sampled: Optional[bool] = None) -> torch.Tensor:
         """Apply ``queue`` to a density matrix (the loop of abstract.py:3321-3322).
 
         Unitary gates become pairs of planned ops on the 2n-qubit vectorized
@@ -1308,9 +1310,9 @@ class MI355XBackend(GatePlanner):
         gates run in order between the passes through ``gate.apply``."""
         state = state.contiguous()
         self._dm_check(state, nqubits, "run_queue_density_matrix")
-        if self._run_dm_cached(queue, state, nqubits):
+        if self._run_dm_cached(queue, state, nqubits, sampled):
             return state
-        keep = self._keeps_samples(state.dtype, queue)
+        keep = self._keeps_samples(state.dtype, queue, sampled)
         ops = []
         for gate in queue:
             if kinds.is_measurement(gate) and not gate.collapse:
