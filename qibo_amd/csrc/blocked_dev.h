@@ -301,6 +301,16 @@ __device__ __forceinline__ uint32_t lay_slot(uint32_t u) {
   return LdsSlots<R>::kAdd ? slot_f64(u) : swl<R>(u);
 }
 
+// Slot of the single local bit b, from one table of what the layouts add to
+// 2^b (bits 5-11, a byte each): a few scalar operations where b is known at run
+// time only.
+template <typename R>
+__device__ __forceinline__ constexpr uint32_t lay_slot_bit(uint32_t b) {
+  constexpr uint64_t extra = LdsSlots<R>::kAdd ? 0x7E3F2810040201ull
+                                               : (sizeof(R) == 4 ? 0x3E3F2830242201ull : 0x1E1F0810040201ull);
+  return (1u << b) + (b < 5 ? 0u : uint32_t(extra >> (8 * (b - 5))) & 255u);
+}
+
 // All-ones where bit p of the lane number is set.
 __device__ __forceinline__ uint32_t lane_mask(int p) { return uint32_t(int32_t(threadIdx.x << (31 - p)) >> 31); }
 
@@ -309,7 +319,7 @@ template <typename R>
 __device__ __forceinline__ uint32_t lay_lane_slot(uint64_t L) {
   uint32_t s = 0;
 #pragma clang loop unroll(full)
-  for (int p = 0; p < 8; ++p) s = LdsSlots<R>::join(s, lane_mask(p) & lay_slot<R>(1u << lay_bit(L, p)));
+  for (int p = 0; p < 8; ++p) s = LdsSlots<R>::join(s, lane_mask(p) & lay_slot_bit<R>(lay_bit(L, p)));
   return s;
 }
 
@@ -318,7 +328,7 @@ __device__ __forceinline__ uint32_t lay_reg_slot(uint64_t L, uint32_t r) {
   uint32_t s = 0;
 #pragma clang loop unroll(full)
   for (int j = 0; j < 4; ++j)
-    if ((r >> j) & 1) s = LdsSlots<R>::join(s, lay_slot<R>(1u << lay_bit(L, 8 + j)));
+    if ((r >> j) & 1) s = LdsSlots<R>::join(s, lay_slot_bit<R>(lay_bit(L, 8 + j)));
   return s;
 }
 
@@ -1103,63 +1113,71 @@ __device__ __forceinline__ uint64_t insert_local(uint32_t u, const BlkArgs& a) {
 template <typename R, int K>
 __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, uint64_t L, const Hdr& in, const cplx<R>* m,
                                           uint64_t tile_base, const BlkArgs& args) {
+  using S = LdsSlots<R>;
   constexpr int D = 1 << K;
   constexpr int NG = (kBTile >> K) / kBT;  // groups per lane
-  uint32_t srt[K];
-  uint32_t off[D];
+  constexpr uint32_t kB = sizeof(R);
+  uint32_t srt[K], tslot[K];
 #pragma clang loop unroll(full)
-  for (int t = 0; t < K; ++t) srt[t] = hbit(in, 4 + t) < kBTileBits ? hbit(in, 4 + t) : kBTileBits - 1;
-#pragma clang loop unroll(full)
-  for (int r = 0; r < D; ++r) {
-    uint32_t o = 0;
-#pragma clang loop unroll(full)
-    for (int t = 0; t < K; ++t) {
-      const uint32_t b = hbit(in, t) < kBTileBits ? hbit(in, t) : kBTileBits - 1;
-      if ((r >> (K - 1 - t)) & 1) o |= 1u << b;
-    }
-    off[r] = o;
+  for (int t = 0; t < K; ++t) {
+    srt[t] = hbit(in, 4 + t) < kBTileBits ? hbit(in, 4 + t) : kBTileBits - 1;
+    tslot[t] = lay_slot_bit<R>(hbit(in, t) < kBTileBits ? hbit(in, t) : kBTileBits - 1) * kB;
   }
-  uint32_t base[NG];
-  bool act[NG];
-#pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i) {
-    uint32_t b = threadIdx.x + i * kBT;
+  auto spread = [&](uint32_t b) {  // zeros at the target bits
 #pragma clang loop unroll(full)
     for (int t = 0; t < K; ++t) {
       const uint32_t low = b & ((1u << srt[t]) - 1);
       b = low | ((b ^ low) << 1);
     }
-    base[i] = b;
-    act[i] = ((tile_base | insert_local(b, args)) & in.cmask) == in.cmask;
+    return b;
+  };
+  // Input c of group i sits at the lane's bits, i's and c's, disjoint ones, so
+  // its slot is the lane's joined with one that all lanes share: one vector
+  // operation per access. (Twelve 3-qubit blocks on 24 qubits: 322 us in
+  // complex64, 369 in complex128; with slots formed per group from its whole
+  // index, and conditions tested where there are none, 400 and 440.)
+  const uint32_t first = spread(threadIdx.x), lane = lay_slot<R>(first) * kB;
+  uint32_t at[kBReg];  // bytes, uniform
+  bool act[NG];
+#pragma clang loop unroll(full)
+  for (int i = 0; i < NG; ++i) {
+    act[i] = true;
+#pragma clang loop unroll(full)
+    for (int c = 0; c < D; ++c) {
+      uint32_t s = lay_slot<R>(spread(uint32_t(i) * kBT)) * kB;
+#pragma clang loop unroll(full)
+      for (int t = 0; t < K; ++t)
+        if ((c >> (K - 1 - t)) & 1) s = S::join(s, tslot[t]);
+      at[i * D + c] = s;
+    }
   }
-  using S = LdsSlots<R>;
-  uint32_t slot[kBReg];  // the lane's amplitudes in the current layout
-  const uint32_t s0 = lay_lane_slot<R>(L);
+  if (in.cmask != 0) {
+    const uint64_t index = tile_base | insert_local(first, args);
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) slot[r] = S::join(s0, lay_reg_slot<R>(L, uint32_t(r)));
-  // group i's input c sits at base[i] | off[c] (disjoint bits)
-  uint32_t bslot[NG], oslot[D];
+    for (int i = 0; i < NG; ++i)
+      act[i] = ((index | insert_local(spread(uint32_t(i) * kBT), args)) & in.cmask) == in.cmask;
+  }
+  uint32_t own[kBReg];  // the lane's amplitudes in the current layout, likewise
+  const uint32_t home = lay_lane_slot<R>(L) * kB;
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i) bslot[i] = lay_slot<R>(base[i]);
-#pragma clang loop unroll(full)
-  for (int c = 0; c < D; ++c) oslot[c] = lay_slot<R>(off[c]);
+  for (int r = 0; r < kBReg; ++r) own[r] = lay_reg_slot<R>(L, uint32_t(r)) * kB;
+  char* const buf = reinterpret_cast<char*>(lds);
+  auto slot = [&](uint32_t lane_bytes, uint32_t bytes) -> R& {
+    return *reinterpret_cast<R*>(buf + (S::kAdd ? lane_bytes + bytes : slot_bytes(lane_bytes, bytes)));
+  };
   cplx<R> g[kBReg];  // g[i * D + c]: input c of group i
   // gather: real parts, then imaginary parts
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) lds[slot[r]] = v[r].re;
+  for (int r = 0; r < kBReg; ++r) slot(home, own[r]) = v[r].re;
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i)
-#pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) g[i * D + c].re = lds[S::join(bslot[i], oslot[c])];
+  for (int k = 0; k < kBReg; ++k) g[k].re = slot(lane, at[k]);
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) lds[slot[r]] = v[r].im;
+  for (int r = 0; r < kBReg; ++r) slot(home, own[r]) = v[r].im;
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i)
-#pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) g[i * D + c].im = lds[S::join(bslot[i], oslot[c])];
+  for (int k = 0; k < kBReg; ++k) g[k].im = slot(lane, at[k]);
   __syncthreads();
   // multiply (the arithmetic of the one-gate kernels: cmul, then cfma in column order)
 #pragma clang loop unroll(full)
@@ -1178,20 +1196,16 @@ __device__ __forceinline__ void dense_lds(R* lds, cplx<R>* v, uint64_t L, const 
   }
   // scatter back and reload the lane's amplitudes in the current mapping
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i)
-#pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) lds[S::join(bslot[i], oslot[c])] = g[i * D + c].re;
+  for (int k = 0; k < kBReg; ++k) slot(lane, at[k]) = g[k].re;
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) v[r].re = lds[slot[r]];
+  for (int r = 0; r < kBReg; ++r) v[r].re = slot(home, own[r]);
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int i = 0; i < NG; ++i)
-#pragma clang loop unroll(full)
-    for (int c = 0; c < D; ++c) lds[S::join(bslot[i], oslot[c])] = g[i * D + c].im;
+  for (int k = 0; k < kBReg; ++k) slot(lane, at[k]) = g[k].im;
   __syncthreads();
 #pragma clang loop unroll(full)
-  for (int r = 0; r < kBReg; ++r) v[r].im = lds[slot[r]];
+  for (int r = 0; r < kBReg; ++r) v[r].im = slot(home, own[r]);
   __syncthreads();
 }
 
