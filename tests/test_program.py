@@ -280,6 +280,19 @@ def test_phases_cost_no_precision():
     assert ours <= 1.1 * oracle
 
 
+@pytest.mark.parametrize("n,layers", [(12, 10), (12, 20), (14, 10), (20, 10)])
+def test_layouts_change_no_more_often_than_mappings(n, layers):
+    """The free choice of register bits is not behind compile_pass's three groups."""
+    planner = GatePlanner()
+    ops = [op for g in models.random_layered_circuit(n, layers, seed=3, measure=False).queue for op in planner.plan_ops(g)]
+    free = fixed = 0
+    for kind, payload in blocking.partition(iter(ops), n, 3, False):
+        prog, count = blocking.compile_program(payload[0], payload[1], n, np.complex128, 3)
+        free += sum(r[0] == blocking.OP_MAP and r[1] == blocking.MAP_LAYOUT for r in records(prog, count, 16))
+        fixed += blocking.compile_pass(payload[0], payload[1], n, np.complex128)[2]
+    assert free <= fixed + 1  # (the tile may be stored from the last layout only)
+
+
 def test_density_ops(rng):
     """Conjugate pairs and real transfer matrices on (row, column) qubits run
     in registers (the channel's 4x4 touches the pairs (00, 11) and (01, 10))."""
