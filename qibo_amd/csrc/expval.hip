@@ -641,9 +641,9 @@ static int expval_impl(const void* state, int n, int nterms, const uint64_t* xm,
 }
 
 // ---------------------------------------------------------------------------
-// out = sum_t c_t P_t psi of one state of few tiles (gather form, one output
-// amplitude per thread: more workgroups than tiles; 16 qubits: 15 us against
-// 24 us by tiles, equal at 20 qubits, 23 qubits: 294 us against 207 us)
+// out = sum_t c_t P_t psi of one state of few tiles or by few terms (gather
+// form, one output amplitude per thread: more workgroups than tiles; 16 qubits:
+// 15 us against 24 us by tiles; see tiles_pay)
 // ---------------------------------------------------------------------------
 struct PauliApplyArgs {
   uint64_t n;
@@ -688,6 +688,36 @@ __global__ __launch_bounds__(kET) void k_pauli_apply(const cplx<R>* __restrict__
 // Launches of a term table: at most this many (a launch that is full holds 64
 // terms or more, see PauliBatch::fits).
 static int apply_launches(int nterms) { return 1 + nterms / 64; }
+
+// Whether one state of 20 qubits or more (as many tiles as CUs) is cheaper by
+// tiles than by k_pauli_apply. That one reads a partner per term and amplitude;
+// a tile pass costs more before its first term and a little more for each mask
+// that leaves the tile, but next to nothing for a term on the lowest 12 index
+// bits and for further terms of one mask. Equal at so many
+//   qubits                         20      22      24     27
+//   terms in the tile, complex128  18-30   10-13   6-9    4-6   (diagonal ones to X)
+//                      complex64   8-20    5-10    2-5    1
+//   masks outside it, complex64    > 32    24      16     8     (complex128: none)
+// (24 qubits, complex128: one X 89 us against 133 us by tiles, 24 Z pairs 319 us
+// against 138 us).
+static bool tiles_pay(int n, int dtype, int nterms, const uint64_t* xm, const uint64_t* zm, const int* ny,
+                      const double* c) {
+  int near = 0, again = 0, masks = 0;  // terms in the tile; further terms of masks outside it, and those masks
+  uint64_t last = 0;
+  for_each_group(nterms, xm, zm, ny, c, [&](const PauliGroupArgs& g) {
+    if (!(g.x >> kPTileBits)) {
+      near += g.nterms;
+      return;
+    }
+    masks += g.x != last;
+    again += g.nterms - (g.x != last);
+    last = g.x;
+  });
+  // (a state below 24 qubits, complex64 22, stays in cache between its terms)
+  const int small = std::max(0, 27 - n);
+  if (dtype == QSIM_C128) return near + (n < 24 ? 1 : 5) * again - masks >= 4 + 2 * small;
+  return 2 * near + (n < 22 ? 2 : 6) * again + masks - (masks > 0 ? 8 : 0) >= 2 + 3 * small;
+}
 
 template <typename R>
 static int apply_impl(const void* state, int nbatch, int n, int nterms, const uint64_t* xm, const uint64_t* zm,
@@ -932,7 +962,7 @@ int qsim_apply_pauli_sum(const void* state, int nqubits, int dtype, int nterms, 
   for (int t = 0; t < nterms; ++t)
     QSIM_CHECK_ARG((xmasks[t] & ~full) == 0 && (zmasks[t] & ~full) == 0, "qsim_apply_pauli_sum: mask out of range");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (nqubits < kPTileBits + 8) {  // fewer tiles than CUs
+  if (nqubits < kPTileBits + 8 || !tiles_pay(nqubits, dtype, nterms, xmasks, zmasks, ny, coeffs)) {
     const uint64_t N = uint64_t(1) << nqubits;
     for (int t0 = 0; t0 < nterms; t0 += 64) {
       PauliApplyArgs a;

@@ -131,6 +131,37 @@ def test_complex64_products_of_64_terms_round_once(backend64, kind, n, rng):
             assert np.all(np.abs(g - w) <= 2.0**-24 * np.abs(w) + slack)
 
 
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+@pytest.mark.parametrize("n", [20, 22, 24])
+def test_products_on_both_sides_of_the_rule(request, n, dtype, rng):
+    """One state from 20 qubits on is multiplied term by term where the terms
+    are few or leave the tile, else by tiles: the same product either way (to a
+    unit in the last place of complex64, 1e-13 of the coefficients' sum)."""
+    be = request.getfixturevalue("backend" if dtype == "complex128" else "backend64")
+    psi = torch.randn(2**n, dtype=torch.complex128, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    psi = (psi / psi.norm()).to(getattr(torch, dtype))
+    wide = psi.to(torch.complex128)
+    high, idx = n - 1, torch.arange(2**n, device="cuda")
+    for xm in ([1], [1 << high], [0] * 3 + [1 << high], [0, 0, 1, 2, 4, 8] * 4, [1 << high] * 6 + [3],
+               [1 << b for b in range(n)] + [0] * 6):
+        zm = [int(z) for z in rng.integers(0, 2**n, size=len(xm))]
+        ny = [bin(x & z).count("1") for x, z in zip(xm, zm)]
+        c = rng.normal(size=len(xm))
+        want = torch.zeros_like(wide)
+        for x, z, y, k in zip(xm, zm, ny, c):
+            j = idx ^ x
+            p = j & z
+            for s in (32, 16, 8, 4, 2, 1):
+                p = p ^ (p >> s)
+            want += 1j**y * (float(k) * (1 - 2 * (p & 1)).to(torch.float64)) * wide[j]
+        got = be.apply_pauli_sum(psi, n, np.array(xm, dtype=np.uint64), np.array(zm, dtype=np.uint64),
+                                 np.array(ny, dtype=np.int32), c).to(torch.complex128)
+        slack = 1e-13 * float(np.sum(np.abs(c))) * float(wide.abs().max())
+        last = 2.0**-24 if dtype == "complex64" else 0.0
+        err, ref = torch.view_as_real(got - want).abs(), torch.view_as_real(want).abs()
+        assert bool((err <= last * ref + slack).all())
+
+
 def test_batched_pauli_sum_refuses_bad_arguments(backend):
     lib = backend.lib
     n, nb = 5, 2
