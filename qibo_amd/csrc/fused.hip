@@ -14,11 +14,33 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstring>
 
 #include "qsim_common.h"
 
 namespace qsim {
+
+// Workgroups of a kernel that a device keeps resident, the grid of a persistent
+// launch. Kept per kernel (a static of its launcher) and device.
+constexpr int kDevices = 64;
+struct PerDevice {
+  std::atomic<unsigned> blocks[kDevices] = {};
+};
+
+template <typename F>
+static unsigned resident_blocks(PerDevice& cache, F kernel, int threads, int per_cu_if_unknown) {
+  int dev = 0, per_cu = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) dev = 0;
+  if (dev < kDevices)
+    if (const unsigned known = cache.blocks[dev].load(std::memory_order_relaxed)) return known;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1)
+    per_cu = per_cu_if_unknown;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+  const unsigned blocks = unsigned(per_cu) * unsigned(cus);
+  if (dev < kDevices) cache.blocks[dev].store(blocks, std::memory_order_relaxed);
+  return blocks;
+}
 
 constexpr int kFusedThreads = 256;
 
@@ -316,18 +338,8 @@ static int launch_fused_mfma(void* state, const void* source, int n, const int* 
       if (bits[i] == gb) a.rowbit[t] = uint8_t(i);
   }
   // persistent grid: as many workgroups as the device keeps resident
-  static int per_cu[2] = {0, 0};  // per K = 4, 5 (the answer is fixed for the kernel)
-  static int cus = 0;
-  if (per_cu[K - 4] == 0) {
-    int nb = 0, dev = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_fused_mfma_c64<K>, 256, 0) != hipSuccess || nb < 1)
-      nb = 2;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-      cus = 256;
-    per_cu[K - 4] = nb;
-  }
-  const uint64_t resident = uint64_t(cus) * uint64_t(per_cu[K - 4]);
+  static PerDevice cache;
+  const unsigned resident = resident_blocks(cache, k_fused_mfma_c64<K>, 256, 2);
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_mfma_c64<K>), dim3(grid), dim3(256), 0, s, a, reinterpret_cast<const c64*>(mat),
                      reinterpret_cast<const c64*>(source), reinterpret_cast<c64*>(state));
@@ -527,15 +539,8 @@ static int launch_fused_tile_c128(void* state, const void* source, int n, const 
       if (bits[i] == gb) a.rowbit[t] = uint8_t(i);
   }
   // persistent grid: as many workgroups as the device keeps resident
-  static const unsigned resident = [] {
-    int nbk = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nbk, k_fused_tile_c128<K>, 256, 0) != hipSuccess || nbk < 1)
-      nbk = 2;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-      cus = 256;
-    return unsigned(nbk) * unsigned(cus);
-  }();
+  static PerDevice cache;
+  const unsigned resident = resident_blocks(cache, k_fused_tile_c128<K>, 256, 2);
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_tile_c128<K>), dim3(grid), dim3(256), 0, s, a, reinterpret_cast<const c128*>(mat),
                      reinterpret_cast<const c128*>(source), reinterpret_cast<c128*>(state));
@@ -744,16 +749,8 @@ static void pair_args(Pair128Args& a, int n, const int* const targets[2], const 
 template <int K1, int K2>
 static int launch_fused_pair(const Pair128Args& a, const void* m1, const void* m2, void* state, const void* source,
                              hipStream_t s) {
-  static const unsigned resident = [] {
-    int nbk = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nbk, k_fused_pair_c128<K1, K2>, kPairThreads, 0) != hipSuccess ||
-        nbk < 1)
-      nbk = 1;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-      cus = 256;
-    return unsigned(nbk) * unsigned(cus);
-  }();
+  static PerDevice cache;
+  const unsigned resident = resident_blocks(cache, k_fused_pair_c128<K1, K2>, kPairThreads, 1);
   const unsigned grid = unsigned(a.ntiles < resident ? a.ntiles : resident);
   hipLaunchKernelGGL((k_fused_pair_c128<K1, K2>), dim3(grid), dim3(kPairThreads), 0, s, a,
                      reinterpret_cast<const c128*>(m1), reinterpret_cast<const c128*>(m2),
