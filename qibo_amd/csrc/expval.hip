@@ -113,7 +113,7 @@ constexpr int kPLowBits = 3;      // index bits in every tile
 constexpr int kPMaxItems = 64;      // 48 beside more than 32 x = 0 terms (see PauliZ)
 constexpr int kPMaxDiag = 64;
 
-enum : uint32_t { kPImag = 1u << 16, kPFar = 1u << 17, kPTwo = 1u << 18 };
+enum : uint32_t { kPImag = 1u << 16, kPFar = 1u << 17 };
 
 // One or two terms of one X mask, their coefficients both real or both
 // imaginary. A term's sign at amplitude i is a tile part times a lane part

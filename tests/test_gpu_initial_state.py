@@ -50,13 +50,33 @@ def test_states_that_are_copied_first(backend):
     run = lambda s: torch.as_tensor(backend.execute_circuit(_circuit("passes", n), initial_state=s).state()).cuda()  # noqa: E731
     ref = run(psi)
     assert torch.equal(run(psi.cpu().numpy()), ref)
-    twice = torch.empty(2, 2**n, dtype=torch.complex128, device="cuda").t()
+    # a strided view
+    twice = torch.zeros(2**n, 2, dtype=torch.complex128, device="cuda")
     twice[:, 0] = psi
-    assert torch.equal(run(twice[:, 0].contiguous()), ref)
+    before = twice.clone()
+    assert not twice[:, 0].is_contiguous() and torch.equal(run(twice[:, 0]), ref)
+    assert torch.equal(twice, before)
+    # a lazily conjugated one
+    lazy = psi.conj()
+    assert lazy.is_conj() and torch.equal(run(lazy), run(lazy.resolve_conj()))
+    # one that autograd follows
+    assert torch.equal(run(psi.clone().requires_grad_()).detach(), ref)
     single = psi.to(torch.complex64)
     assert torch.equal(run(single), run(single.to(torch.complex128)))
     with pytest.raises(ValueError):
         backend.execute_circuit(c, initial_state=psi[:-1])
+
+
+def test_a_state_at_an_odd_address_is_copied_first(backend64):
+    """complex64 views can start between the 16-byte lines that the passes read."""
+    n = 13
+    buf = torch.randn(2**n + 1, dtype=torch.complex64).cuda()
+    psi = buf[1:]
+    assert psi.data_ptr() % 16 == 8
+    run = lambda s: backend64.execute_circuit(_circuit("passes", n), initial_state=s).state()  # noqa: E731
+    before = buf.clone()
+    assert torch.equal(run(psi), run(psi.clone()))
+    assert torch.equal(buf, before)
 
 
 def test_source_must_not_overlap(backend):
