@@ -43,9 +43,9 @@ constexpr int kBankKind[kTileBits] = {0, 1, 2, 3, 4, 0, 1, 2, 4, 3, 0, 1};
 // and rounded where a record takes them: each record then costs an amplitude
 // the one rounding of its own product.
 struct L {
-  long double re = 1, im = 0;
+  long double re, im;
 
-  L() = default;
+  L() {}  // (not set)
   L(long double r, long double i) : re(r), im(i) {}
   L(const C& c) : re(c.re), im(c.im) {}
   C rounded() const { return {double(re), double(im)}; }
@@ -151,7 +151,7 @@ class Compiler {
   L pending_[16];
   long reg_first_off_ = -1;
   size_t reg_first_ev_ = 0;
-  L gfac_;  // a factor of the whole state, taken by the first record that can
+  L gfac_{1, 0};  // a factor of the whole state, taken by the first record that can
   bool sign_ = false;
   int qpend_ = -1;
   std::vector<std::pair<int, L>> phases_;  // controlled phases of register qpend_ not emitted yet: (bit, phase)
@@ -203,7 +203,7 @@ void Compiler::note(uint8_t op, int arg, uint64_t cmask, uint64_t tmask, int rre
   if (cmask || tmask || rreq || !data) return;
   Event e;
   e.off = long(w_.len) + kHeader;
-  e.entries.assign(data, data + ndata);
+  if (op != kRRegPhase) e.entries.assign(data, data + ndata);  // (a table's: emit_table)
   if (op == kRRegPhase && arg != 0) {
     e.kind = 2;
     e.dep = arg;
@@ -498,9 +498,11 @@ void Compiler::qflush(int j) {
 // registers whose bits it depends on.
 void Compiler::flush_reg(int j) {
   if (!have_pending_) return;
+  C now[16];
+  for (int r = 0; r < 16; ++r) now[r] = pending_[r].rounded();
   auto depends_on = [&](int k) {
     for (int r = 0; r < 16; ++r)
-      if (!ceq(pending_[r].rounded(), pending_[r ^ (1 << k)].rounded())) return true;
+      if (!((r >> k) & 1) && !ceq(now[r], now[r | (1 << k)])) return true;
     return false;
   };
   if (j >= 0 && !depends_on(j)) return;
@@ -519,8 +521,10 @@ void Compiler::flush_reg(int j) {
     if (depends_on(k)) dep |= 1 << k;
   gfac_ = gfac_ * t0;
   if (!dep) return;
+  const L inv = L{1, 0} / t0;
   L table[16];
-  for (int r = 0; r < 16; ++r) table[r] = (r & dep) ? pending_[r] / t0 : L{};
+  for (int r = 0; r < 16; ++r)
+    table[r] = (r & dep) ? pending_[r] * inv : L{1, 0};
   emit_table(dep, table);
 }
 
@@ -570,14 +574,14 @@ void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, co
   }
   if (nreg_t == nt && nreg_c == nc) {
     if (!have_pending_) {
-      for (L& x : pending_) x = L{};
+      for (L& x : pending_) x = {1, 0};
       have_pending_ = true;
     }
     for (int r = 0; r < 16; ++r) {
       if ((r & rreq) != rreq) continue;
       int di = 0;
       for (int k = 0; k < nt; ++k) di = (di << 1) | ((r >> reg(tbits[k])) & 1);
-      pending_[r] = pending_[r] * d[di];
+      if (!d[di].one()) pending_[r] = pending_[r] * d[di];
     }
     return;
   }
@@ -846,6 +850,7 @@ void Compiler::fold_cosines() {
 }
 
 int Compiler::run(std::vector<Op>& ops, int* switches) {
+  events_.reserve(ops.size() + 16);
   build_items(ops);
   dependencies();
   lay_ = make_layout(choose_regs(true), low_);
