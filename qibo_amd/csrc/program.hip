@@ -147,8 +147,10 @@ class Compiler {
   Layout lay_;
   bool stale_ = false;  // lane positions were renamed since the kernel formed the lane's index
   bool relabelled_unseen_ = false;  // any position was renamed since the kernel last saw a layout
-  bool have_pending_ = false;
-  L pending_[16];
+  bool have_pending_ = false;  // diagonal gates on the registers not emitted yet:
+  L bit_[4][2];                // factors of single register bits, and if `mixed_`
+  bool mixed_ = false;
+  L pending_[16];              // a table of the others
   long reg_first_off_ = -1;
   size_t reg_first_ev_ = 0;
   L gfac_{1, 0};  // a factor of the whole state, taken by the first record that can
@@ -499,21 +501,30 @@ void Compiler::qflush(int j) {
 void Compiler::flush_reg(int j) {
   if (!have_pending_) return;
   C now[16];
-  for (int r = 0; r < 16; ++r) now[r] = pending_[r].rounded();
+  for (int r = 0; r < 16 && mixed_; ++r) now[r] = pending_[r].rounded();
   auto depends_on = [&](int k) {
-    for (int r = 0; r < 16; ++r)
+    if (!ceq(bit_[k][0].rounded(), bit_[k][1].rounded())) return true;
+    for (int r = 0; r < 16 && mixed_; ++r)
       if (!((r >> k) & 1) && !ceq(now[r], now[r | (1 << k)])) return true;
     return false;
   };
   if (j >= 0 && !depends_on(j)) return;
   have_pending_ = false;
-  const L t0 = pending_[0];
+  L full[16];
+  full[0] = {1, 0};
+  for (int k = 0; k < 4; ++k)
+    for (int r = 0; r < (1 << k); ++r) {
+      full[r | (1 << k)] = full[r] * bit_[k][1];
+      full[r] = full[r] * bit_[k][0];
+    }
+  for (int r = 0; r < 16 && mixed_; ++r) full[r] = full[r] * pending_[r];
+  const L t0 = full[0];
   if (reg_first_off_ < 0 || std::fabs(double(t0.norm2() - 1)) > 1e-12) {
     if (reg_first_off_ < 0) {
       reg_first_off_ = long(w_.len) + kHeader;
       reg_first_ev_ = events_.size();
     }
-    emit_table(0, pending_);
+    emit_table(0, full);
     return;
   }
   int dep = 0;
@@ -524,7 +535,7 @@ void Compiler::flush_reg(int j) {
   const L inv = L{1, 0} / t0;
   L table[16];
   for (int r = 0; r < 16; ++r)
-    table[r] = (r & dep) ? pending_[r] * inv : L{1, 0};
+    table[r] = (r & dep) ? full[r] * inv : L{1, 0};
   emit_table(dep, table);
 }
 
@@ -574,9 +585,19 @@ void Compiler::emit_phase(const int* tbits, int nt, const int* cbits, int nc, co
   }
   if (nreg_t == nt && nreg_c == nc) {
     if (!have_pending_) {
-      for (L& x : pending_) x = {1, 0};
+      for (auto& x : bit_) x[0] = x[1] = {1, 0};
+      mixed_ = false;
       have_pending_ = true;
     }
+    if (nt + nc == 1) {
+      const int j = nt == 1 ? reg(tbits[0]) : reg(cbits[0]);
+      if (nt == 1) bit_[j][0] = bit_[j][0] * d[0];
+      bit_[j][1] = bit_[j][1] * d[nt];
+      return;
+    }
+    if (!mixed_)
+      for (L& x : pending_) x = {1, 0};
+    mixed_ = true;
     for (int r = 0; r < 16; ++r) {
       if ((r & rreq) != rreq) continue;
       int di = 0;
