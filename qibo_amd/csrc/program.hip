@@ -12,8 +12,8 @@
 //  * a SWAP, and the SWAP part of a gate like iSWAP, only renames two local
 //    bits: no data moves until the next change of layout;
 //  * rotations are divided by their cosines (ROTS: two multiply-adds per real
-//    pair instead of three), the cosines multiplied into the entries of one
-//    unconditional record of the run;
+//    pair instead of three), the cosines multiplied into the entries of records
+//    that multiply the whole state at once, a bounded run of rotations each;
 //  * a diagonal gate between one register bit and lane bits is split into a
 //    table, a per-lane phase and a controlled phase (0.30 CU-cycles as DIAG).
 //    Factors of one table or phase are multiplied in extended precision, a
